@@ -394,8 +394,6 @@ phx_status checkDeviceError(phx_ctx* c)
     return fail(c, static_cast<phx_status>(e.code), os.str());
 }
 
-// arguments of the push kernel; `segOk` lets a cell-segmented domain array use the segmented
-// kernel (callers that need a fate for every slot, the compacting path, pass false)
 // a segment tile that outgrew the LDS budget (an extreme segment shape from phx_set_tuning):
 // the launch deposits every particle straight into the moment arrays, correct but slow; said
 // once per context on stderr
@@ -410,6 +408,8 @@ void noteTileFallback(phx_ctx* c, TileSpec const& T)
                  c->tuning.segment_shape[0], c->tuning.segment_shape[1], c->tuning.segment_shape[2]);
 }
 
+// arguments of the push kernel; `segOk` lets a cell-segmented domain array use the 1D/2D segmented
+// kernel (callers that need a fate for every slot, the compacting path, pass false)
 PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt, bool segOk)
 {
     PushArgs A{};
@@ -446,8 +446,18 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
     A.tile = tileShape(c->cfg.dim, c->cfg.interp_order, ppc, copies);
     Pop const& P   = c->pops[pop];
     Store const& s = P.arr[kind];
-    // (3D: the linear-storage kernel on any storage order; the segmented push stays off in 3D with
-    // the captured fused step)
+    // 3D, FP64: the cell-grouped push takes every segment whole, and gives every slot its fate
+    if (c->cfg.dim == 3 && !mixed(c) && kind == KIND_DOMAIN && s.seg)
+    {
+        A.segOn    = 1;
+        A.sg       = c->sg;
+        A.st       = P.seg;
+        A.rhoFromN = P.hasCharge && P.uniformCharge ? 1 : 0;
+        A.split    = cellSplit(c->cfg.interp_order, c->sg, s.n);
+        A.tile     = cellTileShape(c->cfg.interp_order, c->sg, A.rhoFromN ? 4 : 5, c->tuning.tile_row_pad);
+        noteTileFallback(c, A.tile);
+        return A;
+    }
     if (segOk && c->cfg.dim != 3 && kind == KIND_DOMAIN && s.seg
         && segItemsCap(c->sg, s.cap) <= P.itemsAlloc)
     {
@@ -455,9 +465,10 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
         A.sg          = c->sg;
         A.st          = P.seg;
         A.st.itemsCap = segItemsCap(c->sg, s.cap);
-        A.tile        = mixed(c) ? segTileShape32(c->cfg.dim, c->cfg.interp_order, c->sg)
-                                 : segTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, PHX_SEG_COPIES);
         A.rhoFromN    = !mixed(c) && P.hasCharge && P.uniformCharge ? 1 : 0;
+        A.tile        = mixed(c) ? segTileShape32(c->cfg.dim, c->cfg.interp_order, c->sg)
+                                 : segTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, PHX_SEG_COPIES,
+                                                A.rhoFromN ? 4 : 5);
         A.depositWindow = c->tuning.deposit_window;
         noteTileFallback(c, A.tile);
     }
@@ -716,7 +727,7 @@ phx_status enqueueAdvanceFast(phx_ctx* c, double dt)
 }
 
 // A periodic level in 3D runs SolverPPC::advanceLevel staged from the kernels of the drop-in
-// entry points (linear-storage push, Faraday/Ampere/Ohm on the physical nodes followed by the
+// entry points (the push, Faraday/Ampere/Ohm on the physical nodes followed by the
 // periodic ghost fill, the border sum and max of the moments, the ion totals), eagerly on the
 // context stream: the captured fused step (segmented push, fused field kernels) stays off in 3D,
 // one GPU run of it having faulted without a cause shown.
@@ -729,19 +740,13 @@ void enqueuePushStaged3d(phx_ctx* c, int p, PushArgs& A)
 {
     Pop const& P     = c->pops[p];
     Store const& dom = P.arr[PHX_DOMAIN];
-    A.segOn          = 0;
-    if (dom.seg)
+    if (mixed(c) && dom.seg)
     {
         A.sg   = c->sg;
         A.st   = P.seg;
-        A.tile = segwgTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, mixed(c) ? 4 : 5,
-                                c->tuning.tile_row_pad);
+        A.tile = segwgTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, 4, c->tuning.tile_row_pad);
         noteTileFallback(c, A.tile);
-        A.rhoFromN = !mixed(c) && P.hasCharge && P.uniformCharge ? 1 : 0;
-        if (mixed(c))
-            launchPush32SegWG(A, dom.view32(), c->stream);
-        else
-            launchPushSegWG(A, dom.view(), c->stream);
+        launchPush32SegWG(A, dom.view32(), c->stream);
         return;
     }
     if (mixed(c))
@@ -1289,6 +1294,7 @@ phx_status buildPatchTable(phx_ctx* c, int const* plo, int const* phi, int np)
     S.npatch      = np;
     S.rowsPerItem = c->tuning.rows_per_item;
     S.rowPad      = c->tuning.tile_row_pad;
+    S.dense       = D == 3 && !mixed(c) ? 1 : 0;
     size_t boxCells = 1;
     for (int d = 0; d < 3; ++d)
     {
@@ -1391,21 +1397,24 @@ phx_status allocSegTables(phx_ctx* c)
 
 // the launch shapes of this build before any tuning: the autotuner's winners on the 2D Harris
 // workload (segments of 2x32 cells, at most 32 rows per work item, tile rows padded to 16 nodes,
-// a sort every 30 PPC steps); runs of 64 cells in 1D, 4x4x4 blocks in 3D (the staged 3D path's
-// one-workgroup-per-segment push gives each lane of a wavefront one cell of the block)
-phx_tuning defaultTuning(int dim, int order)
+// a sort every 30 PPC steps); runs of 64 cells in 1D, 4x4x4 blocks in 3D
+phx_tuning defaultTuning(int dim, int order, bool fp32)
 {
     phx_tuning t{};
     static int const pref[3][3] = {{64, 1, 1}, {2, 32, 1}, {4, 4, 4}};
     for (int d = 0; d < 3; ++d)
         t.segment_shape[d] = pref[dim - 1][d];
     t.rows_per_item = PHX_SEG_ROWS;
-    // 3D: the segment tile's pitches padded to a multiple of 4 nodes at orders 1 and 3 (every
-    // particle's stencil starts at a fixed node of its cell, so the 64 lanes of one LDS atomic
-    // fall on distinct bank pairs); unpadded at order 2 (starts shift with the delta at random,
-    // and the larger tile would halve the workgroups per CU)
-    t.tile_row_pad  = dim == 3 ? (order == 2 ? 1 : 4) : PHX_TILE_ROW_PAD;
-    t.sort_interval = 30;
+    // 3D, mixed precision: the segment tile's pitches padded to a multiple of 4 nodes at orders 1
+    // and 3 (every particle's stencil starts at a fixed node of its cell, so the 64 lanes of one LDS
+    // atomic fall on distinct bank pairs); unpadded at order 2 (starts shift with the delta at
+    // random, and the larger tile would halve the workgroups per CU), and in FP64, whose particles
+    // deposit by cell
+    t.tile_row_pad  = dim == 3 ? (order == 2 || !fp32 ? 1 : 4) : PHX_TILE_ROW_PAD;
+    // the cell-grouped 3D push slows with every particle that has left its cell since the sort (64^3
+    // cells, order 2, 64 per cell, per PPC step: 3.61 ms sorted every 30 steps, 3.27 every 15, 3.12
+    // every 7, 3.17 every 3; orders 1 and 3 within 1 % of their best at 7 too)
+    t.sort_interval = dim == 3 && !fp32 ? 7 : 30;
     t.tile_copies   = dim == 1 ? PHX_TILE_COPIES_1D : (dim == 2 ? PHX_TILE_COPIES_2D : PHX_TILE_COPIES_3D);
     t.deposit_window = 0;
     return t;
@@ -1571,7 +1580,7 @@ phx_status createLevel(phx_config const* cfg, phx_patch const* patch, int const*
         for (int k = 0; k < 5 && s == PHX_OK; ++k)
             s = storeAlloc(c, c->pops[p].arr[k], k == 0 ? std::max<size_t>(particle_capacity, 1024) : 1024);
     }
-    c->tuning = defaultTuning(D, cfg->interp_order);
+    c->tuning = defaultTuning(D, cfg->interp_order, mixed(c));
     c->sortInterval = c->tuning.sort_interval;
     if (s == PHX_OK)
         s = buildPatchTable(c, plo, phi, np);
@@ -2829,7 +2838,7 @@ phx_status phx_set_tuning(phx_ctx* c, phx_tuning const* t)
         return PHX_ERR_ARG;
     int const D       = c->cfg.dim;
     phx_tuning next   = *t;
-    phx_tuning const d = defaultTuning(D, c->cfg.interp_order);
+    phx_tuning const d = defaultTuning(D, c->cfg.interp_order, mixed(c));
     int cells         = 1;
     for (int k = 0; k < 3; ++k)
     {

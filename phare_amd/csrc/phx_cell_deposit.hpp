@@ -1,0 +1,330 @@
+// phx_cell_deposit.hpp -- moment deposit of particles grouped by cell on the FP64 matrix cores.
+//
+// The particles of one cell deposit into one window of W nodes per direction (W = 2 at order 1:
+// nodes cell, cell + 1; W = 4 at orders 2 and 3: nodes cell - 1 .. cell + 2, a particle's weight
+// being zero on the node its order-2 stencil leaves out). Over the particles p of the cell the
+// window is the contraction
+//     window[(a, b), (c, m)] = sum_p (wx_p[a] wy_p[b]) (wz_p[c] value_p[m])
+// with m the moments n, Fx, Fy, Fz: at W = 4 one 16x16x4 FP64 MFMA per four particles, at W = 2 one
+// 4x4x4 (four-block) MFMA per eight. The window stays in a wavefront's registers while its
+// particles stay in the cell and is then added to the workgroup's LDS tile, 4 (W = 4) or 1 (W = 2)
+// LDS atomics per wavefront and cell instead of one per particle, node and moment: a particle cost
+// 108 (order 2) or 256 (order 3) lanes of ds_add_f64, about 30 cycles of the CU's LDS per
+// wavefront instruction, and costs about a quarter (W = 4) or a sixteenth (W = 2) of an MFMA here.
+//
+// The lanes of a wavefront hand their weights over through a small LDS buffer of the wavefront, 32
+// particles at a time: array j (the weights along x, y, z, then the values) of particle p at
+// j * WSTR + p. WSTR is 36 words, so that the four arrays and four particle pairs that one read
+// touches lie in distinct banks.
+#pragma once
+
+#include "phx_push_common.hpp"
+
+namespace phx
+{
+namespace pc
+{
+typedef double d4 __attribute__((ext_vector_type(4)));
+
+constexpr int WHALF = 32; // particles handed over at a time
+constexpr int WSTR  = 36; // words between two arrays of the buffer (even: pairs are read as 16 bytes)
+
+// order of the wavefront's own LDS writes before its later reads of other lanes' words
+__device__ __forceinline__ void waveLds()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// window of a cell in 3D. RN: the charge density is derived from n and has no column
+template<int O, bool RN>
+struct CellWin
+{
+    static constexpr int W    = O == 1 ? 2 : 4;
+    static constexpr int WB   = O == 1 ? 0 : 1; // window base = local cell - WB
+    static constexpr int NVAL = RN ? 4 : 5;
+    static constexpr int ARR  = 3 * W + NVAL;
+    static constexpr int BUF  = ARR * WSTR; // words of LDS per wavefront
+    static constexpr int NACC = W == 4 ? 4 : 1;
+
+    double a[NACC];            // n, Fx, Fy, Fz columns
+    double rho[RN ? 1 : NACC]; // the charge density's column
+
+    __device__ __forceinline__ void zero()
+    {
+#pragma unroll
+        for (int r = 0; r < NACC; ++r)
+            a[r] = 0.;
+        if constexpr (!RN)
+#pragma unroll
+            for (int r = 0; r < NACC; ++r)
+                rho[r] = 0.;
+    }
+};
+
+// B-spline weights (interpolator.hpp:54-125) from the offset of the particle in its cell alone: u is
+// the particle's position less the stencil's first node, of the size of the stencil, where the
+// absolute position would cost its last digits; w[0 .. O]
+template<int O>
+__device__ __forceinline__ void splineWeights(double u, double* w)
+{
+    if constexpr (O == 1)
+    {
+        w[0] = 1. - u;
+        w[1] = u;
+    }
+    else if constexpr (O == 2)
+    {
+        double const d = u - 1.;
+        double const lo = 0.5 - d, hi = 0.5 + d;
+        w[0] = 0.5 * lo * lo;
+        w[1] = __builtin_fma(-d, d, 0.75);
+        w[2] = 0.5 * hi * hi;
+    }
+    else
+    {
+        // u = 1 + t, t in [0, 1): cubic B-spline at t + 1, t, 1 - t, 2 - t
+        double const t = u - 1., s = 1. - t;
+        double const t2 = t * t, s2 = s * s;
+        w[0] = s2 * s * (1. / 6.);
+        w[1] = __builtin_fma(t2, __builtin_fma(0.5, t, -1.), 2. / 3.);
+        w[2] = __builtin_fma(s2, __builtin_fma(0.5, s, -1.), 2. / 3.);
+        w[3] = t2 * t * (1. / 6.);
+    }
+}
+
+// stencil of one direction: shift of its first node from the particle's cell (interpolator.hpp:
+// 519-549) and weights, centering c
+template<int O>
+__device__ __forceinline__ int splineStencil(int c, double delta, double* w)
+{
+    int const sh   = startShift<O>(c, delta);
+    double const u = delta + (c == CD ? static_cast<double>(sh) - 0.5 : static_cast<double>(sh));
+    splineWeights<O>(u, w);
+    return sh;
+}
+
+// the primal weights of one direction on the cell's window (zero on the node an order-2 stencil
+// leaves out)
+template<int O>
+__device__ __forceinline__ void windowWeights(double delta, double* out)
+{
+    if constexpr (O == 2)
+    {
+        double w[3];
+        bool const low = splineStencil<2>(CP, delta, w) == 1;
+        out[0]         = low ? w[0] : 0.;
+        out[1]         = low ? w[1] : w[0];
+        out[2]         = low ? w[2] : w[1];
+        out[3]         = low ? 0. : w[2];
+    }
+    else
+        splineStencil<O>(CP, delta, out);
+}
+
+// the 32 particles of lanes [32 half, 32 half + 32) into the wavefront's buffer: the window weights
+// of delta along x, y, z, then the values n, Fx, Fy, Fz (and rho); lanes without `ok` hand over finite
+// weights and zero values
+template<int O, bool RN>
+__device__ __forceinline__ void cellStage(double* buf, int half, bool ok, double const* delta, double w,
+                                          double q, double const* v, double coef)
+{
+    using C        = CellWin<O, RN>;
+    int const lane = static_cast<int>(threadIdx.x & 63u);
+    waveLds(); // the reads of the half before are done
+    if ((lane >> 5) == half)
+    {
+        double* const b = buf + (lane & (WHALF - 1));
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+        {
+            double ww[C::W];
+            windowWeights<O>(ok ? delta[d] : 0., ww);
+#pragma unroll
+            for (int a = 0; a < C::W; ++a)
+                b[(d * C::W + a) * WSTR] = ww[a];
+        }
+        // the reference's products: 1. * w * coef, v * w * coef, q * w * coef
+        b[3 * C::W * WSTR] = ok ? w * coef : 0.;
+#pragma unroll
+        for (int d = 0; d < 3; ++d)
+            b[(3 * C::W + 1 + d) * WSTR] = ok ? v[d] * w * coef : 0.;
+        if constexpr (!RN)
+            b[(3 * C::W + 4) * WSTR] = ok ? q * w * coef : 0.;
+    }
+    waveLds();
+}
+
+// the staged particles whose bit of `mask` is set (all of one cell) added to the window. ALL: every
+// instruction of the half row is issued, without a branch between them (many particles set)
+template<int O, bool RN, bool ALL>
+__device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, CellWin<O, RN>& acc)
+{
+    using C        = CellWin<O, RN>;
+    int const lane = static_cast<int>(threadIdx.x & 63u);
+    int const i    = lane & 15;
+    int const k    = lane >> 4;
+    if constexpr (C::W == 4)
+    {
+        // rows (a, b) = (i / 4, i % 4) of A, columns (c, m) = (i / 4, i % 4) of B; four particles
+        // per instruction, lane group k taking a pair of particles for two instructions
+        double const* const px = buf + (i >> 2) * WSTR + 2 * k;
+        double const* const py = buf + (4 + (i & 3)) * WSTR + 2 * k;
+        double const* const pz = buf + (8 + (i >> 2)) * WSTR + 2 * k;
+        double const* const pv = buf + (12 + (i & 3)) * WSTR + 2 * k;
+        double const* const pr = buf + 16 * WSTR + 2 * k;
+        unsigned int const mk  = mask >> (2 * k);
+        d4 c  = {acc.a[0], acc.a[1], acc.a[2], acc.a[3]};
+        d4 cr = {0., 0., 0., 0.};
+        if constexpr (!RN)
+            cr = d4{acc.rho[0], acc.rho[1], acc.rho[2], acc.rho[3]};
+#pragma unroll
+        for (int t = 0; t < WHALF / 8; ++t)
+        {
+            if (!ALL && ((mask >> (8 * t)) & 0xffu) == 0u)
+                continue;
+            double2 const x = *reinterpret_cast<double2 const*>(px + 8 * t);
+            double2 const y = *reinterpret_cast<double2 const*>(py + 8 * t);
+            double2 const z = *reinterpret_cast<double2 const*>(pz + 8 * t);
+            double2 const v = *reinterpret_cast<double2 const*>(pv + 8 * t);
+            double const a0 = x.x * y.x, a1 = x.y * y.y;
+            double const z0 = (mk >> (8 * t)) & 1u ? z.x : 0.;
+            double const z1 = (mk >> (8 * t)) & 2u ? z.y : 0.;
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, z0 * v.x, c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, z1 * v.y, c, 0, 0, 0);
+            if constexpr (!RN)
+            {
+                double2 const q = *reinterpret_cast<double2 const*>(pr + 8 * t);
+                bool const on   = (i & 3) == 0;
+                cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, on ? z0 * q.x : 0., cr, 0, 0, 0);
+                cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, on ? z1 * q.y : 0., cr, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            acc.a[r] = c[r];
+            if constexpr (!RN)
+                acc.rho[r] = cr[r];
+        }
+    }
+    else
+    {
+        // block beta = (c, s): node c along z and half s of the particles; rows (a, b) = bits of
+        // lane % 4, columns m; eight particles per instruction
+        int const s = (lane >> 3) & 1, c = (lane >> 2) & 1;
+        int const o = 4 * k + 2 * s;
+        double const* const px = buf + ((lane >> 1) & 1) * WSTR + o;
+        double const* const py = buf + (2 + (lane & 1)) * WSTR + o;
+        double const* const pz = buf + (4 + c) * WSTR + o;
+        double const* const pv = buf + (6 + (lane & 3)) * WSTR + o;
+        double const* const pr = buf + 10 * WSTR + o;
+        unsigned int const mk  = mask >> o;
+#pragma unroll
+        for (int t = 0; t < WHALF / 16; ++t)
+        {
+            if (!ALL && ((mask >> (16 * t)) & 0xffffu) == 0u)
+                continue;
+            double2 const x = *reinterpret_cast<double2 const*>(px + 16 * t);
+            double2 const y = *reinterpret_cast<double2 const*>(py + 16 * t);
+            double2 const z = *reinterpret_cast<double2 const*>(pz + 16 * t);
+            double2 const v = *reinterpret_cast<double2 const*>(pv + 16 * t);
+            double const a0 = x.x * y.x, a1 = x.y * y.y;
+            double const z0 = (mk >> (16 * t)) & 1u ? z.x : 0.;
+            double const z1 = (mk >> (16 * t)) & 2u ? z.y : 0.;
+            acc.a[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, z0 * v.x, acc.a[0], 0, 0, 0);
+            acc.a[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, z1 * v.y, acc.a[0], 0, 0, 0);
+            if constexpr (!RN)
+            {
+                double2 const q = *reinterpret_cast<double2 const*>(pr + 16 * t);
+                bool const on   = (lane & 3) == 0;
+                acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, on ? z0 * q.x : 0., acc.rho[0], 0, 0, 0);
+                acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, on ? z1 * q.y : 0., acc.rho[0], 0, 0, 0);
+            }
+        }
+    }
+}
+
+template<int O, bool RN>
+__device__ __forceinline__ void cellAdd(double const* buf, unsigned int mask, CellWin<O, RN>& acc)
+{
+    if (__popc(mask) >= WHALF / 2)
+        cellAddT<O, RN, true>(buf, mask, acc);
+    else
+        cellAddT<O, RN, false>(buf, mask, acc);
+}
+
+// one staged particle (p, in no larger group) added to the LDS tile by itself
+template<int O, bool RN>
+__device__ __forceinline__ void cellAddOne(double const* buf, int p, double* tile, int stride, int node0,
+                                           int p12, int p2)
+{
+    using C        = CellWin<O, RN>;
+    int const lane = static_cast<int>(threadIdx.x & 63u);
+    int const m    = lane & 3;
+    int const slab = RN || m == 0 ? m : m + 1;
+    if constexpr (C::W == 4)
+    {
+        int const b = lane >> 4, c = (lane & 15) >> 2;
+        double const yz = buf[(4 + b) * WSTR + p] * buf[(8 + c) * WSTR + p];
+        double const t  = yz * buf[(12 + m) * WSTR + p];
+        int const n     = node0 + b * p2 + c;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            double const x = buf[r * WSTR + p];
+            atomicAdd(tile + slab * stride + n + r * p12, x * t);
+            if constexpr (!RN)
+                if (m == 0)
+                    atomicAdd(tile + stride + n + r * p12, x * (yz * buf[16 * WSTR + p]));
+        }
+    }
+    else if (lane < 32)
+    {
+        int const a = lane >> 4, b = (lane >> 3) & 1, c = (lane >> 2) & 1;
+        double const xyz = buf[a * WSTR + p] * buf[(2 + b) * WSTR + p] * buf[(4 + c) * WSTR + p];
+        int const n      = node0 + a * p12 + b * p2 + c;
+        atomicAdd(tile + slab * stride + n, xyz * buf[(6 + m) * WSTR + p]);
+        if constexpr (!RN)
+            if (m == 0)
+                atomicAdd(tile + stride + n, xyz * buf[10 * WSTR + p]);
+    }
+}
+
+// add the window to the LDS tile: node0 is the tile node of the window's origin, p12 and p2 the
+// node distances along x and y, slab m of the tile the moments in the order n, (rho,) Fx, Fy, Fz
+template<int O, bool RN>
+__device__ __forceinline__ void cellFlush(CellWin<O, RN> const& acc, double* tile, int stride, int node0,
+                                          int p12, int p2)
+{
+    using C        = CellWin<O, RN>;
+    int const lane = static_cast<int>(threadIdx.x & 63u);
+    int const m    = lane & 3;
+    int const slab = RN || m == 0 ? m : m + 1;
+    if constexpr (C::W == 4)
+    {
+        // result register r of lane (q, i): row 4 r + q = (a, b) = (r, q), column i
+        int const n = node0 + (lane >> 4) * p2 + ((lane & 15) >> 2);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+        {
+            atomicAdd(tile + slab * stride + n + r * p12, acc.a[r]);
+            if constexpr (!RN)
+                if (m == 0)
+                    atomicAdd(tile + stride + n + r * p12, acc.rho[r]);
+        }
+    }
+    else
+    {
+        int const i = lane >> 4;
+        int const n = node0 + (i >> 1) * p12 + (i & 1) * p2 + ((lane >> 2) & 1);
+        atomicAdd(tile + slab * stride + n, acc.a[0]);
+        if constexpr (!RN)
+            if (m == 0)
+                atomicAdd(tile + stride + n, acc.rho[0]);
+    }
+}
+
+} // namespace pc
+} // namespace phx

@@ -207,8 +207,9 @@ __device__ __forceinline__ void stencilOf(int q, Stencil<D, O> const& s, int* st
 }
 
 // interpolation of a C-order array with row strides s1 (dimension 1) and s2 (dimension 2) from
-// the stencil starting at st, in the reference's order of sums (MeshToParticle)
-template<int D, int O>
+// the stencil starting at st, in the reference's order of sums (MeshToParticle). LEAN: the loads of
+// one 3D plane in flight at a time (fewer registers)
+template<int D, int O, bool LEAN = false>
 __device__ __forceinline__ double interpStrided(double const* __restrict__ f, int const* st,
                                                 double const* const* w, int s1, int s2)
 {
@@ -254,19 +255,21 @@ __device__ __forceinline__ double interpStrided(double const* __restrict__ f, in
                 yi += zi * w[1][j];
             }
             r += yi * w[0][i];
+            if constexpr (LEAN)
+                __builtin_amdgcn_sched_barrier(0);
         }
         return r;
     }
 }
 
-template<int D, int O>
+template<int D, int O, bool LEAN = false>
 __device__ __forceinline__ double interp(Geom const& G, double const* __restrict__ f, int q,
                                          Stencil<D, O> const& s)
 {
     int st[D];
     double const* w[D];
     stencilOf<D, O>(q, s, st, w);
-    return interpStrided<D, O>(f, st, w, G.shape[q][1], G.shape[q][2]);
+    return interpStrided<D, O, LEAN>(f, st, w, G.shape[q][1], G.shape[q][2]);
 }
 
 struct EMPtrs

@@ -70,6 +70,9 @@ struct TileSpec
     int copies; // moment copies (power of two): lane l accumulates into copy l % copies
     int stride;
     unsigned int bytes; // dynamic LDS of the launch
+    // cell-grouped 3D push: fields staged beside the tile, from node (tile origin + emLo), extents
+    // emExt, emStride words of LDS for the six components; emFix: emExt is that of a 4x4x4 segment
+    int emLo[3], emExt[3], emStride, emFix;
     int brick;          // > 0: the tile covers the brick (cube of `brick` cells, on the grid of
                         // bricks from the patch's lower cell) of the chunk's first particle
 };
@@ -81,7 +84,9 @@ constexpr int BRICK = 4;
 // table, patches of uneven sizes) is cut into segments, boxes of at most 64 cells (shape `seg`),
 // numbered patch after patch; a segment holding P particles has R = ceil(P / 64) rows of 64 slots.
 // Its particles, in the order of their cells (row-major inside the segment), take the slots
-// column by column: position p is slot p / R of row p % R. The slots past P hold dead particles.
+// column by column (position p is slot p / R of row p % R) or, `dense`, row by row (position p is
+// slot p, so that a row holds particles of one cell or of neighbours in that order: the cell-grouped
+// push). The slots past P in that order hold dead particles.
 // One more segment at the end holds, unordered, the particles outside every patch. A particle
 // belongs to the patch whose domain box holds its cell (the owner map), so a sort also migrates
 // the particles that crossed into a neighbouring patch.
@@ -104,6 +109,7 @@ struct SegGeom
     int n[3];      // level box cells per dimension
     int maxSeg[3]; // largest segment extent over the patches (the launch's LDS tile)
     int rowsPerItem; // most segment rows per work item of the segmented push
+    int dense;       // positions fill the rows one after the other
     int rowPad;      // 2D LDS tile rows padded to a multiple of this many nodes
     SegPatch first;               // patch 0 (a one-patch level reads it from the kernel arguments)
     SegPatch const* patch;        // [npatch] (device)
@@ -149,6 +155,7 @@ struct PushArgs
     uint8_t* status;
     unsigned int* dropped;
     int segOn; // the array is cell-segmented (sg, st valid)
+    unsigned int split; // 3D cell-grouped push: workgroups per segment
     SegGeom sg;
     SegTables st;
     float const* em32[6]; // mixed-precision family: FP32 copy of the E/B set (Ex..Bz)
@@ -185,7 +192,7 @@ unsigned int compactBlocks(unsigned long long n);
 // segmented storage: segment shape of a patch box (segBase/cellBase left to the caller), LDS
 // tile of the segmented push, the most work items a storage of `capacity` slots can need
 SegPatch segPatchOf(int dim, int const* lo, int const* hi, int const* pref);
-TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies);
+TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies, int slabs);
 unsigned int segItemsCap(SegGeom const& sg, unsigned long long capacity);
 // first half of a sort of src (n slots) into cell-segmented storage: counts per cell, the rank
 // of every particle in its cell (rank: n words) and the segment tables up to the total slot count
@@ -213,10 +220,15 @@ TileSpec segTileShape32(int dim, int order, SegGeom const& sg);
 // the same over brick-ordered linear FP32 storage (3D), in place; the LDS tile of brickTileShape32
 void launchPush32Linear(PushArgs const& A, PView32 const& v, hipStream_t s);
 TileSpec brickTileShape32(int order);
-// push + gather + deposit over cell-segmented storage with one workgroup per segment and all its
-// rows, in place (3D; the staged 3D path), FP64 and mixed precision; grid nsegs + 1; the LDS tile
-// of segwgTileShape (5 slabs FP64, 4 mixed precision)
-void launchPushSegWG(PushArgs const& A, PView const& in, hipStream_t s);
+// push + gather + deposit (A.pushOn 0: deposit only) over dense cell-segmented 3D storage, in place,
+// A.split workgroups per segment, the particles of a cell deposited together; the LDS tile of
+// cellTileShape (5 slabs, 4 with A.rhoFromN)
+void launchPushCell(PushArgs const& A, PView const& in, hipStream_t s);
+TileSpec cellTileShape(int order, SegGeom const& sg, int slabs, int pad);
+// workgroups per segment (A.split) for an array of `slots` slots
+unsigned int cellSplit(int order, SegGeom const& sg, unsigned long long slots);
+// mixed-precision push + gather + deposit over cell-segmented storage with one workgroup per segment
+// and all its rows, in place (3D); grid nsegs + 1; the LDS tile of segwgTileShape (4 slabs)
 void launchPush32SegWG(PushArgs const& A, PView32 const& v, hipStream_t s);
 TileSpec segwgTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad);
 // BorisPusher::move in place over A.n slots with box-list selectors; status[i] gets the slot's

@@ -17,7 +17,7 @@
 // tile with one HBM atomic per touched node and moment; the gather reads E/B through the L1/L2
 // caches, leaving the LDS to the deposit. Particles whose stencil leaves the tile deposit
 // straight into HBM.
-#include "phx_push_common.hpp"
+#include "phx_cell_deposit.hpp"
 
 #include <algorithm>
 #include <mutex>
@@ -37,6 +37,40 @@ using pc::inNLGB;
 using pc::LANES;
 using pc::NW;
 using pc::TILE_BYTES_MAX;
+
+// the cell-grouped push, per order: work-items of a workgroup, waves per SIMD the register allocation
+// targets (what a workgroup's LDS leaves room for), and whether the next row is loaded while a row is
+// worked on. Order 1 runs best on many waves without the prefetch's registers (58x47x52 cells, 50
+// particles per cell: 0.243 ms for mode domain_only, against 0.259 with two workgroups of 256 and
+// the prefetch); at order 2 two workgroups of 256 fit a CU (64^3 cells, 64 per cell: 0.95 ms; 1.09 with
+// one of 512); at order 3 the larger stage leaves room for one workgroup, of 512 (36x41x30 cells, 32
+// per cell: 0.207 ms, 0.260 with 256)
+template<int O>
+struct CellCfg
+{
+    static constexpr int BLOCK     = O == 2 ? 256 : 512;
+    static constexpr int WAVES     = O == 1 ? 4 : 2;
+    static constexpr bool PREFETCH = O != 1;
+    static constexpr int NW        = BLOCK / LANES;
+};
+constexpr int cellBlock(int order) { return order == 2 ? 256 : 512; }
+// particles listed for the one-by-one push between two passes over the rows (every wavefront that
+// finds room for a workgroup's particles may add its row)
+constexpr unsigned int CELL_LIST = 1024;
+// the smallest group of lanes of one cell (of the 32 of a half row) that deposits on the matrix cores,
+// and the smallest that moves the accumulated window to its cell
+constexpr int CELL_GROUP = 2;
+constexpr int CELL_MOVE  = 8;
+constexpr unsigned long long CUS = 256; // compute units of the GPU
+// most LDS of a workgroup's tile, stage and buffers
+constexpr unsigned int CELL_LDS_MAX = 131072;
+// nodes of a cell's gather stencils: the first, relative to the cell, and how many; the stage holds
+// them for the segment's cells and those one cell around it
+constexpr int cellGatherLo(int order) { return order == 3 ? -2 : -1; }
+constexpr int cellGatherNodes(int order) { return order == 1 ? 3 : (order == 2 ? 4 : 5); }
+// nodes per direction of the stage of a 4x4x4 segment
+template<int O>
+constexpr int CELL_STAGE = 4 + 1 + cellGatherNodes(O);
 
 // Per (dim, order): whether the deposit is accumulated in registers over a union window, the
 // particles per thread of the linear push and the window. With accumulation, a thread's
@@ -68,7 +102,12 @@ struct TileView
     int ext[3];
     int pitch[3];
     int copies, stride;
-    __device__ double* mom(int m, int copy) const { return lds + (m * copies + copy) * stride; }
+    // slab of moment m (n, rho, Fx, Fy, Fz); RN: the tile leaves the charge density (m = 1) out
+    template<bool RN = false>
+    __device__ double* mom(int m, int copy) const
+    {
+        return lds + ((RN && m > 1 ? m - 1 : m) * copies + copy) * stride;
+    }
     __device__ int node(int i, int j, int k) const { return (i * pitch[1] + j) * pitch[2] + k; }
     // the O+1 nodes from start lie in the tile along d
     template<int O>
@@ -114,22 +153,22 @@ __device__ __forceinline__ double nodeWeight(DepositData<D, O> const& dd, double
 
 
 // E and B at the particle (Interpolator::operator() for the fields, interpolator.hpp:420-456)
-template<int D, int O>
+template<int D, int O, bool LEAN = false>
 __device__ __forceinline__ void gatherEB(Geom const& G, EMPtrs const& em, Stencil<D, O> const& s,
                                          double* E, double* B)
 {
-    E[0] = interp<D, O>(G, em.E[0], QEX, s);
-    E[1] = interp<D, O>(G, em.E[1], QEY, s);
-    E[2] = interp<D, O>(G, em.E[2], QEZ, s);
-    B[0] = interp<D, O>(G, em.B[0], QBX, s);
-    B[1] = interp<D, O>(G, em.B[1], QBY, s);
-    B[2] = interp<D, O>(G, em.B[2], QBZ, s);
+    E[0] = interp<D, O, LEAN>(G, em.E[0], QEX, s);
+    E[1] = interp<D, O, LEAN>(G, em.E[1], QEY, s);
+    E[2] = interp<D, O, LEAN>(G, em.E[2], QEZ, s);
+    B[0] = interp<D, O, LEAN>(G, em.B[0], QBX, s);
+    B[1] = interp<D, O, LEAN>(G, em.B[1], QBY, s);
+    B[2] = interp<D, O, LEAN>(G, em.B[2], QBZ, s);
 }
 
 // scatter-add the 5 moments of one particle: into the lane's copy of the LDS tile when its
 // whole stencil lies in the tile, else straight into the HBM moment arrays. RN: the population
 // has one charge, the tile skips the charge density and its flush derives it from n
-template<int D, int O, bool RN = false>
+template<int D, int O, bool RN = false, bool LEAN = false>
 __device__ __forceinline__ void depositOne(DepositData<D, O> const& dd, Geom const& G,
                                            TileView const& T, int copy, double* const* mom)
 {
@@ -145,7 +184,7 @@ __device__ __forceinline__ void depositOne(DepositData<D, O> const& dd, Geom con
         double* slab[5];
 #pragma unroll
         for (int m = 0; m < 5; ++m)
-            slab[m] = T.mom(m, copy);
+            slab[m] = T.mom<RN>(m, copy);
 #pragma unroll
         for (int a = 0; a < S; ++a)
 #pragma unroll
@@ -160,6 +199,8 @@ __device__ __forceinline__ void depositOne(DepositData<D, O> const& dd, Geom con
                     for (int m = 0; m < 5; ++m)
                         if (!RN || m != 1)
                             atomicAdd(slab[m] + node, nodeWeight<D, O>(dd, dd.val[m], a, b, c));
+                    if constexpr (LEAN)
+                        __builtin_amdgcn_sched_barrier(0);
                 }
     }
     else
@@ -176,6 +217,8 @@ __device__ __forceinline__ void depositOne(DepositData<D, O> const& dd, Geom con
 #pragma unroll
                     for (int m = 0; m < 5; ++m)
                         atomicAdd(mom[m] + node, nodeWeight<D, O>(dd, dd.val[m], a, b, c));
+                    if constexpr (LEAN)
+                        __builtin_amdgcn_sched_barrier(0);
                 }
     }
 }
@@ -204,7 +247,7 @@ __device__ __forceinline__ void accZero(Acc<D, O>& A)
 
 // scatter the window: nodes inside the LDS tile by LDS atomics into the lane's copy, others
 // straight to HBM; never-touched nodes hold exactly zero and are skipped
-template<int D, int O>
+template<int D, int O, bool RN>
 __device__ __forceinline__ void accFlush(Acc<D, O> const& A, Geom const& G, TileView const& T,
                                          int copy, double* const* mom)
 {
@@ -230,10 +273,10 @@ __device__ __forceinline__ void accFlush(Acc<D, O> const& A, Geom const& G, Tile
             double const v = A.a[m][x];
             if (v != 0.)
             {
-                if (inTile)
-                    atomicAdd(T.mom(m, copy) + tnode, v);
-                else
+                if (!inTile)
                     atomicAdd(mom[m] + G.idx(QMOM, g[0], g[1], g[2]), v);
+                else if (!RN || m != 1)
+                    atomicAdd(T.mom<RN>(m, copy) + tnode, v);
             }
         }
     }
@@ -309,10 +352,140 @@ __device__ __forceinline__ void loadPart(PView const& in, unsigned long long i, 
     p.q    = in.q[i];
 }
 
+// prePushStep_ (boris.hpp:180-216) and the first selector (noop for the domain, inGhostBox for level
+// ghosts): false when the particle moved two cells or (selected) its E/B stencil s leaves the ghost
+// box, which REPORT raises
+template<int D, int O, bool REPORT>
+__device__ __forceinline__ bool prePush(PushArgs const& A, unsigned long long i, int* cell, double* delta,
+                                        double const* v, bool& sel1, Stencil<D, O>& s)
+{
+    Geom const& G = A.G;
+    double bd, bv;
+    if (!advancePosition<D>(cell, delta, v, A.hdtdx, bd, bv))
+    {
+        if (REPORT)
+            raiseError(A.err, 3u, 1u, i, bd, bv, A.kind, A.pop);
+        return false;
+    }
+    sel1 = A.kind == KIND_DOMAIN ? true : inBox(cell, A.box.gh_lo, A.box.gh_hi, D);
+    if (!sel1)
+        return true;
+    makeStencil<D, O>(G, cell, delta, s);
+    bool safe = true;
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+    {
+        int const icl = cell[d] - (G.lower[d] - G.g);
+        safe          = safe && icl >= G.safeLo[d] && icl <= G.safeHi[d];
+    }
+    if (!safe
+        && (!stencilInside<D, O>(G, s, QEX) || !stencilInside<D, O>(G, s, QBX)
+            || !stencilInside<D, O>(G, s, QEY) || !stencilInside<D, O>(G, s, QBY)
+            || !stencilInside<D, O>(G, s, QEZ) || !stencilInside<D, O>(G, s, QBZ)))
+    {
+        if (REPORT)
+            raiseError(A.err, 4u, 2u, i, delta[0], v[0], A.kind, A.pop);
+        return false;
+    }
+    return true;
+}
+
+// Boris and postPushStep_ (boris.hpp:218-300) of a particle the first selector keeps; false when
+// it moved two cells, which REPORT raises
+template<int D, bool REPORT>
+__device__ __forceinline__ bool postPush(PushArgs const& A, unsigned long long i, int* cell, double* delta,
+                                         double* v, double q, double const* E, double const* B)
+{
+    double bd, bv;
+    borisAccelerate(v, E, B, q, A.dto2m);
+    if (advancePosition<D>(cell, delta, v, A.hdtdx, bd, bv))
+        return true;
+    if (REPORT)
+        raiseError(A.err, 3u, 2u, i, bd, bv, A.kind, A.pop);
+    return false;
+}
+
+// what is deposited and what the array keeps of a pushed particle (ion_updater.hpp:169-295)
+template<int D>
+__device__ __forceinline__ void selectPushed(PushArgs const& A, int const* cell, bool sel1, bool& deposit,
+                                             uint8_t& st)
+{
+    bool const inDom = inBox(cell, A.box.dom_lo, A.box.dom_hi, D);
+    if (A.kind == KIND_DOMAIN)
+    {
+        bool const nl = inNLGB(cell, A.box, D);
+        deposit       = nl;
+        st            = inDom ? ST_KEEP : (nl ? ST_LEAVE : ST_DROP);
+    }
+    else
+    {
+        deposit = sel1 && inDom;
+        bool const layer = sel1 && !inDom && inBox(cell, A.box.gh_lo, A.box.gh_hi, D);
+        st = !sel1 ? ST_DROP : (inDom ? ST_EXPORT : (layer ? ST_KEEP : ST_DROP));
+    }
+}
+
+// the deposited values of a particle: n, rho, Fx, Fy, Fz
+__device__ __forceinline__ void depositValues(double w, double q, double const* v, double coef, double* val)
+{
+    val[0] = 1. * w * coef;
+    val[1] = q * w * coef;
+    val[2] = v[0] * w * coef;
+    val[3] = v[1] * w * coef;
+    val[4] = v[2] * w * coef;
+}
+
+// mode all: the pushed particle written to its slot (a leaver of a periodic level re-enters through
+// the periodic image) and its fate
+template<int D>
+__device__ __forceinline__ void storePushed(PushArgs const& A, PView const& out, bool outOfPlace,
+                                            unsigned long long i, int* cell, double const* delta,
+                                            double const* v, double w, double q, uint8_t st)
+{
+    if (A.periodicWrap && A.kind == KIND_DOMAIN)
+    {
+        if (st == ST_LEAVE)
+        {
+            // fillIonGhostParticles: the leaver re-enters through the periodic image
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+            {
+                if (cell[d] < A.box.dom_lo[d])
+                    cell[d] += A.G.n[d];
+                else if (cell[d] > A.box.dom_hi[d])
+                    cell[d] -= A.G.n[d];
+            }
+            st = ST_KEEP;
+        }
+        else if (st == ST_DROP)
+        {
+            cell[0] = DEAD_CELL;
+            atomicAdd(A.dropped, 1u);
+        }
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+    {
+        out.ic[d][i] = cell[d];
+        out.de[d][i] = delta[d];
+    }
+    out.v[0][i] = v[0];
+    out.v[1][i] = v[1];
+    out.v[2][i] = v[2];
+    if (outOfPlace)
+    {
+        out.w[i] = w;
+        out.q[i] = q;
+    }
+    if (A.status)
+        A.status[i] = st;
+}
+
 // One particle of updatePopulations: prePush, gather, Boris, postPush (boris.hpp:93-138), the
 // selection of ion_updater.hpp:169-295, the deposit and, in mode all, the write-back. Dead slots
 // (lost particles, empty slots of segmented storage) are skipped, and dropped by a compaction.
-template<int D, int O, bool RN = false>
+// LEAN: few loads and atomics in flight, for a rare path inside a kernel that needs the registers.
+template<int D, int O, bool RN = false, bool LEAN = false>
 __device__ __forceinline__ void pushLoaded(PushArgs const& A, PView const& out, bool outOfPlace,
                                            unsigned long long i, Part<D> const& P,
                                            TileView const& T, int copy, Acc<D, O>& acc)
@@ -338,62 +511,21 @@ __device__ __forceinline__ void pushLoaded(PushArgs const& A, PView const& out, 
     v[2] = P.v[2];
     double const w = P.w, q = P.q;
 
-    bool deposit = true, sel1 = true, inDom = true;
+    bool deposit = true, sel1 = true;
     uint8_t st   = ST_KEEP;
     if (A.pushOn)
     {
-        double bd, bv;
-        // prePushStep_ (boris.hpp:180-216)
-        if (!advancePosition<D>(cell, delta, v, A.hdtdx, bd, bv))
-        {
-            raiseError(A.err, 3u, 1u, i, bd, bv, A.kind, A.pop);
+        Stencil<D, O> s;
+        if (!prePush<D, O, true>(A, i, cell, delta, v, sel1, s))
             return;
-        }
-        // first selector: noop (domain) or inGhostBox (level ghosts)
-        sel1 = A.kind == KIND_DOMAIN ? true : inBox(cell, A.box.gh_lo, A.box.gh_hi, D);
         if (sel1)
         {
-            Stencil<D, O> s;
-            makeStencil<D, O>(G, cell, delta, s);
-            bool safe = true;
-#pragma unroll
-            for (int d = 0; d < D; ++d)
-            {
-                int const icl = cell[d] - (G.lower[d] - G.g);
-                safe          = safe && icl >= G.safeLo[d] && icl <= G.safeHi[d];
-            }
-            if (!safe
-                && (!stencilInside<D, O>(G, s, QEX) || !stencilInside<D, O>(G, s, QBX)
-                    || !stencilInside<D, O>(G, s, QEY) || !stencilInside<D, O>(G, s, QBY)
-                    || !stencilInside<D, O>(G, s, QEZ) || !stencilInside<D, O>(G, s, QBZ)))
-            {
-                raiseError(A.err, 4u, 2u, i, delta[0], v[0], A.kind, A.pop);
-                return;
-            }
             double E[3], B[3];
-            gatherEB<D, O>(G, A.em, s, E, B);
-            borisAccelerate(v, E, B, q, A.dto2m);
-            // postPushStep_ (boris.hpp:218-234)
-            if (!advancePosition<D>(cell, delta, v, A.hdtdx, bd, bv))
-            {
-                raiseError(A.err, 3u, 2u, i, bd, bv, A.kind, A.pop);
+            gatherEB<D, O, LEAN>(G, A.em, s, E, B);
+            if (!postPush<D, true>(A, i, cell, delta, v, q, E, B))
                 return;
-            }
         }
-        // what is deposited and what the array keeps (ion_updater.hpp:169-295)
-        inDom = inBox(cell, A.box.dom_lo, A.box.dom_hi, D);
-        if (A.kind == KIND_DOMAIN)
-        {
-            bool const nl = inNLGB(cell, A.box, D);
-            deposit       = nl;
-            st            = inDom ? ST_KEEP : (nl ? ST_LEAVE : ST_DROP);
-        }
-        else
-        {
-            deposit = sel1 && inDom;
-            bool const layer = sel1 && !inDom && inBox(cell, A.box.gh_lo, A.box.gh_hi, D);
-            st = !sel1 ? ST_DROP : (inDom ? ST_EXPORT : (layer ? ST_KEEP : ST_DROP));
-        }
+        selectPushed<D>(A, cell, sel1, deposit, st);
     }
 
     if (deposit)
@@ -408,11 +540,7 @@ __device__ __forceinline__ void pushLoaded(PushArgs const& A, PView const& out, 
             raiseError(A.err, 4u, 3u, i, delta[0], v[0], A.kind, A.pop);
         else
         {
-            dd.val[0] = 1. * w * A.coef;
-            dd.val[1] = q * w * A.coef;
-            dd.val[2] = v[0] * w * A.coef;
-            dd.val[3] = v[1] * w * A.coef;
-            dd.val[4] = v[2] * w * A.coef;
+            depositValues(w, q, v, A.coef, dd.val);
             if constexpr (C::ACC)
             {
                 // same cell as the window -> accumulate; else flush and restart there
@@ -422,7 +550,7 @@ __device__ __forceinline__ void pushLoaded(PushArgs const& A, PView const& out, 
                     same = same && acc.base[d] == cell[d] - (G.lower[d] - G.g) - C::WB;
                 if (!same)
                 {
-                    accFlush<D, O>(acc, G, T, copy, A.mom);
+                    accFlush<D, O, RN>(acc, G, T, copy, A.mom);
                     accZero(acc);
 #pragma unroll
                     for (int d = 0; d < D; ++d)
@@ -432,66 +560,28 @@ __device__ __forceinline__ void pushLoaded(PushArgs const& A, PView const& out, 
                 accAdd<D, O>(acc, dd);
             }
             else
-                depositOne<D, O, RN>(dd, G, T, copy, A.mom);
+                depositOne<D, O, RN, LEAN>(dd, G, T, copy, A.mom);
         }
     }
 
     if (A.pushOn && A.mode == MODE_ALL)
-    {
-        if (A.periodicWrap && A.kind == KIND_DOMAIN)
-        {
-            if (st == ST_LEAVE)
-            {
-                // fillIonGhostParticles: the leaver re-enters through the periodic image
-#pragma unroll
-                for (int d = 0; d < D; ++d)
-                {
-                    if (cell[d] < A.box.dom_lo[d])
-                        cell[d] += G.n[d];
-                    else if (cell[d] > A.box.dom_hi[d])
-                        cell[d] -= G.n[d];
-                }
-                st = ST_KEEP;
-            }
-            else if (st == ST_DROP)
-            {
-                cell[0] = DEAD_CELL;
-                atomicAdd(A.dropped, 1u);
-            }
-        }
-#pragma unroll
-        for (int d = 0; d < D; ++d)
-        {
-            out.ic[d][i] = cell[d];
-            out.de[d][i] = delta[d];
-        }
-        out.v[0][i] = v[0];
-        out.v[1][i] = v[1];
-        out.v[2][i] = v[2];
-        if (outOfPlace)
-        {
-            out.w[i] = w;
-            out.q[i] = q;
-        }
-        if (A.status)
-            A.status[i] = st;
-    }
+        storePushed<D>(A, out, outOfPlace, i, cell, delta, v, w, q, st);
 }
 
-template<int D, int O, bool RN = false>
+template<int D, int O, bool RN = false, bool LEAN = false>
 __device__ __forceinline__ void pushParticle(PushArgs const& A, PView const& in, PView const& out,
                                              unsigned long long i, TileView const& T, int copy,
                                              Acc<D, O>& acc)
 {
     Part<D> P;
     loadPart<D>(in, i, P);
-    pushLoaded<D, O, RN>(A, out, out.w != in.w, i, P, T, copy, acc);
+    pushLoaded<D, O, RN, LEAN>(A, out, out.w != in.w, i, P, T, copy, acc);
 }
 
-template<int TB = BLOCK>
+template<bool RN = false, int TB = BLOCK>
 __device__ __forceinline__ void zeroTile(double* lds, TileSpec const& S)
 {
-    for (int x = threadIdx.x; x < 5 * S.copies * S.stride; x += TB)
+    for (int x = threadIdx.x; x < (RN ? 4 : 5) * S.copies * S.stride; x += TB)
         lds[x] = 0.;
 }
 
@@ -512,12 +602,12 @@ __device__ __forceinline__ void flushTile(Geom const& G, TileView const& T, int 
             if (RN && m == 1)
             {
                 for (int c = 0; c < T.copies; ++c)
-                    val += T.mom(0, c)[x];
+                    val += T.mom<RN>(0, c)[x];
                 val *= charge;
             }
             else
                 for (int c = 0; c < T.copies; ++c)
-                    val += T.mom(m, c)[x];
+                    val += T.mom<RN>(m, c)[x];
             if (val != 0.)
             {
                 if (node < 0)
@@ -600,7 +690,7 @@ __global__ __launch_bounds__(BLOCK) void k_push(PushArgs A, PView in, PView out)
             pushParticle<D, O>(A, in, out, i, T, copy, acc);
     }
     if constexpr (C::ACC)
-        accFlush<D, O>(acc, G, T, copy, A.mom);
+        accFlush<D, O, false>(acc, G, T, copy, A.mom);
     __syncthreads();
     flushTile<D>(G, T, A.tile.nodes, A.mom);
 }
@@ -622,7 +712,7 @@ __device__ __forceinline__ void pushPiece(PushArgs const& A, PView const& in, do
     int const lane = t & 63;
     int const copy = lane & (A.tile.copies - 1);
 
-    zeroTile<pc::SEG_BLOCK>(lds, A.tile);
+    zeroTile<RN, pc::SEG_BLOCK>(lds, A.tile);
     // the tile covers the segment's cells with host-chosen margins (stencil, one cell of
     // motion, drift since the sort); the overflow segment has no cell range
     TileView T;
@@ -637,7 +727,7 @@ __device__ __forceinline__ void pushPiece(PushArgs const& A, PView const& in, do
         pushParticle<D, O, RN>(A, in, out, off + static_cast<unsigned long long>(r) * LANES + lane, T,
                                copy, acc);
     if constexpr (C::ACC)
-        accFlush<D, O>(acc, G, T, copy, A.mom);
+        accFlush<D, O, RN>(acc, G, T, copy, A.mom);
     __syncthreads();
     flushTile<D, RN, pc::SEG_BLOCK>(G, T, A.tile.nodes, A.mom, A.charge);
 }
@@ -670,40 +760,357 @@ void k_push_seg(PushArgs A, PView in)
 }
 
 // ---------------------------------------------------------------------------------------------
-// fused push + deposit over cell-segmented storage, one workgroup per segment with all its rows
-// (the staged 3D path, segments of 4x4x4 cells): wavefront w takes rows w, w + 4, ..., so that
-// each instruction's 64 lanes walk 64 cells of the segment; the tile covers the segment with the
-// stencil and one cell of motion on each side; the overflow segment (number nsegs) deposits
-// straight into HBM. RN: the population has one charge, the tile leaves the charge density out
-// and its flush takes the charge times n
+// fused push + deposit over cell-ordered segmented storage, A.split workgroups per segment (3D,
+// segments of 4x4x4 cells): the rows of a segment hold its particles in cell order, each wavefront
+// takes a run of them, and the particles of one cell deposit together on the matrix cores
+// (phx_cell_deposit.hpp). The tile covers the segment with the stencil and one cell of motion on
+// each side, and E and B of the segment's surroundings are staged beside it. A particle that leaves
+// the domain, the tile or the stage is left as it is and noted in a list in LDS; the listed
+// particles of the whole workgroup are pushed 64 to a wavefront, gathering from HBM, and deposit one
+// by one, into the tile or straight into HBM (the overflow segment, number nsegs, has no tile). RN:
+// the population has one charge: the particles' own is not read, and the tile leaves the charge
+// density out, its flush taking the charge times n.
 // ---------------------------------------------------------------------------------------------
-template<int D, int O, bool RN>
-__global__ __launch_bounds__(BLOCK) void k_push_segwg(PushArgs A, PView in)
+namespace
 {
-    extern __shared__ double lds[];
-    if (A.G.stopped())
+// address of a row of one particle component, kept in scalar registers (the lane is the offset of
+// the access; folded into a per-lane base the ten components took 20 vector registers)
+template<class R>
+using GlobalPtr = __attribute__((address_space(1))) R*;
+template<class R>
+__device__ __forceinline__ GlobalPtr<R> rowOf(R* p, unsigned long long row)
+{
+    GlobalPtr<R> q = (GlobalPtr<R>)(p + row);
+    asm volatile("" : "+s"(q));
+    return q;
+}
+
+// one row of the segment: the particles of 64 consecutive slots
+template<bool RN>
+__device__ __forceinline__ void loadRow(PView const& in, unsigned long long row, unsigned int lane, Part<3>& p)
+{
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        p.cell[d] = rowOf(in.ic[d], row)[lane];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        p.delta[d] = rowOf(in.de[d], row)[lane];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        p.v[d] = rowOf(in.v[d], row)[lane];
+    p.w = rowOf(in.w, row)[lane];
+    if constexpr (!RN)
+        p.q = rowOf(in.q, row)[lane];
+}
+
+struct CellArgs
+{
+    PushArgs A;
+    PView v;
+};
+
+// the kernel's arguments, read again from the argument segment: a use after a long stretch of code
+// reloads what it needs instead of holding registers over it
+__device__ __forceinline__ CellArgs const& cellArgs()
+{
+    auto* p = (__attribute__((address_space(4))) char const*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(CellArgs const*)p;
+}
+
+// half a step of the position without a branch; false when it moves more than two cells
+__device__ __forceinline__ bool halfStep(int* cell, double* delta, double const* v, double const* hdtdx)
+{
+    bool ok = true;
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+        double const dl = delta[d] + hdtdx[d] * v[d];
+        ok              = ok & !(fabs(dl) > 2);
+        int const ic    = static_cast<int>(floor(dl));
+        delta[d]        = dl - ic;
+        cell[d] += ic;
+    }
+    return ok;
+}
+
+// E and B of the segment's surroundings in LDS: component f (Ex .. Bz) on `nodes` nodes from `org`,
+// row-major with extents ext; nodes beyond a component's array repeat its last ones (no stencil
+// inside the domain reaches them)
+template<int TB>
+__device__ __forceinline__ void stageFields(PushArgs const& A, double* em, int const* org, int e1, int e2,
+                                            int nodes)
+{
+    Geom const& G = A.G;
+    int const e12 = e1 * e2;
+    for (int x = threadIdx.x; x < nodes; x += TB)
+    {
+        int const i = x / e12, r = x - i * e12;
+        int const j = r / e2, k = r - j * e2;
+#pragma unroll
+        for (int f = 0; f < 6; ++f)
+        {
+            int const q    = f < 3 ? QEX + f : QBX + f - 3;
+            int const n[3] = {org[0] + i, org[1] + j, org[2] + k};
+            int c[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+                c[d] = min(max(n[d], 0), G.shape[q][d] - 1);
+            em[f * nodes + x] = (f < 3 ? A.em.E[f] : A.em.B[f - 3])[G.idx(q, c[0], c[1], c[2])];
+        }
+    }
+}
+
+// E and B at a particle from the staged fields; rel: its cell less the stage's first node
+template<int O>
+__device__ __forceinline__ void gatherStaged(double const* em, int e1, int e2, int nodes, int const* rel,
+                                             double const* delta, double* E, double* B)
+{
+    constexpr int S = O + 1;
+    double w[2][3][S];
+    int st[2][3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+        st[CP][d] = rel[d] - pc::splineStencil<O>(CP, delta[d], w[CP][d]);
+        st[CD][d] = rel[d] - pc::splineStencil<O>(CD, delta[d], w[CD][d]);
+    }
+#pragma unroll
+    for (int f = 0; f < 6; ++f)
+    {
+        int const q  = f < 3 ? QEX + f : QBX + f - 3;
+        int const cx = centering(q, 0), cy = centering(q, 1), cz = centering(q, 2);
+        double const* const p = em + f * nodes + (st[cx][0] * e1 + st[cy][1]) * e2 + st[cz][2];
+        double r = 0.;
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+        {
+            double y = 0.;
+#pragma unroll
+            for (int j = 0; j < S; ++j)
+            {
+                double z = 0.;
+#pragma unroll
+                for (int k = 0; k < S; ++k)
+                    z = __builtin_fma(p[(i * e1 + j) * e2 + k], w[cz][2][k], z);
+                y = __builtin_fma(z, w[cy][1][j], y);
+            }
+            r = __builtin_fma(y, w[cx][0][i], r);
+        }
+        (f < 3 ? E[f] : B[f - 3]) = r;
+    }
+}
+} // namespace
+
+// FIX: the stage has the extents of a 4x4x4 segment (the stencils' offsets are then constants)
+template<int O, bool RN, bool FIX>
+__global__ __launch_bounds__(CellCfg<O>::BLOCK) __attribute__((amdgpu_waves_per_eu(CellCfg<O>::WAVES)))
+void k_push_cell(CellArgs K)
+{
+    using C             = pc::CellWin<O, RN>;
+    constexpr int CB    = CellCfg<O>::BLOCK;
+    constexpr bool NEXT = CellCfg<O>::PREFETCH;
+    // 16-byte aligned: the hand-over buffers are read as pairs of words (a pair read 8 bytes off
+    // took 8 times as long)
+    extern __shared__ __align__(16) double cellLds[];
+    double* const lds = cellLds;
+    __shared__ unsigned int list[CELL_LIST];
+    __shared__ unsigned int listed;
+    if (K.A.G.stopped())
         return;
-    Geom const& G          = A.G;
-    unsigned int const seg = pc::xcdItem(blockIdx.x, gridDim.x);
-    int const t            = threadIdx.x;
-    int const lane         = t & 63;
-    unsigned long long const off = A.st.off[seg];
-    unsigned int const R         = A.st.rows[seg];
-    zeroTile(lds, A.tile);
+    unsigned int const item = pc::xcdItem(blockIdx.x, gridDim.x);
+    unsigned int const seg  = item / K.A.split;
+    unsigned int const lane = threadIdx.x & 63u;
+    unsigned int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned long long const off = K.A.st.off[seg];
+    unsigned int const R         = K.A.st.rows[seg];
+    unsigned int const part = item - seg * K.A.split;
+    unsigned int const rA   = static_cast<unsigned int>(static_cast<unsigned long long>(R) * part / K.A.split);
+    unsigned int const rows
+        = static_cast<unsigned int>(static_cast<unsigned long long>(R) * (part + 1) / K.A.split) - rA;
+    if (rows == 0)
+        return;
+    // stage pitches: odd along z, so that stencils of different cells start in different banks
+    constexpr int EX  = CELL_STAGE<O>;
+    int const e1      = FIX ? EX : K.A.tile.emExt[1], e2 = (FIX ? EX : K.A.tile.emExt[2]) | 1;
+    int const emNodes = (FIX ? EX : K.A.tile.emExt[0]) * e1 * e2;
+    double* const em  = lds + (RN ? 4 : 5) * K.A.tile.stride;
+    double* const buf = em + K.A.tile.emStride + wave * C::BUF;
+    zeroTile<RN, CB>(lds, K.A.tile);
+    if (threadIdx.x == 0)
+        listed = 0u;
     TileView T;
-    tileView(T, lds, A.tile);
-    pc::segTileOrigin<D>(G, A.sg, A.tile, seg, T.org);
+    tileView(T, lds, K.A.tile);
+    pc::segTileOrigin<3>(K.A.G, K.A.sg, K.A.tile, seg, T.org);
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+        T.org[d] = __builtin_amdgcn_readfirstlane(T.org[d]); // the same in every lane: scalar from here on
+    int const p2 = T.pitch[2], p12 = T.pitch[1] * T.pitch[2];
+    bool const push   = K.A.pushOn;
+    bool const writes = push && K.A.mode == MODE_ALL;
+    // per direction: AMR cell of the deposit tile's and of the stage's first cell, and the number
+    // of cells whose windows (stencils) they hold; the stage's cells are clipped to those whose
+    // stencils lie in the arrays
+    int tileCell[3], tileCells[3], emCell[3], emLow[3], emCells[3], emOrg[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d)
+    {
+        int const shift = K.A.G.lower[d] - K.A.G.g; // AMR cell of local cell 0
+        tileCell[d]     = T.org[d] + C::WB + shift;
+        tileCells[d]    = max(T.ext[d] - C::W + 1, 0);
+        emOrg[d]        = T.org[d] + K.A.tile.emLo[d];
+        emCell[d]       = emOrg[d] + shift;
+        int const lo    = max(emOrg[d] - cellGatherLo(O), K.A.G.safeLo[d]);
+        int const hi    = min(emOrg[d] - cellGatherLo(O) + K.A.tile.emExt[d] - cellGatherNodes(O), K.A.G.safeHi[d]);
+        emLow[d]        = lo + shift;
+        emCells[d]      = max(hi - lo + 1, 0);
+    }
+    double const h[3] = {K.A.hdtdx[0], K.A.hdtdx[1], K.A.hdtdx[2]};
+    double const dto2m = K.A.dto2m, coef = K.A.coef, charge = K.A.charge;
+    int const dom[6] = {K.A.box.dom_lo[0], K.A.box.dom_lo[1], K.A.box.dom_lo[2],
+                        K.A.box.dom_hi[0], K.A.box.dom_hi[1], K.A.box.dom_hi[2]};
+    if (push)
+        stageFields<CB>(K.A, em, emOrg, e1, e2, emNodes);
     __syncthreads();
-    Acc<D, O> acc;
-    if constexpr (Cfg<D, O>::ACC)
-        accZero(acc);
-#pragma unroll 1
-    for (unsigned int r = static_cast<unsigned int>(t >> 6); r < R; r += NW)
-        pushParticle<D, O, RN>(A, in, in, off + static_cast<unsigned long long>(r) * LANES + lane, T, 0, acc);
-    if constexpr (Cfg<D, O>::ACC)
-        accFlush<D, O>(acc, G, T, 0, A.mom);
-    __syncthreads();
-    flushTile<D, RN>(G, T, A.tile.nodes, A.mom, A.charge);
+
+    unsigned int r          = rA + rows * wave / CellCfg<O>::NW;
+    unsigned int const rEnd = rA + rows * (wave + 1) / CellCfg<O>::NW;
+    do
+    {
+        C acc;
+        acc.zero();
+        int cur = -1; // tile node of the accumulated window's origin
+        Part<3> next;
+        if (NEXT && r < rEnd)
+            loadRow<RN>(K.v, off + static_cast<unsigned long long>(r) * LANES, lane, next);
+        for (; r < rEnd; ++r)
+        {
+            // until the list might overflow (each wavefront that still finds room may add 64)
+            if (__builtin_amdgcn_readfirstlane(*static_cast<unsigned int volatile*>(&listed)) > CELL_LIST - CB)
+                break;
+            unsigned long long const row = off + static_cast<unsigned long long>(r) * LANES;
+            Part<3> P;
+            if constexpr (NEXT)
+            {
+                P = next;
+                if (r + 1 < rEnd)
+                    loadRow<RN>(K.v, row + LANES, lane, next); // in flight over this row's work
+            }
+            else
+                loadRow<RN>(K.v, row, lane, P);
+            double const q  = RN ? charge : P.q;
+            bool const live = P.cell[0] != DEAD_CELL;
+            bool ok         = live;
+            if (push)
+            {
+                ok = halfStep(P.cell, P.delta, P.v, h) & ok;
+                int rel[3];
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                {
+                    ok     = ok & (static_cast<unsigned int>(P.cell[d] - emLow[d]) < static_cast<unsigned int>(emCells[d]));
+                    rel[d] = P.cell[d] - emCell[d];
+                }
+                double E[3] = {0., 0., 0.}, B[3] = {0., 0., 0.};
+                if (ok)
+                    gatherStaged<O>(em, e1, e2, emNodes, rel, P.delta, E, B);
+                borisAccelerate(P.v, E, B, q, dto2m);
+                ok = halfStep(P.cell, P.delta, P.v, h) & ok;
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    ok = ok & (P.cell[d] >= dom[d]) & (P.cell[d] <= dom[3 + d]);
+            }
+            // the tile node of the window's origin; a value that is not finite (it would reach the
+            // whole window) deposits by itself
+            ok = ok & __builtin_isfinite(P.w * coef) & (RN || __builtin_isfinite(q * P.w * coef));
+            int rel[3];
+#pragma unroll
+            for (int d = 0; d < 3; ++d)
+            {
+                rel[d] = P.cell[d] - tileCell[d];
+                ok = ok & (static_cast<unsigned int>(rel[d]) < static_cast<unsigned int>(tileCells[d]))
+                     & (P.delta[d] == P.delta[d]) & __builtin_isfinite(P.v[d] * P.w * coef);
+            }
+            int const key = ok ? rel[0] * p12 + rel[1] * p2 + rel[2] : -1;
+            // the half rows in turn: first the accumulated window's cell, then every other cell
+#pragma unroll
+            for (int half = 0; half < 2; ++half)
+            {
+                unsigned int rest = static_cast<unsigned int>(__ballot(ok) >> (32 * half));
+                if (rest == 0u)
+                    continue;
+                pc::cellStage<O, RN>(buf, half, ok, P.delta, P.w, q, P.v, coef);
+                unsigned int m = cur < 0 ? 0u : static_cast<unsigned int>(__ballot(key == cur) >> (32 * half));
+                if (m)
+                    pc::cellAdd<O, RN>(buf, m, acc);
+                rest &= ~m;
+                while (rest)
+                {
+                    int const p = __builtin_ctz(rest);
+                    int const c = __builtin_amdgcn_readlane(key, p + 32 * half);
+                    m           = static_cast<unsigned int>(__ballot(key == c) >> (32 * half)) & rest;
+                    rest &= ~m;
+                    int const n = __popc(m);
+                    if (n >= CELL_MOVE || cur < 0)
+                    {
+                        if (cur >= 0)
+                            pc::cellFlush<O, RN>(acc, lds, T.stride, cur, p12, p2);
+                        acc.zero();
+                        cur = c;
+                        pc::cellAdd<O, RN>(buf, m, acc);
+                    }
+                    else if (n >= CELL_GROUP)
+                    {
+                        C one;
+                        one.zero();
+                        pc::cellAdd<O, RN>(buf, m, one);
+                        pc::cellFlush<O, RN>(one, lds, T.stride, c, p12, p2);
+                    }
+                    else
+                        pc::cellAddOne<O, RN>(buf, p, lds, T.stride, c, p12, p2);
+                }
+            }
+            unsigned long long const left = __ballot(live && !ok);
+            if (left)
+            {
+                unsigned int base = 0;
+                if (lane == 0)
+                    base = atomicAdd(&listed, static_cast<unsigned int>(__popcll(left)));
+                base = __builtin_amdgcn_readfirstlane(base);
+                if ((left >> lane) & 1ull)
+                    list[base + __popcll(left & ((1ull << lane) - 1ull))] = r * LANES + lane;
+            }
+            if (writes)
+            {
+                if (ok)
+                {
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+                    {
+                        rowOf(K.v.ic[d], row)[lane] = P.cell[d];
+                        rowOf(K.v.de[d], row)[lane] = P.delta[d];
+                        rowOf(K.v.v[d], row)[lane]  = P.v[d];
+                    }
+                }
+                uint8_t* const status = K.A.status;
+                if (status && (ok || !live))
+                    rowOf(status, row)[lane] = live ? ST_KEEP : ST_DROP;
+            }
+        }
+        if (cur >= 0)
+            pc::cellFlush<O, RN>(acc, lds, T.stride, cur, p12, p2);
+        __syncthreads();
+        unsigned int const n = listed;
+        CellArgs const& L    = cellArgs();
+        Acc<3, O> none;
+        for (unsigned int x = threadIdx.x; x < n; x += CB)
+            pushParticle<3, O, RN, true>(L.A, L.v, L.v, off + list[x], T, 0, none);
+        __syncthreads();
+        if (threadIdx.x == 0)
+            listed = 0u;
+    } while (__syncthreads_or(r < rEnd));
+    PushArgs const& A = cellArgs().A;
+    flushTile<3, RN, CB>(A.G, T, A.tile.nodes, A.mom, A.charge);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -901,19 +1308,46 @@ __global__ __launch_bounds__(BLOCK) void k_seg_zero(unsigned int* __restrict__ p
 }
 
 // particles per cell key, and the rank of each particle among those of its key (the order in
-// which the atomics reached the count): the scatter places particle i at row rank[i] of its cell
+// which the atomics reached the count): the scatter places particle i at position rank[i] of its cell.
+// Storage sorted before in the dense order holds most particles of a wavefront in one or a few cells:
+// the lanes of up to SAME_KEYS cells then add with one atomic per cell (lane by lane the adds of one
+// address queue up: 1.68 ms for 16.8 M particles, 0.30 ms when the lanes' cells differ), the other
+// lanes one by one.
+constexpr int SAME_KEYS = 8;
 template<class V>
 __global__ __launch_bounds__(BLOCK) void k_seg_count(SegGeom S, V v, unsigned long long n,
                                                      unsigned int* __restrict__ counts,
                                                      unsigned int* __restrict__ rank)
 {
     unsigned long long const i = static_cast<unsigned long long>(blockIdx.x) * BLOCK + threadIdx.x;
-    if (i >= n)
-        return;
     int c[3], p = 0;
-    unsigned int const key = cellKey(S, v, i, c, p);
+    unsigned int const key = i < n ? cellKey(S, v, i, c, p) : DEAD_KEY;
+    unsigned int add = 1, before = 0; // what the lane adds, and the particles before it in its group
+    int const lane = static_cast<int>(threadIdx.x & 63u);
+    int lead       = lane;
+    if (S.dense)
+    {
+        unsigned long long rest = __ballot(key != DEAD_KEY);
+        for (int g = 0; g < SAME_KEYS && rest; ++g)
+        {
+            int const first            = __builtin_ctzll(rest);
+            unsigned int const k       = __builtin_amdgcn_readlane(key, first);
+            unsigned long long const m = __ballot(key == k);
+            if (key == k)
+            {
+                lead   = first;
+                add    = lane == first ? static_cast<unsigned int>(__popcll(m)) : 0u;
+                before = static_cast<unsigned int>(__popcll(m & ((1ull << lane) - 1ull)));
+            }
+            rest &= ~m;
+        }
+    }
+    unsigned int base = 0;
+    if (key != DEAD_KEY && add)
+        base = atomicAdd(counts + key, add);
+    base = __shfl(base, lead);
     if (key != DEAD_KEY)
-        rank[i] = atomicAdd(counts + key, 1u);
+        rank[i] = base + before;
 }
 
 // rows of each segment, ceil(particles / 64), and its work items; the count of each cell becomes
@@ -1029,7 +1463,7 @@ constexpr unsigned int NO_PARTICLE = 0xFFFFFFFFu;
 
 // the slot of source particle i, recorded as perm[slot] = i: position p of segment s (R rows) is
 // row p % R, lane p / R, so that the lanes of a row are R positions apart in the segment's cell
-// order; the overflow segment packs its particles in rank order
+// order, or slot p (dense); the overflow segment packs its particles in rank order
 template<class V>
 __global__ __launch_bounds__(BLOCK) void k_seg_perm(SegGeom S, V src, unsigned long long n,
                                                     unsigned int const* __restrict__ rank,
@@ -1053,7 +1487,7 @@ __global__ __launch_bounds__(BLOCK) void k_seg_perm(SegGeom S, V src, unsigned l
         segLane(S, pt, c, seg, lane);
         unsigned int const p = first[key] + rank[i];
         unsigned int const R = rows[seg];
-        j = off[seg] + static_cast<unsigned long long>(p % R) * LANES + p / R;
+        j = off[seg] + (S.dense ? p : static_cast<unsigned long long>(p % R) * LANES + p / R);
     }
     else
         j = off[S.nsegs] + rank[i];
@@ -1071,10 +1505,10 @@ __global__ __launch_bounds__(BLOCK) void k_seg_pad(SegGeom S, unsigned int const
     unsigned int const R     = rows[s];
     unsigned int const slots = R * LANES;
     unsigned int const T     = total[s];
-    bool const packed        = s < static_cast<unsigned int>(S.nsegs);
+    bool const columns       = s < static_cast<unsigned int>(S.nsegs) && !S.dense;
     for (unsigned int x = threadIdx.x; x < slots; x += BLOCK)
     {
-        unsigned int const p = packed ? (x % LANES) * R + x / LANES : x;
+        unsigned int const p = columns ? (x % LANES) * R + x / LANES : x;
         if (p >= T)
             perm[off[s] + x] = NO_PARTICLE;
     }
@@ -1230,7 +1664,7 @@ SegPatch segPatchOf(int dim, int const* lo, int const* hi, int const* pref)
     return P;
 }
 
-TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies)
+TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies, int slabs)
 {
     TileSpec T{};
     T.copies = copies;
@@ -1244,7 +1678,7 @@ TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies)
     pc::tilePitch(T, dim, sg.rowPad);
     T.nodes  = T.ext[0] * T.pitch[1] * T.pitch[2];
     T.stride = (T.nodes + 15) / 16 * 16; // copies 16 words apart: neighbouring lanes' banks differ
-    T.bytes  = static_cast<unsigned int>(8 * 5 * copies * T.stride);
+    T.bytes  = static_cast<unsigned int>(8 * slabs * copies * T.stride);
     if (T.bytes > TILE_BYTES_MAX)
     {
         // no room: every deposit goes straight to HBM
@@ -1256,7 +1690,7 @@ TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies)
         T.lo[0]  = -0x10000000;
         T.nodes  = 1;
         T.stride = 16;
-        T.bytes  = static_cast<unsigned int>(8 * 5 * copies * T.stride);
+        T.bytes  = static_cast<unsigned int>(8 * slabs * copies * T.stride);
     }
     return T;
 }
@@ -1275,7 +1709,15 @@ unsigned int segItemsCap(SegGeom const& sg, unsigned long long capacity)
 template<int D, int O>
 static void launchPushT(PushArgs const& A, PView const& in, PView const& out, hipStream_t s)
 {
-    if (A.segOn)
+    if constexpr (D == 3)
+    {
+        if (A.segOn)
+        {
+            launchPushCell(A, in, s);
+            return;
+        }
+    }
+    else if (A.segOn)
     {
         // segmented arrays are pushed in place (out is in)
         if (A.rhoFromN)
@@ -1429,63 +1871,116 @@ void launchCompact(PView const& src, PView const& dst, uint8_t const* status, un
                                           wrap);
 }
 
-// tile of the workgroup-per-segment push: the largest segment plus the stencil and one cell of
-// motion below (2 nodes) and above (order + 2 nodes), `slabs` moment slabs, the pitches of
-// dimensions 1 and 2 padded to a multiple of `pad` nodes
-TileSpec segwgTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad)
+// tile of the cell-grouped 3D push: the window of every cell of the largest segment and of the
+// cells around it (one cell of motion), and the staged fields of the segment's gather
+TileSpec cellTileShape(int order, SegGeom const& sg, int slabs, int pad)
 {
     TileSpec T{};
     T.copies = 1;
+    int emNodes = 1;
+    bool fix    = true; // the stage of a 4x4x4 segment holds every segment's
+    for (int d = 0; d < 3; ++d)
+        fix = fix && sg.maxSeg[d] <= 4;
+    T.emFix = fix;
     for (int d = 0; d < 3; ++d)
     {
-        T.lo[d]    = d < dim ? 2 : 0;
-        T.ext[d]   = d < dim ? sg.maxSeg[d] + 2 + order + 2 : 1;
+        T.lo[d]    = order == 1 ? 1 : 2;
+        T.ext[d]   = sg.maxSeg[d] + (order == 1 ? 3 : 5);
         T.pitch[d] = T.ext[d];
+        T.emLo[d]  = T.lo[d] + cellGatherLo(order) - 1;
+        T.emExt[d] = (fix ? 4 : sg.maxSeg[d]) + 1 + cellGatherNodes(order);
+        emNodes *= d == 2 ? T.emExt[d] | 1 : T.emExt[d];
     }
+    T.emStride = (6 * emNodes + 15) / 16 * 16;
+    // the hand-over buffers of the workgroup's wavefronts
+    unsigned int const waves = static_cast<unsigned int>(cellBlock(order)) / LANES;
+    unsigned int const rest = 8u * static_cast<unsigned int>(T.emStride)
+                              + waves * 8u * static_cast<unsigned int>(pc::WSTR * ((order == 1 ? 6 : 12) + slabs));
     auto size = [&]() {
         T.nodes  = T.ext[0] * T.pitch[1] * T.pitch[2];
         T.stride = (T.nodes + 15) / 16 * 16;
-        T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride);
+        T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride) + rest;
     };
-    if (dim == 3 && pad > 1)
+    if (pad > 1)
     {
         // pitches of dimensions 1 and 2 padded to a multiple of pad nodes (the padding nodes are
         // never deposited into: the flush skips them as zeros); dropped if the tile outgrows LDS
         for (int d = 1; d < 3; ++d)
             T.pitch[d] = (T.ext[d] + pad - 1) / pad * pad;
         size();
-        if (T.bytes > TILE_BYTES_MAX)
+        if (T.bytes > CELL_LDS_MAX)
             for (int d = 1; d < 3; ++d)
                 T.pitch[d] = T.ext[d];
     }
     size();
-    if (T.bytes > TILE_BYTES_MAX)
+    if (T.bytes > CELL_LDS_MAX)
     {
-        // no room: every deposit goes straight to HBM
+        // no room: every particle is pushed by itself and its deposits go straight to HBM
+        T.emFix = 0;
         for (int d = 0; d < 3; ++d)
         {
             T.ext[d]   = 1;
             T.pitch[d] = 1;
+            T.emExt[d] = 1;
         }
-        T.lo[0]  = -0x10000000;
-        T.nodes  = 1;
-        T.stride = 16;
-        T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride);
+        T.lo[0]    = -0x10000000;
+        T.emLo[0]  = 0;
+        T.nodes    = 1;
+        T.stride   = 16;
+        T.emStride = 16;
+        T.bytes    = static_cast<unsigned int>(8 * (slabs * T.stride + T.emStride)) + NW * 8u * pc::WSTR * 17u;
     }
     return T;
 }
 
-void launchPushSegWG(PushArgs const& A, PView const& in, hipStream_t s)
+// workgroups per segment of the cell-grouped push: as many as give three rounds of the workgroups the
+// GPU holds at once, while each of a segment's wavefronts keeps two rows (a workgroup zeroes, stages
+// and flushes its tile whatever its rows)
+unsigned int cellSplit(int order, SegGeom const& sg, unsigned long long slots)
 {
-    unsigned int const grid = static_cast<unsigned int>(A.sg.nsegs) + 1u;
-    switch (A.G.dim * 10 + A.G.order)
+    unsigned long long const segs = static_cast<unsigned long long>(std::max(sg.nsegs, 1));
+    unsigned long long const held = CUS * (order == 3 ? 1 : 2);
+    unsigned long long const rows = slots / LANES / segs;
+    unsigned long long const most = rows / (2 * static_cast<unsigned long long>(cellBlock(order)) / LANES);
+    unsigned long long const want = (3 * held + segs - 1) / segs;
+    return static_cast<unsigned int>(std::max(1ull, std::min(want, most)));
+}
+
+template<int O, bool RN, bool FIX>
+static void launchPushCellT(PushArgs const& A, PView const& in, hipStream_t s)
+{
+    // more than 64 KB of dynamic LDS has to be allowed for the kernel (once per device)
+    static std::mutex mtx;
+    static bool allowed[64] = {};
+    int dev                 = 0;
+    if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64)
     {
-        case 31: A.rhoFromN ? k_push_segwg<3, 1, true><<<grid, BLOCK, A.tile.bytes, s>>>(A, in)
-                            : k_push_segwg<3, 1, false><<<grid, BLOCK, A.tile.bytes, s>>>(A, in); break;
-        case 32: A.rhoFromN ? k_push_segwg<3, 2, true><<<grid, BLOCK, A.tile.bytes, s>>>(A, in)
-                            : k_push_segwg<3, 2, false><<<grid, BLOCK, A.tile.bytes, s>>>(A, in); break;
-        case 33: A.rhoFromN ? k_push_segwg<3, 3, true><<<grid, BLOCK, A.tile.bytes, s>>>(A, in)
-                            : k_push_segwg<3, 3, false><<<grid, BLOCK, A.tile.bytes, s>>>(A, in); break;
+        std::lock_guard<std::mutex> lock(mtx);
+        if (!allowed[dev])
+            allowed[dev] = hipFuncSetAttribute(reinterpret_cast<void const*>(&k_push_cell<O, RN, FIX>),
+                                               hipFuncAttributeMaxDynamicSharedMemorySize, CELL_LDS_MAX)
+                           == hipSuccess;
+    }
+    unsigned int const grid = (static_cast<unsigned int>(A.sg.nsegs) + 1u) * A.split;
+    k_push_cell<O, RN, FIX><<<grid, CellCfg<O>::BLOCK, A.tile.bytes, s>>>(CellArgs{A, in});
+}
+
+template<int O>
+static void launchPushCellO(PushArgs const& A, PView const& in, hipStream_t s)
+{
+    if (A.rhoFromN)
+        A.tile.emFix ? launchPushCellT<O, true, true>(A, in, s) : launchPushCellT<O, true, false>(A, in, s);
+    else
+        A.tile.emFix ? launchPushCellT<O, false, true>(A, in, s) : launchPushCellT<O, false, false>(A, in, s);
+}
+
+void launchPushCell(PushArgs const& A, PView const& in, hipStream_t s)
+{
+    switch (A.G.order)
+    {
+        case 1: launchPushCellO<1>(A, in, s); break;
+        case 2: launchPushCellO<2>(A, in, s); break;
+        case 3: launchPushCellO<3>(A, in, s); break;
         default: break;
     }
 }

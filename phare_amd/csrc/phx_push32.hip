@@ -829,7 +829,7 @@ __global__ __launch_bounds__(BLOCK) void k_push32_lin(PushArgs A, PView32 v)
 } // namespace
 
 // the same over cell-segmented FP32 storage, one workgroup per segment with all its rows (the
-// staged 3D path's layout after its sorts; the FP64 family's k_push_segwg in FP32)
+// staged 3D path's layout after its sorts)
 template<int D, int O>
 __global__ __launch_bounds__(BLOCK) void k_push32_segwg(PushArgs A, PView32 v)
 {
@@ -868,6 +868,52 @@ __global__ __launch_bounds__(BLOCK) void k_push32_segwg(PushArgs A, PView32 v)
         pushSlot32<D, O, false>(A, K, v, off + static_cast<unsigned long long>(r) * LANES + lane, T, win);
     __syncthreads();
     flushTile32<D, BLOCK>(A, T);
+}
+
+// tile of the workgroup-per-segment push: the largest segment plus the stencil and one cell of
+// motion below (2 nodes) and above (order + 2 nodes), `slabs` moment slabs, the pitches of
+// dimensions 1 and 2 padded to a multiple of `pad` nodes
+TileSpec segwgTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad)
+{
+    TileSpec T{};
+    T.copies = 1;
+    for (int d = 0; d < 3; ++d)
+    {
+        T.lo[d]    = d < dim ? 2 : 0;
+        T.ext[d]   = d < dim ? sg.maxSeg[d] + 2 + order + 2 : 1;
+        T.pitch[d] = T.ext[d];
+    }
+    auto size = [&]() {
+        T.nodes  = T.ext[0] * T.pitch[1] * T.pitch[2];
+        T.stride = (T.nodes + 15) / 16 * 16;
+        T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride);
+    };
+    if (dim == 3 && pad > 1)
+    {
+        // pitches of dimensions 1 and 2 padded to a multiple of pad nodes (the padding nodes are
+        // never deposited into: the flush skips them as zeros); dropped if the tile outgrows LDS
+        for (int d = 1; d < 3; ++d)
+            T.pitch[d] = (T.ext[d] + pad - 1) / pad * pad;
+        size();
+        if (T.bytes > pc::TILE_BYTES_MAX)
+            for (int d = 1; d < 3; ++d)
+                T.pitch[d] = T.ext[d];
+    }
+    size();
+    if (T.bytes > pc::TILE_BYTES_MAX)
+    {
+        // no room: every deposit goes straight to HBM
+        for (int d = 0; d < 3; ++d)
+        {
+            T.ext[d]   = 1;
+            T.pitch[d] = 1;
+        }
+        T.lo[0]  = -0x10000000;
+        T.nodes  = 1;
+        T.stride = 16;
+        T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride);
+    }
+    return T;
 }
 
 void launchPush32SegWG(PushArgs const& A, PView32 const& v, hipStream_t s)
