@@ -113,7 +113,7 @@ struct phx_ctx
     double* Bold[3]    = {}; // SolverPPC::Bold_ (prepareStep)
     double* fluxSum[3] = {}; // SolverPPC::fluxSumE_ (E-centered)
     double* Ve[3]    = {};
-    double* Pe = nullptr, *rho = nullptr, *massD = nullptr, *tmp = nullptr;
+    double* Pe = nullptr, *rho = nullptr, *massD = nullptr;
     double* Vi[3] = {};
     Pop pops[PHX_MAX_POP];
     Store scratch;
@@ -477,24 +477,23 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
 
 long count(phx_ctx const* c, int q) { return c->G.size(q); }
 
-void zeroMoments(phx_ctx* c)
+FieldList momentList(phx_ctx const* c)
 {
+    FieldList F{};
     for (int p = 0; p < c->cfg.n_pop; ++p)
         for (int m = 0; m < 5; ++m)
-            launchZero(c->pops[p].mom[m], count(c, QMOM), c->stream);
+            F.f[F.n++] = c->pops[p].mom[m];
+    return F;
 }
+
+void zeroMoments(phx_ctx* c) { launchZeroList(momentList(c), count(c, QMOM), c->stream); }
 
 // fillFluxBorders + fillDensityBorders: sum = copy(moment); sum += periodic images; copy back
 phx_status fillMomentBorders(phx_ctx* c)
 {
     if (!c->patch.periodic)
         return PHX_OK;
-    for (int p = 0; p < c->cfg.n_pop; ++p)
-        for (int m = 0; m < 5; ++m)
-        {
-            launchCopy(c->pops[p].mom[m], c->tmp, count(c, QMOM), c->stream);
-            launchBorderSum(c->G, c->tmp, c->pops[p].mom[m], c->stream);
-        }
+    launchBorderSum(c->G, momentList(c), c->stream);
     return checkLaunch(c, "fillMomentBorders");
 }
 
@@ -502,21 +501,14 @@ phx_status fillIonBorders(phx_ctx* c)
 {
     if (!c->patch.periodic)
         return PHX_OK;
-    double* f[5] = {c->rho, c->massD, c->Vi[0], c->Vi[1], c->Vi[2]};
-    for (auto* x : f)
-    {
-        launchCopy(x, c->tmp, count(c, QMOM), c->stream);
-        launchBorderMax(c->G, c->tmp, x, c->stream);
-    }
+    launchBorderMax(c->G, FieldList{{c->rho, c->massD, c->Vi[0], c->Vi[1], c->Vi[2]}, 5}, c->stream);
     return checkLaunch(c, "fillIonBorders");
 }
 
 void fillGhosts(phx_ctx* c, double* const* comps, int q0)
 {
-    if (!c->patch.periodic)
-        return;
-    for (int k = 0; k < 3; ++k)
-        launchFillGhosts(c->G, q0 + k, comps[k], c->stream);
+    if (c->patch.periodic)
+        launchFill3(c->G, q0, vec(comps), c->stream);
 }
 
 void updateIons(phx_ctx* c)
@@ -1564,8 +1556,6 @@ phx_status createLevel(phx_config const* cfg, phx_patch const* patch, int const*
         s = alloc(&c->rho, QMOM);
     if (s == PHX_OK)
         s = alloc(&c->massD, QMOM);
-    if (s == PHX_OK)
-        s = alloc(&c->tmp, QMOM);
     for (int k = 0; k < 5 && s == PHX_OK; ++k)
         s = alloc(&c->tot5[k], QMOM);
     for (int p = 0; p < cfg->n_pop && s == PHX_OK; ++p)
@@ -1614,7 +1604,7 @@ phx_status createLevel(phx_config const* cfg, phx_patch const* patch, int const*
         launchZero(c->Ve[k], G.size(QMOM), c->stream);
         launchZero(c->Vi[k], G.size(QMOM), c->stream);
     }
-    for (double* p : {c->Pe, c->rho, c->massD, c->tmp})
+    for (double* p : {c->Pe, c->rho, c->massD})
         launchZero(p, G.size(QMOM), c->stream);
     for (int k = 0; k < 5; ++k)
         launchZero(c->tot5[k], G.size(QMOM), c->stream);

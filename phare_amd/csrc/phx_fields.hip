@@ -584,134 +584,139 @@ __global__ __launch_bounds__(FB) void k_nan_ghosts(Geom G0, int q, double* f)
         f[G.idx(q, i, j, k)] = __builtin_nan("");
 }
 
-// the nodes of the all-primal ghost box (S nodes per direction) that a periodic image overlaps:
-// the m = S - N layers at each end of every direction, all S when the two ends meet (K nodes);
-// enumerated as the nodes near along direction 0, then those inside along 0 and near along 1,
-// then inside along 0 and 1 and near along 2
-struct Shell
+// the sets of nodes of the all-primal ghost box that are periodic images of one another. Along a
+// direction the nodes c and c + N of the lower c <= end - N are images of each other (K of them; a
+// periodic level is wider than both ghost layers, so no node has two images along one direction), the
+// others have none; a set takes one choice per direction. The sets of more than one node are
+// enumerated by their lowest node: near along direction 0, then not along 0 and near along 1, then
+// neither along 0 nor 1 and near along 2
+struct Orbits
 {
-    int S[3], m[3], K[3];
+    int N[3], K[3];
     long count;
 };
 
-Shell shellOf(Geom const& G)
+Orbits orbitsOf(Geom const& G)
 {
-    Shell H{};
+    Orbits H{};
     for (int d = 0; d < 3; ++d)
     {
-        H.S[d] = d < G.dim ? G.shape[QMOM][d] : 1;
-        H.m[d] = d < G.dim ? H.S[d] - G.n[d] : 0;
-        H.K[d] = d < G.dim ? (2 * H.m[d] < H.S[d] ? 2 * H.m[d] : H.S[d]) : 0;
+        H.N[d] = d < G.dim ? G.n[d] : 1;
+        H.K[d] = d < G.dim ? G.shape[QMOM][d] - G.n[d] : 0;
     }
-    long const in0 = H.S[0] - H.K[0], in1 = H.S[1] - H.K[1];
-    H.count = static_cast<long>(H.K[0]) * H.S[1] * H.S[2];
+    long const in0 = H.N[0] - H.K[0], in1 = H.N[1] - H.K[1];
+    H.count = static_cast<long>(H.K[0]) * H.N[1] * H.N[2];
     if (G.dim > 1)
-        H.count += in0 * H.K[1] * H.S[2];
+        H.count += in0 * H.K[1] * H.N[2];
     if (G.dim > 2)
         H.count += in0 * in1 * H.K[2];
     return H;
 }
 
-// coordinate of the u-th near node / v-th inner node along d
-__device__ __forceinline__ int shellNear(Shell const& H, int d, int u)
-{
-    return H.K[d] == H.S[d] || u < H.m[d] ? u : H.S[d] - H.K[d] + u;
-}
-
 template<int DIM>
-__device__ __forceinline__ bool shellNode(Shell const& H, long t, int* c)
+__device__ __forceinline__ bool orbitNode(Orbits const& H, long t, int* c)
 {
     if (t >= H.count)
         return false;
-    long const r0 = static_cast<long>(H.K[0]) * H.S[1] * H.S[2];
+    long const r0 = static_cast<long>(H.K[0]) * H.N[1] * H.N[2];
     c[1] = c[2] = 0;
     if (t < r0)
     {
-        long const pl = static_cast<long>(H.S[1]) * H.S[2];
-        c[0]          = shellNear(H, 0, static_cast<int>(t / pl));
-        long const r  = t % pl;
-        c[1]          = static_cast<int>(r / H.S[2]);
-        c[2]          = static_cast<int>(r % H.S[2]);
+        int const pl = H.N[1] * H.N[2];
+        c[0]         = static_cast<int>(t / pl);
+        int const r  = static_cast<int>(t % pl);
+        c[1]         = r / H.N[2];
+        c[2]         = r % H.N[2];
         return true;
     }
     t -= r0;
-    int const in0 = H.S[0] - H.K[0];
-    long const r1 = DIM > 1 ? static_cast<long>(in0) * H.K[1] * H.S[2] : 0;
+    int const in0 = H.N[0] - H.K[0];
+    long const r1 = DIM > 1 ? static_cast<long>(in0) * H.K[1] * H.N[2] : 0;
     if (t < r1)
     {
-        long const pl = static_cast<long>(H.K[1]) * H.S[2];
-        c[0]          = H.m[0] + static_cast<int>(t / pl);
-        long const r  = t % pl;
-        c[1]          = shellNear(H, 1, static_cast<int>(r / H.S[2]));
-        c[2]          = static_cast<int>(r % H.S[2]);
+        int const pl = H.K[1] * H.N[2];
+        c[0]         = H.K[0] + static_cast<int>(t / pl);
+        int const r  = static_cast<int>(t % pl);
+        c[1]         = r / H.N[2];
+        c[2]         = r % H.N[2];
         return true;
     }
     t -= r1;
-    int const in1 = H.S[1] - H.K[1];
-    long const pl = static_cast<long>(in1) * H.K[2];
-    c[0]          = H.m[0] + static_cast<int>(t / pl);
-    long const r  = t % pl;
-    c[1]          = H.m[1] + static_cast<int>(r / H.K[2]);
-    c[2]          = shellNear(H, 2, static_cast<int>(r % H.K[2]));
+    int const pl = (H.N[1] - H.K[1]) * H.K[2];
+    c[0]         = H.K[0] + static_cast<int>(t / pl);
+    int const r  = static_cast<int>(t % pl);
+    c[1]         = H.K[1] + r / H.K[2];
+    c[2]         = r % H.K[2];
     return true;
 }
 
-// image k of {-1,0,1}^dim (lexicographic, zero excluded) overlaps the all-primal ghost box on
-// [max(0, k*N), min(end, end + k*N)]; node n receives orig[n - k*N]. Launched over the shell of
-// nodes some image overlaps: the others keep their value (out already holds it, the callers
-// copy out into orig first)
+// in place, per array (grid row) and set of periodic images: every node takes its own value combined
+// (sum / max) with those of its images, in the order of the images' shifts, upper nodes first along
+// each direction. One thread reads a whole set before it writes it, so that no copy of the arrays is
+// needed; a launch per array with a loop over all 26 shifts and a copy before it took 25 + 5 us per
+// moment at 64^3 cells
 template<int DIM, bool MAX>
-__global__ __launch_bounds__(FB) void k_border(Geom G0, Shell H, double const* orig, double* out)
+__global__ __launch_bounds__(FB) void k_border(Geom G0, Orbits H, FieldList F)
 {
     GeomD<DIM> const G(G0);
-    long const t = static_cast<long>(blockIdx.x) * FB + threadIdx.x;
-    int c[3];
-    if (!shellNode<DIM>(H, t, c))
+    if (G.stopped())
         return;
-    int const i = c[0], j = c[1], k = c[2];
-    int total = 1;
-    for (int d = 0; d < G.dim; ++d)
-        total *= 3;
-    int const n = G.idx(QMOM, i, j, k);
-    double v    = orig[n];
-    for (int im = 0; im < total; ++im)
+    int c[3];
+    if (!orbitNode<DIM>(H, static_cast<long>(blockIdx.x) * FB + threadIdx.x, c))
+        return;
+    double* const f = F.f[blockIdx.y];
+    constexpr int M = 1 << DIM;
+    // node y of the set: bit d clear is the upper node along d (where there are two)
+    int off[M];
+    bool in[M];
+    double v[M];
+#pragma unroll
+    for (int y = 0; y < M; ++y)
     {
-        int kk[3] = {0, 0, 0};
-        int r     = im;
-        bool zero = true;
-        for (int d = G.dim - 1; d >= 0; --d)
+        int n[3] = {c[0], c[1], c[2]};
+        in[y]    = true;
+#pragma unroll
+        for (int d = 0; d < DIM; ++d)
         {
-            kk[d] = (r % 3) - 1;
-            r /= 3;
-            if (kk[d])
-                zero = false;
-        }
-        if (zero)
-            continue;
-        bool in = true;
-        int s[3] = {i, j, k};
-        for (int d = 0; d < G.dim; ++d)
-        {
-            int const end = G.ghostEnd(QMOM, d);
-            int const sh  = kk[d] * G.n[d];
-            int const lo  = sh > 0 ? sh : 0;
-            int const hi  = end + sh < end ? end + sh : end;
-            if (c[d] < lo || c[d] > hi)
+            bool const two   = c[d] < H.K[d];
+            bool const lower = (y >> (DIM - 1 - d)) & 1;
+            if (!lower)
             {
-                in = false;
-                break;
+                if (two)
+                    n[d] += H.N[d];
+                else
+                    in[y] = false; // one node along d: the lower one
             }
-            s[d] = c[d] - sh;
         }
-        if (!in)
-            continue;
-        double const o = orig[G.idx(QMOM, s[0], s[1], s[2])];
-        if (MAX)
-            v = v < o ? o : v;
-        else
-            v += o;
+        off[y] = G.idx(QMOM, n[0], n[1], n[2]);
+        v[y]   = in[y] ? f[off[y]] : 0.;
     }
-    out[n] = v;
+#pragma unroll
+    for (int x = 0; x < M; ++x)
+    {
+        if (!in[x])
+            continue;
+        double r = v[x];
+#pragma unroll
+        for (int y = 0; y < M; ++y)
+        {
+            if (y == x || !in[y])
+                continue;
+            if (MAX)
+                r = r < v[y] ? v[y] : r;
+            else
+                r += v[y];
+        }
+        f[off[x]] = r;
+    }
+}
+
+// zeros in every array of the list (grid rows)
+__global__ __launch_bounds__(FB) void k_zero_list(FieldList F, long n)
+{
+    long const t = static_cast<long>(blockIdx.x) * FB + threadIdx.x;
+    if (t < n)
+        F.f[blockIdx.y][t] = 0.;
 }
 
 // ---- fused kernels of the periodic fast path ------------------------------------------------
@@ -1327,29 +1332,36 @@ void launchFillGhosts(Geom const& G, int q, double* f, hipStream_t s)
         case 3: k_fill_ghosts<3><<<gridFor(G.size(q)), FB, 0, s>>>(G, q, f); break;
     }
 }
-void launchBorderSum(Geom const& G, double const* orig, double* out, hipStream_t s)
+void launchBorderSum(Geom const& G, FieldList const& F, hipStream_t s)
 {
-    Shell const H = shellOf(G);
-    if (H.count == 0)
+    Orbits const H = orbitsOf(G);
+    if (H.count == 0 || F.n == 0)
         return;
+    dim3 const grid(gridFor(H.count), static_cast<unsigned int>(F.n));
     switch (G.dim)
     {
-        case 1: k_border<1, false><<<gridFor(H.count), FB, 0, s>>>(G, H, orig, out); break;
-        case 2: k_border<2, false><<<gridFor(H.count), FB, 0, s>>>(G, H, orig, out); break;
-        case 3: k_border<3, false><<<gridFor(H.count), FB, 0, s>>>(G, H, orig, out); break;
+        case 1: k_border<1, false><<<grid, FB, 0, s>>>(G, H, F); break;
+        case 2: k_border<2, false><<<grid, FB, 0, s>>>(G, H, F); break;
+        case 3: k_border<3, false><<<grid, FB, 0, s>>>(G, H, F); break;
     }
 }
-void launchBorderMax(Geom const& G, double const* orig, double* inout, hipStream_t s)
+void launchBorderMax(Geom const& G, FieldList const& F, hipStream_t s)
 {
-    Shell const H = shellOf(G);
-    if (H.count == 0)
+    Orbits const H = orbitsOf(G);
+    if (H.count == 0 || F.n == 0)
         return;
+    dim3 const grid(gridFor(H.count), static_cast<unsigned int>(F.n));
     switch (G.dim)
     {
-        case 1: k_border<1, true><<<gridFor(H.count), FB, 0, s>>>(G, H, orig, inout); break;
-        case 2: k_border<2, true><<<gridFor(H.count), FB, 0, s>>>(G, H, orig, inout); break;
-        case 3: k_border<3, true><<<gridFor(H.count), FB, 0, s>>>(G, H, orig, inout); break;
+        case 1: k_border<1, true><<<grid, FB, 0, s>>>(G, H, F); break;
+        case 2: k_border<2, true><<<grid, FB, 0, s>>>(G, H, F); break;
+        case 3: k_border<3, true><<<grid, FB, 0, s>>>(G, H, F); break;
     }
+}
+void launchZeroList(FieldList const& F, long count, hipStream_t s)
+{
+    if (F.n)
+        k_zero_list<<<dim3(gridFor(count), static_cast<unsigned int>(F.n)), FB, 0, s>>>(F, count);
 }
 void launchIonTotals(PopMoments const& P, double* rho, double* massDensity, VecPtr Vi, long count,
                      hipStream_t s)
