@@ -210,7 +210,8 @@ def family_line(wl, workload_name, precision, res):
     elif precision == "fp32":
         kernel = "k_push_seg32 (mixed precision, mode all)"
     else:
-        kernel = "k_push_seg (fused prePush+gather+Boris+postPush+deposit on cell-segmented storage, mode all)"
+        kernel = ("k_push_seg" if wl.dim == 1 else "k_push_cell") + \
+            " (fused prePush+gather+Boris+postPush+deposit on cell-segmented storage, mode all)"
     return {"value": res["value"], "unit": "particle-steps/s", "ms_per_step": res["ms_step"],
             "roofline": {"bound": "hbm", "achieved": a, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                          "frac": a / HBM_PEAK_GBS,

@@ -94,6 +94,7 @@ struct Pop
     double* mom[5] = {};
     SegTables seg{}; // tables of the segmented domain array (items sized for itemsAlloc items)
     unsigned int itemsAlloc = 0;
+    size_t itemsFor = 0; // slots that seg.rowsPerItem was chosen for (0: to be chosen)
 };
 
 } // namespace
@@ -408,8 +409,8 @@ void noteTileFallback(phx_ctx* c, TileSpec const& T)
                  c->tuning.segment_shape[0], c->tuning.segment_shape[1], c->tuning.segment_shape[2]);
 }
 
-// arguments of the push kernel; `segOk` lets a cell-segmented domain array use the 1D/2D segmented
-// kernel (callers that need a fate for every slot, the compacting path, pass false)
+// arguments of the push kernel; `segOk` lets a cell-segmented domain array use the segmented kernel of
+// the 1D and mixed-precision levels (callers that need a fate for every slot, the compacting path, pass false)
 PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt, bool segOk)
 {
     PushArgs A{};
@@ -446,25 +447,26 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
     A.tile = tileShape(c->cfg.dim, c->cfg.interp_order, ppc, copies);
     Pop const& P   = c->pops[pop];
     Store const& s = P.arr[kind];
-    // 3D, FP64: the cell-grouped push takes every segment whole, and gives every slot its fate
-    if (c->cfg.dim == 3 && !mixed(c) && kind == KIND_DOMAIN && s.seg)
-    {
-        A.segOn    = 1;
-        A.sg       = c->sg;
-        A.st       = P.seg;
-        A.rhoFromN = P.hasCharge && P.uniformCharge ? 1 : 0;
-        A.split    = cellSplit(c->cfg.interp_order, c->sg, s.n);
-        A.tile     = cellTileShape(c->cfg.interp_order, c->sg, A.rhoFromN ? 4 : 5, c->tuning.tile_row_pad);
-        noteTileFallback(c, A.tile);
-        return A;
-    }
-    if (segOk && c->cfg.dim != 3 && kind == KIND_DOMAIN && s.seg
-        && segItemsCap(c->sg, s.cap) <= P.itemsAlloc)
+    // 2D and 3D, FP64: the cell-grouped push, which gives every slot its fate
+    if (c->sg.dense && kind == KIND_DOMAIN && s.seg)
     {
         A.segOn       = 1;
         A.sg          = c->sg;
         A.st          = P.seg;
-        A.st.itemsCap = segItemsCap(c->sg, s.cap);
+        A.st.itemsCap = segItemsCap(c->sg, P.seg, s.cap);
+        A.rhoFromN    = P.hasCharge && P.uniformCharge ? 1 : 0;
+        A.split       = cellSplit(c->cfg.interp_order, c->sg, s.n);
+        A.tile = cellTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, A.rhoFromN ? 4 : 5, c->tuning.tile_row_pad);
+        noteTileFallback(c, A.tile);
+        return A;
+    }
+    if (segOk && c->cfg.dim != 3 && kind == KIND_DOMAIN && s.seg
+        && segItemsCap(c->sg, P.seg, s.cap) <= P.itemsAlloc)
+    {
+        A.segOn       = 1;
+        A.sg          = c->sg;
+        A.st          = P.seg;
+        A.st.itemsCap = segItemsCap(c->sg, P.seg, s.cap);
         A.rhoFromN    = !mixed(c) && P.hasCharge && P.uniformCharge ? 1 : 0;
         A.tile        = mixed(c) ? segTileShape32(c->cfg.dim, c->cfg.interp_order, c->sg)
                                  : segTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, PHX_SEG_COPIES,
@@ -1107,6 +1109,13 @@ phx_status sortDomain(phx_ctx* c)
             PHX_TRY(devAlloc(c, (void**)&c->sortRank, want * 4));
             c->rankCap = want;
         }
+        // kept while the array stays segmented and of about this size: a captured step holds it
+        if (!dom.seg || P.itemsFor == 0 || dom.n > 2 * P.itemsFor || 2 * dom.n < P.itemsFor)
+        {
+            P.seg.rowsPerItem = mixed(c) ? static_cast<unsigned int>(c->tuning.rows_per_item)
+                                         : itemRowsFor(c->sg, dom.n, c->tuning.rows_per_item);
+            P.itemsFor        = std::max<size_t>(dom.n, 1);
+        }
         if (mixed(c))
             launchSegCount(c->sg, dom.view32(), dom.n, c->segWork, c->sortRank, P.seg, c->stream);
         else
@@ -1132,7 +1141,7 @@ phx_status sortDomain(phx_ctx* c)
             c->permCap = buf.cap;
         }
         // work items for the larger of the two storages the sort alternates between
-        unsigned int const need = segItemsCap(c->sg, std::max(buf.cap, dom.cap));
+        unsigned int const need = segItemsCap(c->sg, P.seg, std::max(buf.cap, dom.cap));
         if (need > P.itemsAlloc)
         {
             devFree(c, P.seg.items);
@@ -1187,7 +1196,7 @@ phx_status sortIfLinear(phx_ctx* c)
     {
         Pop const& P = c->pops[p];
         Store const& s = P.arr[PHX_DOMAIN];
-        if (!s.seg || segItemsCap(c->sg, s.cap) > P.itemsAlloc)
+        if (!s.seg || segItemsCap(c->sg, P.seg, s.cap) > P.itemsAlloc)
             return sortDomain(c);
     }
     return PHX_OK;
@@ -1201,6 +1210,7 @@ std::vector<unsigned long long> storageKey(phx_ctx const* c)
     {
         // the segment tables a segmented push reads (reallocated when the storage grows)
         k.push_back(reinterpret_cast<unsigned long long>(c->pops[p].seg.items));
+        k.push_back(c->pops[p].seg.rowsPerItem);
         // the population's charge, which the push takes as an argument when it is uniform
         double const q = c->pops[p].charge;
         unsigned long long qb;
@@ -1284,9 +1294,10 @@ phx_status buildPatchTable(phx_ctx* c, int const* plo, int const* phi, int np)
     S             = SegGeom{};
     S.dim         = D;
     S.npatch      = np;
-    S.rowsPerItem = c->tuning.rows_per_item;
+    for (Pop& P : c->pops)
+        P.itemsFor = 0;
     S.rowPad      = c->tuning.tile_row_pad;
-    S.dense       = D == 3 && !mixed(c) ? 1 : 0;
+    S.dense       = D > 1 && !mixed(c) ? 1 : 0;
     size_t boxCells = 1;
     for (int d = 0; d < 3; ++d)
     {

@@ -5,10 +5,11 @@
 // being zero on the node its order-2 stencil leaves out). Over the particles p of the cell the
 // window is the contraction
 //     window[(a, b), (c, m)] = sum_p (wx_p[a] wy_p[b]) (wz_p[c] value_p[m])
-// with m the moments n, Fx, Fy, Fz: at W = 4 one 16x16x4 FP64 MFMA per four particles, at W = 2 one
-// 4x4x4 (four-block) MFMA per eight. The window stays in a wavefront's registers while its
-// particles stay in the cell and is then added to the workgroup's LDS tile, 4 (W = 4) or 1 (W = 2)
-// LDS atomics per wavefront and cell instead of one per particle, node and moment: a particle cost
+// with m the moments n, Fx, Fy, Fz (in 2D without c): in 3D at W = 4 one 16x16x4 FP64 MFMA per four
+// particles, at W = 2 one 4x4x4 (four-block) MFMA per eight; in 2D one 4x4x4 MFMA per four (W = 4) or
+// sixteen (W = 2). The window stays in a wavefront's registers while its
+// particles stay in the cell and is then added to the workgroup's LDS tile, 4 (3D, W = 4) or 1
+// LDS atomics per wavefront and cell instead of one per particle, node and moment: in 3D a particle cost
 // 108 (order 2) or 256 (order 3) lanes of ds_add_f64, about 30 cycles of the CU's LDS per
 // wavefront instruction, and costs about a quarter (W = 4) or a sixteenth (W = 2) of an MFMA here.
 //
@@ -37,16 +38,16 @@ __device__ __forceinline__ void waveLds()
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// window of a cell in 3D. RN: the charge density is derived from n and has no column
-template<int O, bool RN>
+// window of a cell. RN: the charge density is derived from n and has no column
+template<int D, int O, bool RN>
 struct CellWin
 {
     static constexpr int W    = O == 1 ? 2 : 4;
     static constexpr int WB   = O == 1 ? 0 : 1; // window base = local cell - WB
     static constexpr int NVAL = RN ? 4 : 5;
-    static constexpr int ARR  = 3 * W + NVAL;
+    static constexpr int ARR  = D * W + NVAL;
     static constexpr int BUF  = ARR * WSTR; // words of LDS per wavefront
-    static constexpr int NACC = W == 4 ? 4 : 1;
+    static constexpr int NACC = D == 3 && W == 4 ? 4 : 1;
 
     double a[NACC];            // n, Fx, Fy, Fz columns
     double rho[RN ? 1 : NACC]; // the charge density's column
@@ -124,20 +125,20 @@ __device__ __forceinline__ void windowWeights(double delta, double* out)
 }
 
 // the 32 particles of lanes [32 half, 32 half + 32) into the wavefront's buffer: the window weights
-// of delta along x, y, z, then the values n, Fx, Fy, Fz (and rho); lanes without `ok` hand over finite
+// of delta along each direction, then the values n, Fx, Fy, Fz (and rho); lanes without `ok` hand over finite
 // weights and zero values
-template<int O, bool RN>
+template<int D, int O, bool RN>
 __device__ __forceinline__ void cellStage(double* buf, int half, bool ok, double const* delta, double w,
                                           double q, double const* v, double coef)
 {
-    using C        = CellWin<O, RN>;
+    using C        = CellWin<D, O, RN>;
     int const lane = static_cast<int>(threadIdx.x & 63u);
     waveLds(); // the reads of the half before are done
     if ((lane >> 5) == half)
     {
         double* const b = buf + (lane & (WHALF - 1));
 #pragma unroll
-        for (int d = 0; d < 3; ++d)
+        for (int d = 0; d < D; ++d)
         {
             double ww[C::W];
             windowWeights<O>(ok ? delta[d] : 0., ww);
@@ -146,26 +147,79 @@ __device__ __forceinline__ void cellStage(double* buf, int half, bool ok, double
                 b[(d * C::W + a) * WSTR] = ww[a];
         }
         // the reference's products: 1. * w * coef, v * w * coef, q * w * coef
-        b[3 * C::W * WSTR] = ok ? w * coef : 0.;
+        b[D * C::W * WSTR] = ok ? w * coef : 0.;
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-            b[(3 * C::W + 1 + d) * WSTR] = ok ? v[d] * w * coef : 0.;
+            b[(D * C::W + 1 + d) * WSTR] = ok ? v[d] * w * coef : 0.;
         if constexpr (!RN)
-            b[(3 * C::W + 4) * WSTR] = ok ? q * w * coef : 0.;
+            b[(D * C::W + 4) * WSTR] = ok ? q * w * coef : 0.;
     }
     waveLds();
 }
 
 // the staged particles whose bit of `mask` is set (all of one cell) added to the window. ALL: every
 // instruction of the half row is issued, without a branch between them (many particles set)
-template<int O, bool RN, bool ALL>
-__device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, CellWin<O, RN>& acc)
+template<int D, int O, bool RN, bool ALL>
+__device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, CellWin<D, O, RN>& acc)
 {
-    using C        = CellWin<O, RN>;
+    using C        = CellWin<D, O, RN>;
     int const lane = static_cast<int>(threadIdx.x & 63u);
     int const i    = lane & 15;
     int const k    = lane >> 4;
-    if constexpr (C::W == 4)
+    if constexpr (D == 2)
+    {
+        // W = 4: block m, rows a, columns b; four particles per instruction, lane group k taking a
+        // pair of particles for two instructions. W = 2: block of particles, rows (a, b), columns m;
+        // sixteen particles per instruction
+        constexpr bool W4 = C::W == 4;
+        constexpr int PP  = W4 ? 8 : 32; // particles of two instructions
+        int const l4 = lane & 3, blk = (lane >> 2) & 3;
+        int const o  = W4 ? 2 * k : 8 * k + 2 * blk;
+        double const* const px = buf + (W4 ? l4 : l4 >> 1) * WSTR + o;
+        double const* const py = buf + (C::W + (W4 ? l4 : l4 & 1)) * WSTR + o;
+        double const* const pv = buf + (2 * C::W + (W4 ? blk : l4)) * WSTR + o;
+        double const* const pr = buf + (2 * C::W + 4) * WSTR + o;
+        unsigned int const mk  = mask >> o;
+#pragma unroll
+        for (int t = 0; t < WHALF / PP; ++t)
+        {
+            if (!ALL && W4 && ((mask >> (8 * t)) & 0xffu) == 0u)
+                continue;
+            double2 const x = *reinterpret_cast<double2 const*>(px + PP * t);
+            double2 const y = *reinterpret_cast<double2 const*>(py + PP * t);
+            double2 const v = *reinterpret_cast<double2 const*>(pv + PP * t);
+            double const v0 = (mk >> (PP * t % 32)) & 1u ? v.x : 0.;
+            double const v1 = (mk >> (PP * t % 32)) & 2u ? v.y : 0.;
+            if constexpr (W4)
+            {
+                acc.a[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.x * v0, y.x, acc.a[0], 0, 0, 0);
+                acc.a[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.y * v1, y.y, acc.a[0], 0, 0, 0);
+            }
+            else
+            {
+                acc.a[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.x * y.x, v0, acc.a[0], 0, 0, 0);
+                acc.a[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.y * y.y, v1, acc.a[0], 0, 0, 0);
+            }
+            if constexpr (!RN)
+            {
+                double2 const q = *reinterpret_cast<double2 const*>(pr + PP * t);
+                bool const on   = W4 ? blk == 0 : l4 == 0;
+                double const q0 = on && ((mk >> (PP * t % 32)) & 1u) ? q.x : 0.;
+                double const q1 = on && ((mk >> (PP * t % 32)) & 2u) ? q.y : 0.;
+                if constexpr (W4)
+                {
+                    acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.x * q0, y.x, acc.rho[0], 0, 0, 0);
+                    acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.y * q1, y.y, acc.rho[0], 0, 0, 0);
+                }
+                else
+                {
+                    acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.x * y.x, q0, acc.rho[0], 0, 0, 0);
+                    acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(x.y * y.y, q1, acc.rho[0], 0, 0, 0);
+                }
+            }
+        }
+    }
+    else if constexpr (C::W == 4)
     {
         // rows (a, b) = (i / 4, i % 4) of A, columns (c, m) = (i / 4, i % 4) of B; four particles
         // per instruction, lane group k taking a pair of particles for two instructions
@@ -246,25 +300,38 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
     }
 }
 
-template<int O, bool RN>
-__device__ __forceinline__ void cellAdd(double const* buf, unsigned int mask, CellWin<O, RN>& acc)
+template<int D, int O, bool RN>
+__device__ __forceinline__ void cellAdd(double const* buf, unsigned int mask, CellWin<D, O, RN>& acc)
 {
     if (__popc(mask) >= WHALF / 2)
-        cellAddT<O, RN, true>(buf, mask, acc);
+        cellAddT<D, O, RN, true>(buf, mask, acc);
     else
-        cellAddT<O, RN, false>(buf, mask, acc);
+        cellAddT<D, O, RN, false>(buf, mask, acc);
 }
 
 // one staged particle (p, in no larger group) added to the LDS tile by itself
-template<int O, bool RN>
+template<int D, int O, bool RN>
 __device__ __forceinline__ void cellAddOne(double const* buf, int p, double* tile, int stride, int node0,
                                            int p12, int p2)
 {
-    using C        = CellWin<O, RN>;
+    using C        = CellWin<D, O, RN>;
     int const lane = static_cast<int>(threadIdx.x & 63u);
     int const m    = lane & 3;
     int const slab = RN || m == 0 ? m : m + 1;
-    if constexpr (C::W == 4)
+    if constexpr (D == 2)
+    {
+        int const a = lane / (4 * C::W), b = lane / 4 % C::W;
+        if (a < C::W)
+        {
+            double const xy = buf[a * WSTR + p] * buf[(C::W + b) * WSTR + p];
+            int const n     = node0 + a * p12 + b * p2;
+            atomicAdd(tile + slab * stride + n, xy * buf[(2 * C::W + m) * WSTR + p]);
+            if constexpr (!RN)
+                if (m == 0)
+                    atomicAdd(tile + stride + n, xy * buf[(2 * C::W + 4) * WSTR + p]);
+        }
+    }
+    else if constexpr (C::W == 4)
     {
         int const b = lane >> 4, c = (lane & 15) >> 2;
         double const yz = buf[(4 + b) * WSTR + p] * buf[(8 + c) * WSTR + p];
@@ -293,16 +360,29 @@ __device__ __forceinline__ void cellAddOne(double const* buf, int p, double* til
 }
 
 // add the window to the LDS tile: node0 is the tile node of the window's origin, p12 and p2 the
-// node distances along x and y, slab m of the tile the moments in the order n, (rho,) Fx, Fy, Fz
-template<int O, bool RN>
-__device__ __forceinline__ void cellFlush(CellWin<O, RN> const& acc, double* tile, int stride, int node0,
+// node distances along the first two directions, slab m of the tile the moments in the order n, (rho,) Fx, Fy, Fz
+template<int D, int O, bool RN>
+__device__ __forceinline__ void cellFlush(CellWin<D, O, RN> const& acc, double* tile, int stride, int node0,
                                           int p12, int p2)
 {
-    using C        = CellWin<O, RN>;
+    using C        = CellWin<D, O, RN>;
     int const lane = static_cast<int>(threadIdx.x & 63u);
     int const m    = lane & 3;
     int const slab = RN || m == 0 ? m : m + 1;
-    if constexpr (C::W == 4)
+    if constexpr (D == 2)
+    {
+        // W = 4: lane (a, m, b) = (lane / 16, lane / 4 % 4, lane % 4); W = 2: rows (a, b) = lane / 16,
+        // column lane % 4, the four blocks of particles adding to the same node
+        constexpr bool W4 = C::W == 4;
+        int const mm = W4 ? (lane >> 2) & 3 : m, sl = RN || mm == 0 ? mm : mm + 1;
+        int const n  = W4 ? node0 + (lane >> 4) * p12 + (lane & 3) * p2
+                          : node0 + (lane >> 5) * p12 + ((lane >> 4) & 1) * p2;
+        atomicAdd(tile + sl * stride + n, acc.a[0]);
+        if constexpr (!RN)
+            if (mm == 0)
+                atomicAdd(tile + stride + n, acc.rho[0]);
+    }
+    else if constexpr (C::W == 4)
     {
         // result register r of lane (q, i): row 4 r + q = (a, b) = (r, q), column i
         int const n = node0 + (lane >> 4) * p2 + ((lane & 15) >> 2);

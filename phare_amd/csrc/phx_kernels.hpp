@@ -70,8 +70,9 @@ struct TileSpec
     int copies; // moment copies (power of two): lane l accumulates into copy l % copies
     int stride;
     unsigned int bytes; // dynamic LDS of the launch
-    // cell-grouped 3D push: fields staged beside the tile, from node (tile origin + emLo), extents
-    // emExt, emStride words of LDS for the six components; emFix: emExt is that of a 4x4x4 segment
+    // cell-grouped push: fields staged beside the tile, from node (tile origin + emLo), extents
+    // emExt, emStride words of LDS for the six components; emFix: the pitches are those of the
+    // default segments
     int emLo[3], emExt[3], emStride, emFix;
     int brick;          // > 0: the tile covers the brick (cube of `brick` cells, on the grid of
                         // bricks from the patch's lower cell) of the chunk's first particle
@@ -108,7 +109,6 @@ struct SegGeom
     int lo[3];     // lowest AMR cell of the level box (the box of the owner map)
     int n[3];      // level box cells per dimension
     int maxSeg[3]; // largest segment extent over the patches (the launch's LDS tile)
-    int rowsPerItem; // most segment rows per work item of the segmented push
     int dense;       // positions fill the rows one after the other
     int rowPad;      // 2D LDS tile rows padded to a multiple of this many nodes
     SegPatch first;               // patch 0 (a one-patch level reads it from the kernel arguments)
@@ -124,6 +124,7 @@ struct SegTables
     unsigned int* items;      // [2 * itemsCap] (segment, first row) of each work item
     unsigned int* nItems;     // number of work items
     unsigned int itemsCap;    // work items the storage's capacity allows (grid of the push)
+    unsigned int rowsPerItem; // most segment rows per work item
 };
 
 // in-kernel timing of one push launch site (a node of the captured step): the earliest
@@ -193,7 +194,9 @@ unsigned int compactBlocks(unsigned long long n);
 // tile of the segmented push, the most work items a storage of `capacity` slots can need
 SegPatch segPatchOf(int dim, int const* lo, int const* hi, int const* pref);
 TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies, int slabs);
-unsigned int segItemsCap(SegGeom const& sg, unsigned long long capacity);
+unsigned int segItemsCap(SegGeom const& sg, SegTables const& tables, unsigned long long capacity);
+// rows per work item of an array of `slots` slots, at most `most`
+unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most);
 // first half of a sort of src (n slots) into cell-segmented storage: counts per cell, the rank
 // of every particle in its cell (rank: n words) and the segment tables up to the total slot count
 // (tables.off[nsegs + 1]); `work` holds ncells + 1 + 2 (nsegs + 1) words
@@ -220,11 +223,11 @@ TileSpec segTileShape32(int dim, int order, SegGeom const& sg);
 // the same over brick-ordered linear FP32 storage (3D), in place; the LDS tile of brickTileShape32
 void launchPush32Linear(PushArgs const& A, PView32 const& v, hipStream_t s);
 TileSpec brickTileShape32(int order);
-// push + gather + deposit (A.pushOn 0: deposit only) over dense cell-segmented 3D storage, in place,
-// A.split workgroups per segment, the particles of a cell deposited together; the LDS tile of
-// cellTileShape (5 slabs, 4 with A.rhoFromN)
+// push + gather + deposit (A.pushOn 0: deposit only) over dense cell-segmented 2D or 3D storage, in
+// place, one workgroup per work item (2D) or A.split per segment (3D), the particles of a cell
+// deposited together; the LDS tile of cellTileShape (5 slabs, 4 with A.rhoFromN)
 void launchPushCell(PushArgs const& A, PView const& in, hipStream_t s);
-TileSpec cellTileShape(int order, SegGeom const& sg, int slabs, int pad);
+TileSpec cellTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad);
 // workgroups per segment (A.split) for an array of `slots` slots
 unsigned int cellSplit(int order, SegGeom const& sg, unsigned long long slots);
 // mixed-precision push + gather + deposit over cell-segmented storage with one workgroup per segment

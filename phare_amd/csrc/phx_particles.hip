@@ -8,18 +8,20 @@
 // f64 charge), each component a contiguous stream, in one of two storage orders:
 //  - linear: a workgroup owns a chunk of consecutive particles, lanes taking them with a stride
 //    across the chunk (any order is correct; cell order is faster);
-//  - cell-segmented (built by the sort): the 64 lanes of a wavefront read one row of a segment
-//    (a box of up to 64 cells whose particles, in cell order, fill its rows column by column), so
-//    that each lane walks a run of cell-ordered particles and the lanes of one row hold cells
-//    spread over the segment. Reads stay coalesced and the lanes of one LDS deposit instruction
-//    add into distinct words, except where a crowded cell spans two lanes.
+//  - cell-segmented (built by the sort): the 64 lanes of a wavefront read one row of a segment (a
+//    box of up to 64 cells), coalesced. In FP64 2D and 3D the segment's particles fill its rows in
+//    cell order, and those of one cell deposit together on the matrix cores (k_push_cell). In 1D and
+//    in FP32 they fill the rows column by column, so that each lane walks a run of cell-ordered
+//    particles and the lanes of one LDS deposit instruction add into distinct words, except where a
+//    crowded cell spans two lanes.
 // Either way a workgroup accumulates its moments in an LDS tile over its cells and flushes the
 // tile with one HBM atomic per touched node and moment; the gather reads E/B through the L1/L2
-// caches, leaving the LDS to the deposit. Particles whose stencil leaves the tile deposit
+// caches, leaving the LDS to the deposit (k_push_cell stages E/B in LDS). Particles whose stencil leaves the tile deposit
 // straight into HBM.
 #include "phx_cell_deposit.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <mutex>
 
 #ifndef PHX_PPT_ND
@@ -38,25 +40,28 @@ using pc::LANES;
 using pc::NW;
 using pc::TILE_BYTES_MAX;
 
-// the cell-grouped push, per order: work-items of a workgroup, waves per SIMD the register allocation
-// targets (what a workgroup's LDS leaves room for), and whether the next row is loaded while a row is
-// worked on. Order 1 runs best on many waves without the prefetch's registers (58x47x52 cells, 50
-// particles per cell: 0.243 ms for mode domain_only, against 0.259 with two workgroups of 256 and
-// the prefetch); at order 2 two workgroups of 256 fit a CU (64^3 cells, 64 per cell: 0.95 ms; 1.09 with
-// one of 512); at order 3 the larger stage leaves room for one workgroup, of 512 (36x41x30 cells, 32
-// per cell: 0.207 ms, 0.260 with 256)
-template<int O>
+// the cell-grouped push, per dimension and order: work-items of a workgroup, waves per SIMD the
+// register allocation targets (what a workgroup's LDS leaves room for), and whether the next row is
+// loaded while a row is worked on. In 3D order 1 runs best on many waves without the prefetch's
+// registers (58x47x52 cells, 50 particles per cell: 0.243 ms for mode domain_only, against 0.259 with
+// two workgroups of 256 and the prefetch); at order 2 two workgroups of 256 fit a CU (64^3 cells, 64
+// per cell: 0.95 ms; 1.09 with one of 512); at order 3 the larger stage leaves room for one
+// workgroup, of 512 (36x41x30 cells, 32 per cell: 0.207 ms, 0.260 with 256)
+// In 2D four workgroups of 256 fit a CU (256x128 cells, 100 per cell, order 2: 0.093 ms after a sort,
+// growing to 0.17 over 30 steps, as drifted lanes meet in LDS banks; one particle per lane into the
+// tile, in columns, took 0.137)
+constexpr int cellBlock(int dim, int order) { return dim == 2 || order == 2 ? 256 : 512; }
+template<int D, int O>
 struct CellCfg
 {
-    static constexpr int BLOCK     = O == 2 ? 256 : 512;
-    static constexpr int WAVES     = O == 1 ? 4 : 2;
-    static constexpr bool PREFETCH = O != 1;
+    static constexpr int BLOCK     = cellBlock(D, O);
+    static constexpr int WAVES     = D == 2 ? 4 : (O == 1 ? 4 : 2);
+    static constexpr bool PREFETCH = D == 2 || O != 1;
     static constexpr int NW        = BLOCK / LANES;
+    // particles listed for the one-by-one push between two passes over the rows (every wavefront
+    // that finds room for a workgroup's particles may add its row)
+    static constexpr unsigned int LIST = 2 * BLOCK;
 };
-constexpr int cellBlock(int order) { return order == 2 ? 256 : 512; }
-// particles listed for the one-by-one push between two passes over the rows (every wavefront that
-// finds room for a workgroup's particles may add its row)
-constexpr unsigned int CELL_LIST = 1024;
 // the smallest group of lanes of one cell (of the 32 of a half row) that deposits on the matrix cores,
 // and the smallest that moves the accumulated window to its cell
 constexpr int CELL_GROUP = 2;
@@ -68,9 +73,10 @@ constexpr unsigned int CELL_LDS_MAX = 131072;
 // them for the segment's cells and those one cell around it
 constexpr int cellGatherLo(int order) { return order == 3 ? -2 : -1; }
 constexpr int cellGatherNodes(int order) { return order == 1 ? 3 : (order == 2 ? 4 : 5); }
-// nodes per direction of the stage of a 4x4x4 segment
-template<int O>
-constexpr int CELL_STAGE = 4 + 1 + cellGatherNodes(O);
+// pitch of the stage's last direction for segments of at most cellFixed cells along it, odd so that
+// stencils of different cells start in different banks
+constexpr int cellFixed(int dim) { return dim == 2 ? 32 : 4; }
+constexpr int cellStage(int dim, int order) { return cellFixed(dim) + 1 + cellGatherNodes(order); }
 
 // Per (dim, order): whether the deposit is accumulated in registers over a union window, the
 // particles per thread of the linear push and the window. With accumulation, a thread's
@@ -732,8 +738,8 @@ __device__ __forceinline__ void pushPiece(PushArgs const& A, PView const& in, do
     flushTile<D, RN, pc::SEG_BLOCK>(G, T, A.tile.nodes, A.mom, A.charge);
 }
 
-// one workgroup per work item (a segment and its share of the segment's rows, at most
-// sg.rowsPerItem)
+// 1D: one workgroup per work item (a segment and its share of the segment's rows, at most
+// st.rowsPerItem)
 template<int D, int O, bool RN>
 __global__ __launch_bounds__(pc::SEG_BLOCK) __attribute__((amdgpu_waves_per_eu(PHX_SEG_WAVES)))
 void k_push_seg(PushArgs A, PView in)
@@ -749,7 +755,7 @@ void k_push_seg(PushArgs A, PView in)
         unsigned int const seg = A.st.items[2 * item];
         unsigned int const R   = A.st.rows[seg];
         unsigned int r0, rEnd;
-        pc::itemRows(A.st.items[2 * item + 1], R, static_cast<unsigned int>(A.sg.rowsPerItem), r0, rEnd);
+        pc::itemRows(A.st.items[2 * item + 1], R, A.st.rowsPerItem, r0, rEnd);
         pushPiece<D, O, RN>(A, in, lds, seg, r0, rEnd);
     }
     if (A.kt)
@@ -760,8 +766,8 @@ void k_push_seg(PushArgs A, PView in)
 }
 
 // ---------------------------------------------------------------------------------------------
-// fused push + deposit over cell-ordered segmented storage, A.split workgroups per segment (3D,
-// segments of 4x4x4 cells): the rows of a segment hold its particles in cell order, each wavefront
+// fused push + deposit over cell-ordered segmented storage, A.split workgroups per segment in 3D, one
+// per work item in 2D (segments of 4x4x4 and 2x32 cells): the rows of a segment hold its particles in cell order, each wavefront
 // takes a run of them, and the particles of one cell deposit together on the matrix cores
 // (phx_cell_deposit.hpp). The tile covers the segment with the stencil and one cell of motion on
 // each side, and E and B of the segment's surroundings are staged beside it. A particle that leaves
@@ -786,14 +792,14 @@ __device__ __forceinline__ GlobalPtr<R> rowOf(R* p, unsigned long long row)
 }
 
 // one row of the segment: the particles of 64 consecutive slots
-template<bool RN>
-__device__ __forceinline__ void loadRow(PView const& in, unsigned long long row, unsigned int lane, Part<3>& p)
+template<int D, bool RN>
+__device__ __forceinline__ void loadRow(PView const& in, unsigned long long row, unsigned int lane, Part<D>& p)
 {
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < D; ++d)
         p.cell[d] = rowOf(in.ic[d], row)[lane];
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < D; ++d)
         p.delta[d] = rowOf(in.de[d], row)[lane];
 #pragma unroll
     for (int d = 0; d < 3; ++d)
@@ -819,11 +825,12 @@ __device__ __forceinline__ CellArgs const& cellArgs()
 }
 
 // half a step of the position without a branch; false when it moves more than two cells
+template<int D>
 __device__ __forceinline__ bool halfStep(int* cell, double* delta, double const* v, double const* hdtdx)
 {
     bool ok = true;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < D; ++d)
     {
         double const dl = delta[d] + hdtdx[d] * v[d];
         ok              = ok & !(fabs(dl) > 2);
@@ -835,26 +842,26 @@ __device__ __forceinline__ bool halfStep(int* cell, double* delta, double const*
 }
 
 // E and B of the segment's surroundings in LDS: component f (Ex .. Bz) on `nodes` nodes from `org`,
-// row-major with extents ext; nodes beyond a component's array repeat its last ones (no stencil
-// inside the domain reaches them)
-template<int TB>
+// row-major, e1 and e2 nodes along the second and third direction (e1 in 2D); nodes beyond a
+// component's array repeat its last ones (no stencil inside the domain reaches them)
+template<int D, int TB>
 __device__ __forceinline__ void stageFields(PushArgs const& A, double* em, int const* org, int e1, int e2,
                                             int nodes)
 {
     Geom const& G = A.G;
-    int const e12 = e1 * e2;
+    int const e12 = D == 3 ? e1 * e2 : e1;
     for (int x = threadIdx.x; x < nodes; x += TB)
     {
         int const i = x / e12, r = x - i * e12;
-        int const j = r / e2, k = r - j * e2;
+        int const j = D == 3 ? r / e2 : r, k = D == 3 ? r - j * e2 : 0;
 #pragma unroll
         for (int f = 0; f < 6; ++f)
         {
             int const q    = f < 3 ? QEX + f : QBX + f - 3;
-            int const n[3] = {org[0] + i, org[1] + j, org[2] + k};
-            int c[3];
+            int const n[3] = {org[0] + i, org[1] + j, D == 3 ? org[2] + k : 0};
+            int c[3]       = {0, 0, 0};
 #pragma unroll
-            for (int d = 0; d < 3; ++d)
+            for (int d = 0; d < D; ++d)
                 c[d] = min(max(n[d], 0), G.shape[q][d] - 1);
             em[f * nodes + x] = (f < 3 ? A.em.E[f] : A.em.B[f - 3])[G.idx(q, c[0], c[1], c[2])];
         }
@@ -862,15 +869,16 @@ __device__ __forceinline__ void stageFields(PushArgs const& A, double* em, int c
 }
 
 // E and B at a particle from the staged fields; rel: its cell less the stage's first node
-template<int O>
+template<int D, int O>
 __device__ __forceinline__ void gatherStaged(double const* em, int e1, int e2, int nodes, int const* rel,
                                              double const* delta, double* E, double* B)
 {
-    constexpr int S = O + 1;
-    double w[2][3][S];
-    int st[2][3];
+    constexpr int S  = O + 1;
+    constexpr int SZ = D == 3 ? S : 1;
+    double w[2][D][S];
+    int st[2][D];
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
+    for (int d = 0; d < D; ++d)
     {
         st[CP][d] = rel[d] - pc::splineStencil<O>(CP, delta[d], w[CP][d]);
         st[CD][d] = rel[d] - pc::splineStencil<O>(CD, delta[d], w[CD][d]);
@@ -880,7 +888,8 @@ __device__ __forceinline__ void gatherStaged(double const* em, int e1, int e2, i
     {
         int const q  = f < 3 ? QEX + f : QBX + f - 3;
         int const cx = centering(q, 0), cy = centering(q, 1), cz = centering(q, 2);
-        double const* const p = em + f * nodes + (st[cx][0] * e1 + st[cy][1]) * e2 + st[cz][2];
+        int const at = st[cx][0] * e1 + st[cy][1];
+        double const* const p = em + f * nodes + (D == 3 ? at * e2 + st[cz][D - 1] : at);
         double r = 0.;
 #pragma unroll
         for (int i = 0; i < S; ++i)
@@ -889,11 +898,16 @@ __device__ __forceinline__ void gatherStaged(double const* em, int e1, int e2, i
 #pragma unroll
             for (int j = 0; j < S; ++j)
             {
-                double z = 0.;
+                if constexpr (D == 3)
+                {
+                    double z = 0.;
 #pragma unroll
-                for (int k = 0; k < S; ++k)
-                    z = __builtin_fma(p[(i * e1 + j) * e2 + k], w[cz][2][k], z);
-                y = __builtin_fma(z, w[cy][1][j], y);
+                    for (int k = 0; k < SZ; ++k)
+                        z = __builtin_fma(p[(i * e1 + j) * e2 + k], w[cz][D - 1][k], z);
+                    y = __builtin_fma(z, w[cy][1][j], y);
+                }
+                else
+                    y = __builtin_fma(p[i * e1 + j], w[cy][1][j], y);
             }
             r = __builtin_fma(y, w[cx][0][i], r);
         }
@@ -902,215 +916,243 @@ __device__ __forceinline__ void gatherStaged(double const* em, int e1, int e2, i
 }
 } // namespace
 
-// FIX: the stage has the extents of a 4x4x4 segment (the stencils' offsets are then constants)
-template<int O, bool RN, bool FIX>
-__global__ __launch_bounds__(CellCfg<O>::BLOCK) __attribute__((amdgpu_waves_per_eu(CellCfg<O>::WAVES)))
+// FIX: the stage has the pitches of the default segments (the stencils' offsets are then constants)
+template<int D, int O, bool RN, bool FIX>
+__global__ __launch_bounds__((CellCfg<D, O>::BLOCK)) __attribute__((amdgpu_waves_per_eu(CellCfg<D, O>::WAVES)))
 void k_push_cell(CellArgs K)
 {
-    using C             = pc::CellWin<O, RN>;
-    constexpr int CB    = CellCfg<O>::BLOCK;
-    constexpr bool NEXT = CellCfg<O>::PREFETCH;
+    using C                     = pc::CellWin<D, O, RN>;
+    constexpr int CB            = CellCfg<D, O>::BLOCK;
+    constexpr bool NEXT         = CellCfg<D, O>::PREFETCH;
+    constexpr unsigned int LIST = CellCfg<D, O>::LIST;
     // 16-byte aligned: the hand-over buffers are read as pairs of words (a pair read 8 bytes off
     // took 8 times as long)
     extern __shared__ __align__(16) double cellLds[];
     double* const lds = cellLds;
-    __shared__ unsigned int list[CELL_LIST];
+    __shared__ unsigned int list[LIST];
     __shared__ unsigned int listed;
-    if (K.A.G.stopped())
-        return;
-    unsigned int const item = pc::xcdItem(blockIdx.x, gridDim.x);
-    unsigned int const seg  = item / K.A.split;
-    unsigned int const lane = threadIdx.x & 63u;
-    unsigned int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    unsigned long long const off = K.A.st.off[seg];
-    unsigned int const R         = K.A.st.rows[seg];
-    unsigned int const part = item - seg * K.A.split;
-    unsigned int const rA   = static_cast<unsigned int>(static_cast<unsigned long long>(R) * part / K.A.split);
-    unsigned int const rows
-        = static_cast<unsigned int>(static_cast<unsigned long long>(R) * (part + 1) / K.A.split) - rA;
-    if (rows == 0)
-        return;
-    // stage pitches: odd along z, so that stencils of different cells start in different banks
-    constexpr int EX  = CELL_STAGE<O>;
-    int const e1      = FIX ? EX : K.A.tile.emExt[1], e2 = (FIX ? EX : K.A.tile.emExt[2]) | 1;
-    int const emNodes = (FIX ? EX : K.A.tile.emExt[0]) * e1 * e2;
-    double* const em  = lds + (RN ? 4 : 5) * K.A.tile.stride;
-    double* const buf = em + K.A.tile.emStride + wave * C::BUF;
-    zeroTile<RN, CB>(lds, K.A.tile);
-    if (threadIdx.x == 0)
-        listed = 0u;
-    TileView T;
-    tileView(T, lds, K.A.tile);
-    pc::segTileOrigin<3>(K.A.G, K.A.sg, K.A.tile, seg, T.org);
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-        T.org[d] = __builtin_amdgcn_readfirstlane(T.org[d]); // the same in every lane: scalar from here on
-    int const p2 = T.pitch[2], p12 = T.pitch[1] * T.pitch[2];
-    bool const push   = K.A.pushOn;
-    bool const writes = push && K.A.mode == MODE_ALL;
-    // per direction: AMR cell of the deposit tile's and of the stage's first cell, and the number
-    // of cells whose windows (stencils) they hold; the stage's cells are clipped to those whose
-    // stencils lie in the arrays
-    int tileCell[3], tileCells[3], emCell[3], emLow[3], emCells[3], emOrg[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
+    // 3D: split workgroups per segment; 2D: the work items of the sort (captured steps keep their
+    // grid while the sorts change the items)
+    unsigned int seg, rA, rB, nItems = 0;
+    if constexpr (D == 3)
     {
-        int const shift = K.A.G.lower[d] - K.A.G.g; // AMR cell of local cell 0
-        tileCell[d]     = T.org[d] + C::WB + shift;
-        tileCells[d]    = max(T.ext[d] - C::W + 1, 0);
-        emOrg[d]        = T.org[d] + K.A.tile.emLo[d];
-        emCell[d]       = emOrg[d] + shift;
-        int const lo    = max(emOrg[d] - cellGatherLo(O), K.A.G.safeLo[d]);
-        int const hi    = min(emOrg[d] - cellGatherLo(O) + K.A.tile.emExt[d] - cellGatherNodes(O), K.A.G.safeHi[d]);
-        emLow[d]        = lo + shift;
-        emCells[d]      = max(hi - lo + 1, 0);
+        unsigned int const item = pc::xcdItem(blockIdx.x, gridDim.x);
+        seg                     = item / K.A.split;
+        unsigned int const part = item - seg * K.A.split;
+        unsigned long long const R = K.A.st.rows[seg];
+        rA = static_cast<unsigned int>(R * part / K.A.split);
+        rB = static_cast<unsigned int>(R * (part + 1) / K.A.split);
     }
-    double const h[3] = {K.A.hdtdx[0], K.A.hdtdx[1], K.A.hdtdx[2]};
-    double const dto2m = K.A.dto2m, coef = K.A.coef, charge = K.A.charge;
-    int const dom[6] = {K.A.box.dom_lo[0], K.A.box.dom_lo[1], K.A.box.dom_lo[2],
-                        K.A.box.dom_hi[0], K.A.box.dom_hi[1], K.A.box.dom_hi[2]};
-    if (push)
-        stageFields<CB>(K.A, em, emOrg, e1, e2, emNodes);
-    __syncthreads();
-
-    unsigned int r          = rA + rows * wave / CellCfg<O>::NW;
-    unsigned int const rEnd = rA + rows * (wave + 1) / CellCfg<O>::NW;
-    do
+    else
     {
-        C acc;
-        acc.zero();
-        int cur = -1; // tile node of the accumulated window's origin
-        Part<3> next;
-        if (NEXT && r < rEnd)
-            loadRow<RN>(K.v, off + static_cast<unsigned long long>(r) * LANES, lane, next);
-        for (; r < rEnd; ++r)
-        {
-            // until the list might overflow (each wavefront that still finds room may add 64)
-            if (__builtin_amdgcn_readfirstlane(*static_cast<unsigned int volatile*>(&listed)) > CELL_LIST - CB)
-                break;
-            unsigned long long const row = off + static_cast<unsigned long long>(r) * LANES;
-            Part<3> P;
-            if constexpr (NEXT)
-            {
-                P = next;
-                if (r + 1 < rEnd)
-                    loadRow<RN>(K.v, row + LANES, lane, next); // in flight over this row's work
-            }
-            else
-                loadRow<RN>(K.v, row, lane, P);
-            double const q  = RN ? charge : P.q;
-            bool const live = P.cell[0] != DEAD_CELL;
-            bool ok         = live;
-            if (push)
-            {
-                ok = halfStep(P.cell, P.delta, P.v, h) & ok;
-                int rel[3];
-#pragma unroll
-                for (int d = 0; d < 3; ++d)
-                {
-                    ok     = ok & (static_cast<unsigned int>(P.cell[d] - emLow[d]) < static_cast<unsigned int>(emCells[d]));
-                    rel[d] = P.cell[d] - emCell[d];
-                }
-                double E[3] = {0., 0., 0.}, B[3] = {0., 0., 0.};
-                if (ok)
-                    gatherStaged<O>(em, e1, e2, emNodes, rel, P.delta, E, B);
-                borisAccelerate(P.v, E, B, q, dto2m);
-                ok = halfStep(P.cell, P.delta, P.v, h) & ok;
-#pragma unroll
-                for (int d = 0; d < 3; ++d)
-                    ok = ok & (P.cell[d] >= dom[d]) & (P.cell[d] <= dom[3 + d]);
-            }
-            // the tile node of the window's origin; a value that is not finite (it would reach the
-            // whole window) deposits by itself
-            ok = ok & __builtin_isfinite(P.w * coef) & (RN || __builtin_isfinite(q * P.w * coef));
-            int rel[3];
-#pragma unroll
-            for (int d = 0; d < 3; ++d)
-            {
-                rel[d] = P.cell[d] - tileCell[d];
-                ok = ok & (static_cast<unsigned int>(rel[d]) < static_cast<unsigned int>(tileCells[d]))
-                     & (P.delta[d] == P.delta[d]) & __builtin_isfinite(P.v[d] * P.w * coef);
-            }
-            int const key = ok ? rel[0] * p12 + rel[1] * p2 + rel[2] : -1;
-            // the half rows in turn: first the accumulated window's cell, then every other cell
-#pragma unroll
-            for (int half = 0; half < 2; ++half)
-            {
-                unsigned int rest = static_cast<unsigned int>(__ballot(ok) >> (32 * half));
-                if (rest == 0u)
-                    continue;
-                pc::cellStage<O, RN>(buf, half, ok, P.delta, P.w, q, P.v, coef);
-                unsigned int m = cur < 0 ? 0u : static_cast<unsigned int>(__ballot(key == cur) >> (32 * half));
-                if (m)
-                    pc::cellAdd<O, RN>(buf, m, acc);
-                rest &= ~m;
-                while (rest)
-                {
-                    int const p = __builtin_ctz(rest);
-                    int const c = __builtin_amdgcn_readlane(key, p + 32 * half);
-                    m           = static_cast<unsigned int>(__ballot(key == c) >> (32 * half)) & rest;
-                    rest &= ~m;
-                    int const n = __popc(m);
-                    if (n >= CELL_MOVE || cur < 0)
-                    {
-                        if (cur >= 0)
-                            pc::cellFlush<O, RN>(acc, lds, T.stride, cur, p12, p2);
-                        acc.zero();
-                        cur = c;
-                        pc::cellAdd<O, RN>(buf, m, acc);
-                    }
-                    else if (n >= CELL_GROUP)
-                    {
-                        C one;
-                        one.zero();
-                        pc::cellAdd<O, RN>(buf, m, one);
-                        pc::cellFlush<O, RN>(one, lds, T.stride, c, p12, p2);
-                    }
-                    else
-                        pc::cellAddOne<O, RN>(buf, p, lds, T.stride, c, p12, p2);
-                }
-            }
-            unsigned long long const left = __ballot(live && !ok);
-            if (left)
-            {
-                unsigned int base = 0;
-                if (lane == 0)
-                    base = atomicAdd(&listed, static_cast<unsigned int>(__popcll(left)));
-                base = __builtin_amdgcn_readfirstlane(base);
-                if ((left >> lane) & 1ull)
-                    list[base + __popcll(left & ((1ull << lane) - 1ull))] = r * LANES + lane;
-            }
-            if (writes)
-            {
-                if (ok)
-                {
-#pragma unroll
-                    for (int d = 0; d < 3; ++d)
-                    {
-                        rowOf(K.v.ic[d], row)[lane] = P.cell[d];
-                        rowOf(K.v.de[d], row)[lane] = P.delta[d];
-                        rowOf(K.v.v[d], row)[lane]  = P.v[d];
-                    }
-                }
-                uint8_t* const status = K.A.status;
-                if (status && (ok || !live))
-                    rowOf(status, row)[lane] = live ? ST_KEEP : ST_DROP;
-            }
-        }
-        if (cur >= 0)
-            pc::cellFlush<O, RN>(acc, lds, T.stride, cur, p12, p2);
-        __syncthreads();
-        unsigned int const n = listed;
-        CellArgs const& L    = cellArgs();
-        Acc<3, O> none;
-        for (unsigned int x = threadIdx.x; x < n; x += CB)
-            pushParticle<3, O, RN, true>(L.A, L.v, L.v, off + list[x], T, 0, none);
-        __syncthreads();
+        nItems = *K.A.st.nItems;
+        if (blockIdx.x >= nItems)
+            return;
+        pc::ktBegin(K.A.kt);
+        seg = K.A.st.items[2 * blockIdx.x];
+        pc::itemRows(K.A.st.items[2 * blockIdx.x + 1], K.A.st.rows[seg],
+                     K.A.st.rowsPerItem, rA, rB);
+    }
+    if (rB > rA && !K.A.G.stopped())
+    {
+        unsigned int const rows = rB - rA;
+        unsigned int const lane = threadIdx.x & 63u;
+        unsigned int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        unsigned long long const off = K.A.st.off[seg];
+        constexpr int EX  = cellStage(D, O) | 1;
+        int const e1      = D == 2 ? (FIX ? EX : K.A.tile.emExt[1] | 1) : (FIX ? cellStage(3, O) : K.A.tile.emExt[1]);
+        int const e2      = D == 2 ? 1 : (FIX ? EX : K.A.tile.emExt[2] | 1);
+        int const emNodes = K.A.tile.emExt[0] * e1 * e2;
+        double* const em  = lds + (RN ? 4 : 5) * K.A.tile.stride;
+        double* const buf = em + K.A.tile.emStride + wave * C::BUF;
+        zeroTile<RN, CB>(lds, K.A.tile);
         if (threadIdx.x == 0)
             listed = 0u;
-    } while (__syncthreads_or(r < rEnd));
-    PushArgs const& A = cellArgs().A;
-    flushTile<3, RN, CB>(A.G, T, A.tile.nodes, A.mom, A.charge);
+        TileView T;
+        tileView(T, lds, K.A.tile);
+        pc::segTileOrigin<D>(K.A.G, K.A.sg, K.A.tile, seg, T.org);
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            T.org[d] = __builtin_amdgcn_readfirstlane(T.org[d]); // the same in every lane: scalar from here on
+        int const p2 = T.pitch[2], p12 = T.pitch[1] * T.pitch[2];
+        bool const push   = K.A.pushOn;
+        bool const writes = push && K.A.mode == MODE_ALL;
+        // per direction: AMR cell of the deposit tile's and of the stage's first cell, and the number
+        // of cells whose windows (stencils) they hold; the stage's cells are clipped to those whose
+        // stencils lie in the arrays
+        int tileCell[D], tileCells[D], emCell[D], emLow[D], emCells[D], emOrg[D], dom[D], domCells[D];
+        double h[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+        {
+            int const shift = K.A.G.lower[d] - K.A.G.g; // AMR cell of local cell 0
+            tileCell[d]     = T.org[d] + C::WB + shift;
+            tileCells[d]    = max(T.ext[d] - C::W + 1, 0);
+            emOrg[d]        = T.org[d] + K.A.tile.emLo[d];
+            emCell[d]       = emOrg[d] + shift;
+            int const lo    = max(emOrg[d] - cellGatherLo(O), K.A.G.safeLo[d]);
+            int const hi    = min(emOrg[d] - cellGatherLo(O) + K.A.tile.emExt[d] - cellGatherNodes(O), K.A.G.safeHi[d]);
+            emLow[d]        = lo + shift;
+            emCells[d]      = max(hi - lo + 1, 0);
+            dom[d]          = K.A.box.dom_lo[d];
+            domCells[d]     = K.A.box.dom_hi[d] - dom[d] + 1;
+            h[d]            = K.A.hdtdx[d];
+        }
+        double const dto2m = K.A.dto2m, coef = K.A.coef, charge = K.A.charge;
+        if (push)
+            stageFields<D, CB>(K.A, em, emOrg, e1, e2, emNodes);
+        __syncthreads();
+
+        unsigned int r          = rA + rows * wave / CellCfg<D, O>::NW;
+        unsigned int const rEnd = rA + rows * (wave + 1) / CellCfg<D, O>::NW;
+        do
+        {
+            C acc;
+            acc.zero();
+            int cur = -1; // tile node of the accumulated window's origin
+            Part<D> next;
+            if (NEXT && r < rEnd)
+                loadRow<D, RN>(K.v, off + static_cast<unsigned long long>(r) * LANES, lane, next);
+            for (; r < rEnd; ++r)
+            {
+                // until the list might overflow (each wavefront that still finds room may add 64)
+                if (__builtin_amdgcn_readfirstlane(*static_cast<unsigned int volatile*>(&listed)) > LIST - CB)
+                    break;
+                unsigned long long const row = off + static_cast<unsigned long long>(r) * LANES;
+                Part<D> P;
+                if constexpr (NEXT)
+                {
+                    P = next;
+                    if (r + 1 < rEnd)
+                        loadRow<D, RN>(K.v, row + LANES, lane, next); // in flight over this row's work
+                }
+                else
+                    loadRow<D, RN>(K.v, row, lane, P);
+                double const q  = RN ? charge : P.q;
+                bool const live = P.cell[0] != DEAD_CELL;
+                bool ok         = live;
+                if (push)
+                {
+                    ok = halfStep<D>(P.cell, P.delta, P.v, h) & ok;
+                    int rel[D];
+#pragma unroll
+                    for (int d = 0; d < D; ++d)
+                    {
+                        ok     = ok & (static_cast<unsigned int>(P.cell[d] - emLow[d]) < static_cast<unsigned int>(emCells[d]));
+                        rel[d] = P.cell[d] - emCell[d];
+                    }
+                    double E[3] = {0., 0., 0.}, B[3] = {0., 0., 0.};
+                    if (ok)
+                        gatherStaged<D, O>(em, e1, e2, emNodes, rel, P.delta, E, B);
+                    borisAccelerate(P.v, E, B, q, dto2m);
+                    ok = halfStep<D>(P.cell, P.delta, P.v, h) & ok;
+#pragma unroll
+                    for (int d = 0; d < D; ++d)
+                        ok = ok & (static_cast<unsigned int>(P.cell[d] - dom[d]) < static_cast<unsigned int>(domCells[d]));
+                }
+                // the tile node of the window's origin; a value that is not finite (it would reach the
+                // whole window) deposits by itself
+                ok = ok & __builtin_isfinite(P.w * coef) & (RN || __builtin_isfinite(q * P.w * coef));
+                int key = 0;
+#pragma unroll
+                for (int d = 0; d < D; ++d)
+                {
+                    int const rel = P.cell[d] - tileCell[d];
+                    key += rel * (d == 0 ? p12 : (d == 1 ? p2 : 1));
+                    ok = ok & (static_cast<unsigned int>(rel) < static_cast<unsigned int>(tileCells[d]))
+                         & (P.delta[d] == P.delta[d]);
+                }
+#pragma unroll
+                for (int d = 0; d < 3; ++d)
+                    ok = ok & __builtin_isfinite(P.v[d] * P.w * coef);
+                key = ok ? key : -1;
+                // the half rows in turn: first the accumulated window's cell, then every other cell
+#pragma unroll
+                for (int half = 0; half < 2; ++half)
+                {
+                    unsigned int rest = static_cast<unsigned int>(__ballot(ok) >> (32 * half));
+                    if (rest == 0u)
+                        continue;
+                    pc::cellStage<D, O, RN>(buf, half, ok, P.delta, P.w, q, P.v, coef);
+                    unsigned int m = cur < 0 ? 0u : static_cast<unsigned int>(__ballot(key == cur) >> (32 * half));
+                    if (m)
+                        pc::cellAdd<D, O, RN>(buf, m, acc);
+                    rest &= ~m;
+                    while (rest)
+                    {
+                        int const p = __builtin_ctz(rest);
+                        int const c = __builtin_amdgcn_readlane(key, p + 32 * half);
+                        m           = static_cast<unsigned int>(__ballot(key == c) >> (32 * half)) & rest;
+                        rest &= ~m;
+                        int const n = __popc(m);
+                        if (n >= CELL_MOVE || cur < 0)
+                        {
+                            if (cur >= 0)
+                                pc::cellFlush<D, O, RN>(acc, lds, T.stride, cur, p12, p2);
+                            acc.zero();
+                            cur = c;
+                            pc::cellAdd<D, O, RN>(buf, m, acc);
+                        }
+                        else if (n >= CELL_GROUP)
+                        {
+                            C one;
+                            one.zero();
+                            pc::cellAdd<D, O, RN>(buf, m, one);
+                            pc::cellFlush<D, O, RN>(one, lds, T.stride, c, p12, p2);
+                        }
+                        else
+                            pc::cellAddOne<D, O, RN>(buf, p, lds, T.stride, c, p12, p2);
+                    }
+                }
+                unsigned long long const left = __ballot(live && !ok);
+                if (left)
+                {
+                    unsigned int base = 0;
+                    if (lane == 0)
+                        base = atomicAdd(&listed, static_cast<unsigned int>(__popcll(left)));
+                    base = __builtin_amdgcn_readfirstlane(base);
+                    if ((left >> lane) & 1ull)
+                        list[base + __popcll(left & ((1ull << lane) - 1ull))] = r * LANES + lane;
+                }
+                if (writes)
+                {
+                    if (ok)
+                    {
+#pragma unroll
+                        for (int d = 0; d < D; ++d)
+                        {
+                            rowOf(K.v.ic[d], row)[lane] = P.cell[d];
+                            rowOf(K.v.de[d], row)[lane] = P.delta[d];
+                        }
+#pragma unroll
+                        for (int d = 0; d < 3; ++d)
+                            rowOf(K.v.v[d], row)[lane] = P.v[d];
+                    }
+                    uint8_t* const status = K.A.status;
+                    if (status && (ok || !live))
+                        rowOf(status, row)[lane] = live ? ST_KEEP : ST_DROP;
+                }
+            }
+            if (cur >= 0)
+                pc::cellFlush<D, O, RN>(acc, lds, T.stride, cur, p12, p2);
+            __syncthreads();
+            unsigned int const n = listed;
+            CellArgs const& L    = cellArgs();
+            Acc<D, O> none;
+            for (unsigned int x = threadIdx.x; x < n; x += CB)
+                pushParticle<D, O, RN, true>(L.A, L.v, L.v, off + list[x], T, 0, none);
+            __syncthreads();
+            if (threadIdx.x == 0)
+                listed = 0u;
+        } while (__syncthreads_or(r < rEnd));
+        PushArgs const& A = cellArgs().A;
+        flushTile<D, RN, CB>(A.G, T, A.tile.nodes, A.mom, A.charge);
+    }
+    if (D == 2 && K.A.kt)
+    {
+        __syncthreads();
+        pc::ktEnd(K.A.kt, nItems);
+    }
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1357,7 +1399,8 @@ __global__ __launch_bounds__(BLOCK) void k_seg_count(SegGeom S, V v, unsigned lo
 __global__ __launch_bounds__(BLOCK) void k_seg_rows(SegGeom S, unsigned int* __restrict__ counts,
                                                     unsigned int* __restrict__ rows,
                                                     unsigned int* __restrict__ itemCount,
-                                                    unsigned int* __restrict__ total)
+                                                    unsigned int* __restrict__ total,
+                                                    unsigned int rowsPerItem)
 {
     __shared__ unsigned int sc[BLOCK];
     unsigned int const s = blockIdx.x * (BLOCK / LANES) + threadIdx.x / LANES;
@@ -1388,8 +1431,7 @@ __global__ __launch_bounds__(BLOCK) void k_seg_rows(SegGeom S, unsigned int* __r
     {
         unsigned int const R = (T + LANES - 1) / LANES;
         rows[s]              = R;
-        unsigned int const k = static_cast<unsigned int>(S.rowsPerItem);
-        itemCount[s]         = (R + k - 1) / k;
+        itemCount[s]         = (R + rowsPerItem - 1) / rowsPerItem;
         total[s]             = T;
     }
 }
@@ -1578,7 +1620,8 @@ static void segCountT(SegGeom const& sg, V const& src, unsigned long long n, uns
         k_seg_count<V><<<static_cast<unsigned int>((n + BLOCK - 1) / BLOCK), BLOCK, 0, s>>>(sg, src, n,
                                                                                           counts, rank);
     k_seg_rows<<<(m + SEGS_PER_BLOCK - 1) / SEGS_PER_BLOCK, BLOCK, 0, s>>>(sg, counts, tables.rows,
-                                                                           itemCount, total);
+                                                                           itemCount, total,
+                                                                           tables.rowsPerItem);
     k_seg_scan<<<1, 1024, 0, s>>>(tables.rows, tables.off, itemCount, tables.nItems, m);
 }
 
@@ -1593,7 +1636,7 @@ static void segScatterT(SegGeom const& sg, V const& src, V const& dst, unsigned 
     unsigned int* itemCount = work + nc;
     unsigned int* total     = work + nc + m;
     k_seg_items<<<(m + BLOCK - 1) / BLOCK, BLOCK, 0, s>>>(tables.rows, itemCount, tables.items, m,
-                                                         static_cast<unsigned int>(sg.rowsPerItem));
+                                                         tables.rowsPerItem);
     if (n)
         k_seg_perm<V><<<static_cast<unsigned int>((n + BLOCK - 1) / BLOCK), BLOCK, 0, s>>>(
             sg, src, n, rank, first, tables.rows, tables.off, perm);
@@ -1696,9 +1739,42 @@ TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies, int sla
 }
 
 
-unsigned int segItemsCap(SegGeom const& sg, unsigned long long capacity)
+// rows per work item of an array of `slots` slots, at most `most`: of k items per segment, each as
+// costly as its rows and ITEM_OVERHEAD more (its tile zeroed, staged and flushed), the k whose items
+// finish first in rounds of the workgroups the GPU holds at once (four per CU). 2D Harris, per PPC
+// step: 256x128, order 2, 100 per cell 287 us with one round (51 rows per item), 303 with two; 190x150,
+// order 3, 64 per cell 254 us with 32 rows, 290 with 16 (three rounds). Two species in 1D (order 3, 1000
+// cells, 200 per cell): 184 us per step in 112 workgroups of 32 rows, 121 in one round. The FP32 push holds more
+// workgroups and keeps the tuned rows (2D order 2: 287 us of 24 rows, 294 of one round)
+unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most)
 {
-    return static_cast<unsigned int>(capacity / (LANES * static_cast<unsigned long long>(sg.rowsPerItem)))
+    constexpr double ITEM_OVERHEAD = 6.;
+    constexpr double MIN_ROWS      = 4.;    // a row per wavefront
+    constexpr double SPREAD        = 1.125; // segments this far above the average still take k items
+    constexpr double HELD          = 4. * CUS;
+    constexpr double ROUNDS        = 4.; // past these more items only add overhead
+    double const segs = std::max(sg.nsegs, 1);
+    double const rows = std::max(1., static_cast<double>(slots) / LANES / segs);
+    double best       = 0.;
+    int bestRows      = most;
+    for (int k = 1; k == 1 || rows / k >= MIN_ROWS; ++k)
+    {
+        double const each = rows / k;
+        double const cost = std::ceil(segs * k / HELD) * (each + ITEM_OVERHEAD);
+        if (each <= most && (best == 0. || cost < best))
+        {
+            best     = cost;
+            bestRows = static_cast<int>(std::min(std::ceil(SPREAD * each), static_cast<double>(most)));
+        }
+        if (best > 0. && segs * k > ROUNDS * HELD)
+            break;
+    }
+    return static_cast<unsigned int>(std::max(1, bestRows));
+}
+
+unsigned int segItemsCap(SegGeom const& sg, SegTables const& tables, unsigned long long capacity)
+{
+    return static_cast<unsigned int>(capacity / (LANES * static_cast<unsigned long long>(tables.rowsPerItem)))
            + static_cast<unsigned int>(sg.nsegs)
            + 2u;
 }
@@ -1709,7 +1785,7 @@ unsigned int segItemsCap(SegGeom const& sg, unsigned long long capacity)
 template<int D, int O>
 static void launchPushT(PushArgs const& A, PView const& in, PView const& out, hipStream_t s)
 {
-    if constexpr (D == 3)
+    if constexpr (D > 1)
     {
         if (A.segOn)
         {
@@ -1871,37 +1947,37 @@ void launchCompact(PView const& src, PView const& dst, uint8_t const* status, un
                                           wrap);
 }
 
-// tile of the cell-grouped 3D push: the window of every cell of the largest segment and of the
-// cells around it (one cell of motion), and the staged fields of the segment's gather
-TileSpec cellTileShape(int order, SegGeom const& sg, int slabs, int pad)
+// tile of the cell-grouped push: the window of every cell of the largest segment and of the cells
+// around it (one cell of motion), and the staged fields of the segment's gather
+TileSpec cellTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad)
 {
     TileSpec T{};
-    T.copies = 1;
+    T.copies    = 1;
     int emNodes = 1;
-    bool fix    = true; // the stage of a 4x4x4 segment holds every segment's
-    for (int d = 0; d < 3; ++d)
-        fix = fix && sg.maxSeg[d] <= 4;
-    T.emFix = fix;
+    T.emFix     = 1; // the pitches of the default segments' stage hold every segment
+    for (int d = 1; d < dim; ++d)
+        T.emFix = T.emFix && sg.maxSeg[d] <= cellFixed(dim);
     for (int d = 0; d < 3; ++d)
     {
-        T.lo[d]    = order == 1 ? 1 : 2;
-        T.ext[d]   = sg.maxSeg[d] + (order == 1 ? 3 : 5);
+        bool const on = d < dim;
+        T.lo[d]    = !on ? 0 : (order == 1 ? 1 : 2);
+        T.ext[d]   = !on ? 1 : sg.maxSeg[d] + (order == 1 ? 3 : 5);
         T.pitch[d] = T.ext[d];
         T.emLo[d]  = T.lo[d] + cellGatherLo(order) - 1;
-        T.emExt[d] = (fix ? 4 : sg.maxSeg[d]) + 1 + cellGatherNodes(order);
-        emNodes *= d == 2 ? T.emExt[d] | 1 : T.emExt[d];
+        T.emExt[d] = !on ? 1 : (d > 0 && T.emFix ? cellFixed(dim) : sg.maxSeg[d]) + 1 + cellGatherNodes(order);
+        emNodes *= d == dim - 1 ? T.emExt[d] | 1 : T.emExt[d];
     }
     T.emStride = (6 * emNodes + 15) / 16 * 16;
     // the hand-over buffers of the workgroup's wavefronts
-    unsigned int const waves = static_cast<unsigned int>(cellBlock(order)) / LANES;
-    unsigned int const rest = 8u * static_cast<unsigned int>(T.emStride)
-                              + waves * 8u * static_cast<unsigned int>(pc::WSTR * ((order == 1 ? 6 : 12) + slabs));
+    unsigned int const waves = static_cast<unsigned int>(cellBlock(dim, order)) / LANES;
+    unsigned int const rest  = 8u * static_cast<unsigned int>(T.emStride)
+                              + waves * 8u * static_cast<unsigned int>(pc::WSTR * (dim * (order == 1 ? 2 : 4) + slabs));
     auto size = [&]() {
         T.nodes  = T.ext[0] * T.pitch[1] * T.pitch[2];
         T.stride = (T.nodes + 15) / 16 * 16;
         T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride) + rest;
     };
-    if (pad > 1)
+    if (dim == 3 && pad > 1)
     {
         // pitches of dimensions 1 and 2 padded to a multiple of pad nodes (the padding nodes are
         // never deposited into: the flush skips them as zeros); dropped if the tile outgrows LDS
@@ -1928,7 +2004,7 @@ TileSpec cellTileShape(int order, SegGeom const& sg, int slabs, int pad)
         T.nodes    = 1;
         T.stride   = 16;
         T.emStride = 16;
-        T.bytes    = static_cast<unsigned int>(8 * (slabs * T.stride + T.emStride)) + NW * 8u * pc::WSTR * 17u;
+        T.bytes    = static_cast<unsigned int>(8 * (slabs * T.stride + T.emStride)) + waves * 8u * pc::WSTR * 17u;
     }
     return T;
 }
@@ -1941,12 +2017,12 @@ unsigned int cellSplit(int order, SegGeom const& sg, unsigned long long slots)
     unsigned long long const segs = static_cast<unsigned long long>(std::max(sg.nsegs, 1));
     unsigned long long const held = CUS * (order == 3 ? 1 : 2);
     unsigned long long const rows = slots / LANES / segs;
-    unsigned long long const most = rows / (2 * static_cast<unsigned long long>(cellBlock(order)) / LANES);
+    unsigned long long const most = rows / (2 * static_cast<unsigned long long>(cellBlock(3, order)) / LANES);
     unsigned long long const want = (3 * held + segs - 1) / segs;
     return static_cast<unsigned int>(std::max(1ull, std::min(want, most)));
 }
 
-template<int O, bool RN, bool FIX>
+template<int D, int O, bool RN, bool FIX>
 static void launchPushCellT(PushArgs const& A, PView const& in, hipStream_t s)
 {
     // more than 64 KB of dynamic LDS has to be allowed for the kernel (once per device)
@@ -1957,30 +2033,33 @@ static void launchPushCellT(PushArgs const& A, PView const& in, hipStream_t s)
     {
         std::lock_guard<std::mutex> lock(mtx);
         if (!allowed[dev])
-            allowed[dev] = hipFuncSetAttribute(reinterpret_cast<void const*>(&k_push_cell<O, RN, FIX>),
+            allowed[dev] = hipFuncSetAttribute(reinterpret_cast<void const*>(&k_push_cell<D, O, RN, FIX>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, CELL_LDS_MAX)
                            == hipSuccess;
     }
-    unsigned int const grid = (static_cast<unsigned int>(A.sg.nsegs) + 1u) * A.split;
-    k_push_cell<O, RN, FIX><<<grid, CellCfg<O>::BLOCK, A.tile.bytes, s>>>(CellArgs{A, in});
+    unsigned int const grid = D == 3 ? (static_cast<unsigned int>(A.sg.nsegs) + 1u) * A.split : A.st.itemsCap;
+    k_push_cell<D, O, RN, FIX><<<grid, CellCfg<D, O>::BLOCK, A.tile.bytes, s>>>(CellArgs{A, in});
 }
 
-template<int O>
+template<int D, int O>
 static void launchPushCellO(PushArgs const& A, PView const& in, hipStream_t s)
 {
     if (A.rhoFromN)
-        A.tile.emFix ? launchPushCellT<O, true, true>(A, in, s) : launchPushCellT<O, true, false>(A, in, s);
+        A.tile.emFix ? launchPushCellT<D, O, true, true>(A, in, s) : launchPushCellT<D, O, true, false>(A, in, s);
     else
-        A.tile.emFix ? launchPushCellT<O, false, true>(A, in, s) : launchPushCellT<O, false, false>(A, in, s);
+        A.tile.emFix ? launchPushCellT<D, O, false, true>(A, in, s) : launchPushCellT<D, O, false, false>(A, in, s);
 }
 
 void launchPushCell(PushArgs const& A, PView const& in, hipStream_t s)
 {
-    switch (A.G.order)
+    switch (A.G.dim * 10 + A.G.order)
     {
-        case 1: launchPushCellO<1>(A, in, s); break;
-        case 2: launchPushCellO<2>(A, in, s); break;
-        case 3: launchPushCellO<3>(A, in, s); break;
+        case 21: launchPushCellO<2, 1>(A, in, s); break;
+        case 22: launchPushCellO<2, 2>(A, in, s); break;
+        case 23: launchPushCellO<2, 3>(A, in, s); break;
+        case 31: launchPushCellO<3, 1>(A, in, s); break;
+        case 32: launchPushCellO<3, 2>(A, in, s); break;
+        case 33: launchPushCellO<3, 3>(A, in, s); break;
         default: break;
     }
 }

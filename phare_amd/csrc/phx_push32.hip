@@ -730,7 +730,7 @@ __device__ __forceinline__ void flushTile32(PushArgs const& A, Tile32 const& T)
 } // namespace
 
 // one workgroup per work item (a segment and its share of the segment's rows, at most
-// sg.rowsPerItem)
+// st.rowsPerItem)
 template<int D, int O, bool WIN>
 __global__ __launch_bounds__(pc::SEG_BLOCK)
 __attribute__((amdgpu_waves_per_eu(WIN ? PHX_SEG_WAVES32_WIN : PHX_SEG_WAVES32)))
@@ -747,7 +747,7 @@ void k_push_seg32(PushArgs A, PView32 v)
         unsigned int const seg = A.st.items[2 * item];
         unsigned int const R   = A.st.rows[seg];
         unsigned int r0, rEnd;
-        pc::itemRows(A.st.items[2 * item + 1], R, static_cast<unsigned int>(A.sg.rowsPerItem), r0, rEnd);
+        pc::itemRows(A.st.items[2 * item + 1], R, A.st.rowsPerItem, r0, rEnd);
         pushPiece32<D, O, WIN>(A, v, lds32, seg, r0, rEnd);
     }
     if (A.kt)
