@@ -37,8 +37,8 @@ HBM_PEAK_GBS = 8000.0
 
 # HBM bytes per push dispatch (mode all) from rocprofv3 --pmc FETCH_SIZE and WRITE_SIZE runs of
 # this script, FETCH_SIZE scaled x2 and WRITE_SIZE x1 by a 1 GiB device copy's readings; keyed by
-# workload and precision family (k_push_seg / k_push_seg32 in 2D, k_push_cell / k_push32_segwg on
-# the 3D staged path)
+# workload and precision family (k_push_cell, in 2D mixed precision at orders 1 and 2
+# k_push_seg32)
 MEASURED_TRAFFIC = {("harris2d", "fp64"): 395.0e6, ("harris2d", "fp32"): 224.3e6,
                     ("uniform3d", "fp64"): 19.41e9, ("uniform3d", "fp32"): 11.03e9}
 
@@ -204,7 +204,7 @@ def family_line(wl, workload_name, precision, res):
     b = push_bytes(wl, phx.MODE_ALL, precision)
     a = b / (res["ms_all"] * 1e-3) / 1e9
     if wl.dim == 3:
-        kernel = ("k_push32_segwg (mixed precision" if precision == "fp32" else "k_push_cell (FP64") + \
+        kernel = ("k_push_cell (mixed precision" if precision == "fp32" else "k_push_cell (FP64") + \
             ", cell-segmented storage, one workgroup per 4x4x4-cell segment: prePush+gather+Boris+" \
             "postPush+deposit, mode all; 3D staged path)"
     elif precision == "fp32":

@@ -327,7 +327,7 @@ phx_status phx_advance(phx_ctx* ctx, double dt, int nsteps);
 /* Storage order (no counterpart in the reference, whose ParticleArray keeps insertion order and
    a CellMap): reorders every population's domain particles by cell, row-major over the AMR box,
    the order the push kernel's LDS deposit tile relies on. phx_initialize sorts once and
-   phx_advance every `steps` PPC steps (0: never; default 30, an FP64 level in 3D 7). Results do not depend on the order
+   phx_advance every `steps` PPC steps (0: never; default 30, in 3D 7). Results do not depend on the order
    beyond the summation order of the deposit. */
 phx_status phx_sort_particles(phx_ctx* ctx);
 phx_status phx_set_sort_interval(phx_ctx* ctx, int steps);
@@ -348,14 +348,14 @@ typedef struct {
                              most 64; clipped to each patch, the cells left over go to the slower
                              dimensions); 0 keeps the default of the dimension */
     int rows_per_item;    /* most segment rows per workgroup of the segmented push (1..4096); an
-                             FP64 level takes fewer where that fills the GPU better */
+                             FP64 or cell-grouped FP32 array takes fewer where that fills the GPU */
     int tile_row_pad;     /* LDS tile pitches padded to a multiple of this many nodes (1: none):
-                             the pitches of dimensions 1 and 2; FP32 in 2D its rows */
+                             the pitches of dimensions 1 and 2 */
     int sort_interval;    /* PPC steps of phx_advance between two sorts (0: never) */
     int tile_copies;      /* moment copies of the LDS tile of the linear-storage push (1, 2, 4, 8;
                              lane l adds into copy l % copies) */
     int deposit_window;   /* mixed-precision push: 1 sums each lane's successive particles of one
-                             cell in registers before the LDS tile (1D, 2D and 3D order 1), 0 adds
+                             cell in registers before the LDS tile (1D, and 2D orders 1 and 2), 0 adds
                              every particle into the tile */
 } phx_tuning;
 phx_status phx_get_tuning(const phx_ctx* ctx, phx_tuning* out);

@@ -447,16 +447,16 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
     A.tile = tileShape(c->cfg.dim, c->cfg.interp_order, ppc, copies);
     Pop const& P   = c->pops[pop];
     Store const& s = P.arr[kind];
-    // 2D and 3D, FP64: the cell-grouped push, which gives every slot its fate
+    // the cell-grouped push, which gives every slot its fate
     if (c->sg.dense && kind == KIND_DOMAIN && s.seg)
     {
         A.segOn       = 1;
         A.sg          = c->sg;
         A.st          = P.seg;
         A.st.itemsCap = segItemsCap(c->sg, P.seg, s.cap);
-        A.rhoFromN    = P.hasCharge && P.uniformCharge ? 1 : 0;
-        A.split       = cellSplit(c->cfg.interp_order, c->sg, s.n);
-        A.tile = cellTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, A.rhoFromN ? 4 : 5, c->tuning.tile_row_pad);
+        A.rhoFromN    = mixed(c) || (P.hasCharge && P.uniformCharge) ? 1 : 0;
+        A.split       = cellSplit(mixed(c), c->cfg.interp_order, c->sg, s.n);
+        A.tile = cellTileShape(mixed(c), c->cfg.dim, c->cfg.interp_order, c->sg, A.rhoFromN ? 4 : 5, c->tuning.tile_row_pad);
         noteTileFallback(c, A.tile);
         return A;
     }
@@ -728,19 +728,13 @@ phx_status enqueueAdvanceFast(phx_ctx* c, double dt)
 bool staged3d(phx_ctx const* c) { return c->cfg.dim == 3 && c->patch.periodic; }
 
 // the push (or, pushOn 0, the deposit) of population p's domain array on the staged 3D path:
-// cell-segmented storage (after a sort) with one workgroup per segment, otherwise the linear
-// brick-tiled kernels; FP64 or mixed precision
+// cell-segmented storage (after a sort) by the cell-grouped push, otherwise the linear brick-tiled kernels; FP64 or mixed precision
 void enqueuePushStaged3d(phx_ctx* c, int p, PushArgs& A)
 {
-    Pop const& P     = c->pops[p];
-    Store const& dom = P.arr[PHX_DOMAIN];
+    Store const& dom = c->pops[p].arr[PHX_DOMAIN];
     if (mixed(c) && dom.seg)
     {
-        A.sg   = c->sg;
-        A.st   = P.seg;
-        A.tile = segwgTileShape(c->cfg.dim, c->cfg.interp_order, c->sg, 4, c->tuning.tile_row_pad);
-        noteTileFallback(c, A.tile);
-        launchPush32SegWG(A, dom.view32(), c->stream);
+        launchPush32(A, dom.view32(), c->stream);
         return;
     }
     if (mixed(c))
@@ -1112,7 +1106,7 @@ phx_status sortDomain(phx_ctx* c)
         // kept while the array stays segmented and of about this size: a captured step holds it
         if (!dom.seg || P.itemsFor == 0 || dom.n > 2 * P.itemsFor || 2 * dom.n < P.itemsFor)
         {
-            P.seg.rowsPerItem = mixed(c) ? static_cast<unsigned int>(c->tuning.rows_per_item)
+            P.seg.rowsPerItem = mixed(c) && !c->sg.dense ? static_cast<unsigned int>(c->tuning.rows_per_item)
                                          : itemRowsFor(c->sg, dom.n, c->tuning.rows_per_item);
             P.itemsFor        = std::max<size_t>(dom.n, 1);
         }
@@ -1297,7 +1291,7 @@ phx_status buildPatchTable(phx_ctx* c, int const* plo, int const* phi, int np)
     for (Pop& P : c->pops)
         P.itemsFor = 0;
     S.rowPad      = c->tuning.tile_row_pad;
-    S.dense       = D > 1 && !mixed(c) ? 1 : 0;
+    S.dense       = cellGrouped(D, c->cfg.interp_order, mixed(c)) ? 1 : 0;
     size_t boxCells = 1;
     for (int d = 0; d < 3; ++d)
     {
@@ -1401,23 +1395,20 @@ phx_status allocSegTables(phx_ctx* c)
 // the launch shapes of this build before any tuning: the autotuner's winners on the 2D Harris
 // workload (segments of 2x32 cells, at most 32 rows per work item, tile rows padded to 16 nodes,
 // a sort every 30 PPC steps); runs of 64 cells in 1D, 4x4x4 blocks in 3D
-phx_tuning defaultTuning(int dim, int order, bool fp32)
+phx_tuning defaultTuning(int dim)
 {
     phx_tuning t{};
     static int const pref[3][3] = {{64, 1, 1}, {2, 32, 1}, {4, 4, 4}};
     for (int d = 0; d < 3; ++d)
         t.segment_shape[d] = pref[dim - 1][d];
     t.rows_per_item = PHX_SEG_ROWS;
-    // 3D, mixed precision: the segment tile's pitches padded to a multiple of 4 nodes at orders 1
-    // and 3 (every particle's stencil starts at a fixed node of its cell, so the 64 lanes of one LDS
-    // atomic fall on distinct bank pairs); unpadded at order 2 (starts shift with the delta at
-    // random, and the larger tile would halve the workgroups per CU), and in FP64, whose particles
-    // deposit by cell
-    t.tile_row_pad  = dim == 3 ? (order == 2 || !fp32 ? 1 : 4) : PHX_TILE_ROW_PAD;
+    // 3D: unpadded, the particles of a cell deposit together and a larger tile only costs LDS
+    t.tile_row_pad  = dim == 3 ? 1 : PHX_TILE_ROW_PAD;
     // the cell-grouped 3D push slows with every particle that has left its cell since the sort (64^3
     // cells, order 2, 64 per cell, per PPC step: 3.61 ms sorted every 30 steps, 3.27 every 15, 3.12
-    // every 7, 3.17 every 3; orders 1 and 3 within 1 % of their best at 7 too)
-    t.sort_interval = dim == 3 && !fp32 ? 7 : 30;
+    // every 7, 3.17 every 3; FP32 3.30 every 30, 2.89 every 12, 2.78 every 7; orders 1 and 3 within 1 % of
+    // their best at 7 too)
+    t.sort_interval = dim == 3 ? 7 : 30;
     t.tile_copies   = dim == 1 ? PHX_TILE_COPIES_1D : (dim == 2 ? PHX_TILE_COPIES_2D : PHX_TILE_COPIES_3D);
     t.deposit_window = 0;
     return t;
@@ -1581,7 +1572,7 @@ phx_status createLevel(phx_config const* cfg, phx_patch const* patch, int const*
         for (int k = 0; k < 5 && s == PHX_OK; ++k)
             s = storeAlloc(c, c->pops[p].arr[k], k == 0 ? std::max<size_t>(particle_capacity, 1024) : 1024);
     }
-    c->tuning = defaultTuning(D, cfg->interp_order, mixed(c));
+    c->tuning = defaultTuning(D);
     c->sortInterval = c->tuning.sort_interval;
     if (s == PHX_OK)
         s = buildPatchTable(c, plo, phi, np);
@@ -2839,7 +2830,7 @@ phx_status phx_set_tuning(phx_ctx* c, phx_tuning const* t)
         return PHX_ERR_ARG;
     int const D       = c->cfg.dim;
     phx_tuning next   = *t;
-    phx_tuning const d = defaultTuning(D, c->cfg.interp_order, mixed(c));
+    phx_tuning const d = defaultTuning(D);
     int cells         = 1;
     for (int k = 0; k < 3; ++k)
     {

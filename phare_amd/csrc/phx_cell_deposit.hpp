@@ -106,61 +106,115 @@ __device__ __forceinline__ int splineStencil(int c, double delta, double* w)
     return sh;
 }
 
+// B-spline weights at u = np - start (u in [0, O+1)); the products of interpolator.hpp:54-125
+// written in u: order 2 uses 1 - u for (start + 1 - np), order 3 uses -u for (start - np)
+template<int O>
+__device__ __forceinline__ void bspline32(float u, float* w)
+{
+    if constexpr (O == 1)
+    {
+        w[1] = u;
+        w[0] = 1.f - u;
+    }
+    else if constexpr (O == 2)
+    {
+        float const d  = 1.f - u;
+        float const c1 = .5f + d;
+        float const c3 = .5f - d;
+        w[0]           = .5f * c1 * c1;
+        w[1]           = .75f - d * d;
+        w[2]           = .5f * c3 * c3;
+    }
+    else
+    {
+        float const index = -u;
+        float const c1    = 1.f + .5f * index;
+        float const c2    = index + 1.f;
+        float const c3    = index + 2.f;
+        float const c4    = 1.f - .5f * (index + 3.f);
+        float const c2s   = c2 * c2;
+        float const c3s   = c3 * c3;
+        w[0]              = (4.f / 3.f) * c1 * c1 * c1;
+        w[1]              = (2.f / 3.f) - c2s - .5f * c2s * c2;
+        w[2]              = (2.f / 3.f) - c3s + .5f * c3s * c3;
+        w[3]              = (4.f / 3.f) * c4 * c4 * c4;
+    }
+}
+
+template<int O>
+__device__ __forceinline__ int splineStencil(int c, float delta, float* w)
+{
+    int const sh = startShift<O>(c, static_cast<double>(delta));
+    float u      = static_cast<float>(sh) + delta;
+    if (c == CD)
+        u -= .5f;
+    bspline32<O>(u, w);
+    return sh;
+}
+
 // the primal weights of one direction on the cell's window (zero on the node an order-2 stencil
 // leaves out)
-template<int O>
-__device__ __forceinline__ void windowWeights(double delta, double* out)
+template<int O, class R>
+__device__ __forceinline__ void windowWeights(R delta, R* out)
 {
     if constexpr (O == 2)
     {
-        double w[3];
+        R w[3];
         bool const low = splineStencil<2>(CP, delta, w) == 1;
-        out[0]         = low ? w[0] : 0.;
+        out[0]         = low ? w[0] : R(0);
         out[1]         = low ? w[1] : w[0];
         out[2]         = low ? w[2] : w[1];
-        out[3]         = low ? 0. : w[2];
+        out[3]         = low ? R(0) : w[2];
     }
     else
         splineStencil<O>(CP, delta, out);
 }
 
+// two neighbouring words of the buffer
+__device__ __forceinline__ double2 pairAt(double const* p) { return *reinterpret_cast<double2 const*>(p); }
+__device__ __forceinline__ double2 pairAt(float const* p)
+{
+    float2 const f = *reinterpret_cast<float2 const*>(p);
+    return double2{static_cast<double>(f.x), static_cast<double>(f.y)};
+}
+
 // the 32 particles of lanes [32 half, 32 half + 32) into the wavefront's buffer: the window weights
 // of delta along each direction, then the values n, Fx, Fy, Fz (and rho); lanes without `ok` hand over finite
 // weights and zero values
-template<int D, int O, bool RN>
-__device__ __forceinline__ void cellStage(double* buf, int half, bool ok, double const* delta, double w,
-                                          double q, double const* v, double coef)
+template<int D, int O, bool RN, class R>
+__device__ __forceinline__ void cellStage(R* buf, int half, bool ok, R const* delta, R weight, double q,
+                                          R const* v, double coef)
 {
     using C        = CellWin<D, O, RN>;
     int const lane = static_cast<int>(threadIdx.x & 63u);
     waveLds(); // the reads of the half before are done
     if ((lane >> 5) == half)
     {
-        double* const b = buf + (lane & (WHALF - 1));
+        R* const b = buf + (lane & (WHALF - 1));
 #pragma unroll
         for (int d = 0; d < D; ++d)
         {
-            double ww[C::W];
-            windowWeights<O>(ok ? delta[d] : 0., ww);
+            R ww[C::W];
+            windowWeights<O>(ok ? delta[d] : R(0), ww);
 #pragma unroll
             for (int a = 0; a < C::W; ++a)
                 b[(d * C::W + a) * WSTR] = ww[a];
         }
         // the reference's products: 1. * w * coef, v * w * coef, q * w * coef
-        b[D * C::W * WSTR] = ok ? w * coef : 0.;
+        b[D * C::W * WSTR] = ok ? weight * static_cast<R>(coef) : R(0);
 #pragma unroll
         for (int d = 0; d < 3; ++d)
-            b[(D * C::W + 1 + d) * WSTR] = ok ? v[d] * w * coef : 0.;
+            b[(D * C::W + 1 + d) * WSTR] = ok ? v[d] * weight * static_cast<R>(coef) : R(0);
         if constexpr (!RN)
-            b[(D * C::W + 4) * WSTR] = ok ? q * w * coef : 0.;
+            b[(D * C::W + 4) * WSTR] = ok ? q * weight * coef : 0.;
     }
     waveLds();
 }
 
 // the staged particles whose bit of `mask` is set (all of one cell) added to the window. ALL: every
 // instruction of the half row is issued, without a branch between them (many particles set)
-template<int D, int O, bool RN, bool ALL>
-__device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, CellWin<D, O, RN>& acc)
+template<int D, int O, bool RN, bool ALL, class R>
+__device__ __forceinline__ void cellAddT(R const* buf, unsigned int mask, CellWin<D, O, RN>& acc)
 {
     using C        = CellWin<D, O, RN>;
     int const lane = static_cast<int>(threadIdx.x & 63u);
@@ -175,19 +229,19 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
         constexpr int PP  = W4 ? 8 : 32; // particles of two instructions
         int const l4 = lane & 3, blk = (lane >> 2) & 3;
         int const o  = W4 ? 2 * k : 8 * k + 2 * blk;
-        double const* const px = buf + (W4 ? l4 : l4 >> 1) * WSTR + o;
-        double const* const py = buf + (C::W + (W4 ? l4 : l4 & 1)) * WSTR + o;
-        double const* const pv = buf + (2 * C::W + (W4 ? blk : l4)) * WSTR + o;
-        double const* const pr = buf + (2 * C::W + 4) * WSTR + o;
+        R const* const px = buf + (W4 ? l4 : l4 >> 1) * WSTR + o;
+        R const* const py = buf + (C::W + (W4 ? l4 : l4 & 1)) * WSTR + o;
+        R const* const pv = buf + (2 * C::W + (W4 ? blk : l4)) * WSTR + o;
+        R const* const pr = buf + (2 * C::W + 4) * WSTR + o;
         unsigned int const mk  = mask >> o;
 #pragma unroll
         for (int t = 0; t < WHALF / PP; ++t)
         {
             if (!ALL && W4 && ((mask >> (8 * t)) & 0xffu) == 0u)
                 continue;
-            double2 const x = *reinterpret_cast<double2 const*>(px + PP * t);
-            double2 const y = *reinterpret_cast<double2 const*>(py + PP * t);
-            double2 const v = *reinterpret_cast<double2 const*>(pv + PP * t);
+            double2 const x = pairAt(px + PP * t);
+            double2 const y = pairAt(py + PP * t);
+            double2 const v = pairAt(pv + PP * t);
             double const v0 = (mk >> (PP * t % 32)) & 1u ? v.x : 0.;
             double const v1 = (mk >> (PP * t % 32)) & 2u ? v.y : 0.;
             if constexpr (W4)
@@ -202,7 +256,7 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
             }
             if constexpr (!RN)
             {
-                double2 const q = *reinterpret_cast<double2 const*>(pr + PP * t);
+                double2 const q = pairAt(pr + PP * t);
                 bool const on   = W4 ? blk == 0 : l4 == 0;
                 double const q0 = on && ((mk >> (PP * t % 32)) & 1u) ? q.x : 0.;
                 double const q1 = on && ((mk >> (PP * t % 32)) & 2u) ? q.y : 0.;
@@ -223,11 +277,11 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
     {
         // rows (a, b) = (i / 4, i % 4) of A, columns (c, m) = (i / 4, i % 4) of B; four particles
         // per instruction, lane group k taking a pair of particles for two instructions
-        double const* const px = buf + (i >> 2) * WSTR + 2 * k;
-        double const* const py = buf + (4 + (i & 3)) * WSTR + 2 * k;
-        double const* const pz = buf + (8 + (i >> 2)) * WSTR + 2 * k;
-        double const* const pv = buf + (12 + (i & 3)) * WSTR + 2 * k;
-        double const* const pr = buf + 16 * WSTR + 2 * k;
+        R const* const px = buf + (i >> 2) * WSTR + 2 * k;
+        R const* const py = buf + (4 + (i & 3)) * WSTR + 2 * k;
+        R const* const pz = buf + (8 + (i >> 2)) * WSTR + 2 * k;
+        R const* const pv = buf + (12 + (i & 3)) * WSTR + 2 * k;
+        R const* const pr = buf + 16 * WSTR + 2 * k;
         unsigned int const mk  = mask >> (2 * k);
         d4 c  = {acc.a[0], acc.a[1], acc.a[2], acc.a[3]};
         d4 cr = {0., 0., 0., 0.};
@@ -238,10 +292,10 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
         {
             if (!ALL && ((mask >> (8 * t)) & 0xffu) == 0u)
                 continue;
-            double2 const x = *reinterpret_cast<double2 const*>(px + 8 * t);
-            double2 const y = *reinterpret_cast<double2 const*>(py + 8 * t);
-            double2 const z = *reinterpret_cast<double2 const*>(pz + 8 * t);
-            double2 const v = *reinterpret_cast<double2 const*>(pv + 8 * t);
+            double2 const x = pairAt(px + 8 * t);
+            double2 const y = pairAt(py + 8 * t);
+            double2 const z = pairAt(pz + 8 * t);
+            double2 const v = pairAt(pv + 8 * t);
             double const a0 = x.x * y.x, a1 = x.y * y.y;
             double const z0 = (mk >> (8 * t)) & 1u ? z.x : 0.;
             double const z1 = (mk >> (8 * t)) & 2u ? z.y : 0.;
@@ -249,7 +303,7 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
             c = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, z1 * v.y, c, 0, 0, 0);
             if constexpr (!RN)
             {
-                double2 const q = *reinterpret_cast<double2 const*>(pr + 8 * t);
+                double2 const q = pairAt(pr + 8 * t);
                 bool const on   = (i & 3) == 0;
                 cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, on ? z0 * q.x : 0., cr, 0, 0, 0);
                 cr = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, on ? z1 * q.y : 0., cr, 0, 0, 0);
@@ -269,21 +323,21 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
         // lane % 4, columns m; eight particles per instruction
         int const s = (lane >> 3) & 1, c = (lane >> 2) & 1;
         int const o = 4 * k + 2 * s;
-        double const* const px = buf + ((lane >> 1) & 1) * WSTR + o;
-        double const* const py = buf + (2 + (lane & 1)) * WSTR + o;
-        double const* const pz = buf + (4 + c) * WSTR + o;
-        double const* const pv = buf + (6 + (lane & 3)) * WSTR + o;
-        double const* const pr = buf + 10 * WSTR + o;
+        R const* const px = buf + ((lane >> 1) & 1) * WSTR + o;
+        R const* const py = buf + (2 + (lane & 1)) * WSTR + o;
+        R const* const pz = buf + (4 + c) * WSTR + o;
+        R const* const pv = buf + (6 + (lane & 3)) * WSTR + o;
+        R const* const pr = buf + 10 * WSTR + o;
         unsigned int const mk  = mask >> o;
 #pragma unroll
         for (int t = 0; t < WHALF / 16; ++t)
         {
             if (!ALL && ((mask >> (16 * t)) & 0xffffu) == 0u)
                 continue;
-            double2 const x = *reinterpret_cast<double2 const*>(px + 16 * t);
-            double2 const y = *reinterpret_cast<double2 const*>(py + 16 * t);
-            double2 const z = *reinterpret_cast<double2 const*>(pz + 16 * t);
-            double2 const v = *reinterpret_cast<double2 const*>(pv + 16 * t);
+            double2 const x = pairAt(px + 16 * t);
+            double2 const y = pairAt(py + 16 * t);
+            double2 const z = pairAt(pz + 16 * t);
+            double2 const v = pairAt(pv + 16 * t);
             double const a0 = x.x * y.x, a1 = x.y * y.y;
             double const z0 = (mk >> (16 * t)) & 1u ? z.x : 0.;
             double const z1 = (mk >> (16 * t)) & 2u ? z.y : 0.;
@@ -291,7 +345,7 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
             acc.a[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, z1 * v.y, acc.a[0], 0, 0, 0);
             if constexpr (!RN)
             {
-                double2 const q = *reinterpret_cast<double2 const*>(pr + 16 * t);
+                double2 const q = pairAt(pr + 16 * t);
                 bool const on   = (lane & 3) == 0;
                 acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a0, on ? z0 * q.x : 0., acc.rho[0], 0, 0, 0);
                 acc.rho[0] = __builtin_amdgcn_mfma_f64_4x4x4f64(a1, on ? z1 * q.y : 0., acc.rho[0], 0, 0, 0);
@@ -300,8 +354,8 @@ __device__ __forceinline__ void cellAddT(double const* buf, unsigned int mask, C
     }
 }
 
-template<int D, int O, bool RN>
-__device__ __forceinline__ void cellAdd(double const* buf, unsigned int mask, CellWin<D, O, RN>& acc)
+template<int D, int O, bool RN, class R>
+__device__ __forceinline__ void cellAdd(R const* buf, unsigned int mask, CellWin<D, O, RN>& acc)
 {
     if (__popc(mask) >= WHALF / 2)
         cellAddT<D, O, RN, true>(buf, mask, acc);
@@ -310,52 +364,53 @@ __device__ __forceinline__ void cellAdd(double const* buf, unsigned int mask, Ce
 }
 
 // one staged particle (p, in no larger group) added to the LDS tile by itself
-template<int D, int O, bool RN>
-__device__ __forceinline__ void cellAddOne(double const* buf, int p, double* tile, int stride, int node0,
+template<int D, int O, bool RN, class R>
+__device__ __forceinline__ void cellAddOne(R const* buf, int p, double* tile, int stride, int node0,
                                            int p12, int p2)
 {
     using C        = CellWin<D, O, RN>;
     int const lane = static_cast<int>(threadIdx.x & 63u);
     int const m    = lane & 3;
     int const slab = RN || m == 0 ? m : m + 1;
+    auto const at  = [&](int x) { return static_cast<double>(buf[x]); };
     if constexpr (D == 2)
     {
         int const a = lane / (4 * C::W), b = lane / 4 % C::W;
         if (a < C::W)
         {
-            double const xy = buf[a * WSTR + p] * buf[(C::W + b) * WSTR + p];
+            double const xy = at(a * WSTR + p) * at((C::W + b) * WSTR + p);
             int const n     = node0 + a * p12 + b * p2;
-            atomicAdd(tile + slab * stride + n, xy * buf[(2 * C::W + m) * WSTR + p]);
+            atomicAdd(tile + slab * stride + n, xy * at((2 * C::W + m) * WSTR + p));
             if constexpr (!RN)
                 if (m == 0)
-                    atomicAdd(tile + stride + n, xy * buf[(2 * C::W + 4) * WSTR + p]);
+                    atomicAdd(tile + stride + n, xy * at((2 * C::W + 4) * WSTR + p));
         }
     }
     else if constexpr (C::W == 4)
     {
         int const b = lane >> 4, c = (lane & 15) >> 2;
-        double const yz = buf[(4 + b) * WSTR + p] * buf[(8 + c) * WSTR + p];
-        double const t  = yz * buf[(12 + m) * WSTR + p];
+        double const yz = at((4 + b) * WSTR + p) * at((8 + c) * WSTR + p);
+        double const t  = yz * at((12 + m) * WSTR + p);
         int const n     = node0 + b * p2 + c;
 #pragma unroll
         for (int r = 0; r < 4; ++r)
         {
-            double const x = buf[r * WSTR + p];
+            double const x = at(r * WSTR + p);
             atomicAdd(tile + slab * stride + n + r * p12, x * t);
             if constexpr (!RN)
                 if (m == 0)
-                    atomicAdd(tile + stride + n + r * p12, x * (yz * buf[16 * WSTR + p]));
+                    atomicAdd(tile + stride + n + r * p12, x * (yz * at(16 * WSTR + p)));
         }
     }
     else if (lane < 32)
     {
         int const a = lane >> 4, b = (lane >> 3) & 1, c = (lane >> 2) & 1;
-        double const xyz = buf[a * WSTR + p] * buf[(2 + b) * WSTR + p] * buf[(4 + c) * WSTR + p];
+        double const xyz = at(a * WSTR + p) * at((2 + b) * WSTR + p) * at((4 + c) * WSTR + p);
         int const n      = node0 + a * p12 + b * p2 + c;
-        atomicAdd(tile + slab * stride + n, xyz * buf[(6 + m) * WSTR + p]);
+        atomicAdd(tile + slab * stride + n, xyz * at((6 + m) * WSTR + p));
         if constexpr (!RN)
             if (m == 0)
-                atomicAdd(tile + stride + n, xyz * buf[10 * WSTR + p]);
+                atomicAdd(tile + stride + n, xyz * at(10 * WSTR + p));
     }
 }
 

@@ -217,23 +217,25 @@ void launchSegScatter(SegGeom const& sg, PView32 const& src, PView32 const& dst,
 void launchSegCopy(PView const& src, PView const& dst, unsigned long long n, int dim, hipStream_t s);
 void launchSegCopy(PView32 const& src, PView32 const& dst, unsigned long long n, int dim, hipStream_t s);
 // mixed-precision push + gather + deposit over cell-segmented FP32 storage, in place (A.pushOn 0:
-// deposit only); the LDS tile of segTileShape32
+// deposit only): dense storage by the cell-grouped push, the LDS tile of cellTileShape (4 slabs),
+// other storage one workgroup per work item, the LDS tile of segTileShape32
 void launchPush32(PushArgs const& A, PView32 const& v, hipStream_t s);
 TileSpec segTileShape32(int dim, int order, SegGeom const& sg);
 // the same over brick-ordered linear FP32 storage (3D), in place; the LDS tile of brickTileShape32
 void launchPush32Linear(PushArgs const& A, PView32 const& v, hipStream_t s);
 TileSpec brickTileShape32(int order);
+// whether segmented storage is dense (particles row by row in cell order) and pushed cell by cell: all
+// of 2D and 3D but FP32 in 2D at orders 1 and 2, where one particle per lane into the tile is faster
+// (256x128 cells, 100 per cell, per PPC step: 0.217 and 0.259 ms against 0.234 and 0.280; at order 3,
+// 190x150 cells, 64 per cell, 0.287 against 0.235)
+inline bool cellGrouped(int dim, int order, bool fp32) { return dim == 3 || (dim == 2 && (!fp32 || order == 3)); }
 // push + gather + deposit (A.pushOn 0: deposit only) over dense cell-segmented 2D or 3D storage, in
 // place, one workgroup per work item (2D) or A.split per segment (3D), the particles of a cell
 // deposited together; the LDS tile of cellTileShape (5 slabs, 4 with A.rhoFromN)
 void launchPushCell(PushArgs const& A, PView const& in, hipStream_t s);
-TileSpec cellTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad);
+TileSpec cellTileShape(bool fp32, int dim, int order, SegGeom const& sg, int slabs, int pad);
 // workgroups per segment (A.split) for an array of `slots` slots
-unsigned int cellSplit(int order, SegGeom const& sg, unsigned long long slots);
-// mixed-precision push + gather + deposit over cell-segmented storage with one workgroup per segment
-// and all its rows, in place (3D); grid nsegs + 1; the LDS tile of segwgTileShape (4 slabs)
-void launchPush32SegWG(PushArgs const& A, PView32 const& v, hipStream_t s);
-TileSpec segwgTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad);
+unsigned int cellSplit(bool fp32, int order, SegGeom const& sg, unsigned long long slots);
 // BorisPusher::move in place over A.n slots with box-list selectors; status[i] gets the slot's
 // fate for the partition (0 both selectors, 1 first only, 2 neither, 3 empty slot)
 void launchMove(PushArgs const& A, PView const& v, SelBoxes const& first, SelBoxes const& second,

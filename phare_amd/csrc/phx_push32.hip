@@ -17,10 +17,12 @@
 //    is several times faster than an FP32 one (ds_add_f64 / ds_add_f32), and FP64 sums of FP32
 //    terms are more accurate than compensated FP32 sums (a TwoSum-compensated FP32 tile, whose
 //    adds must return the old value, measured slower still);
+//  - in 3D, and in 2D at order 3, the particles of a cell deposit together (k_push_cell): their FP32
+//    weights and values multiplied and summed in FP64;
 //  - E and B are gathered from an FP32 copy of the averaged set (written beside it by the average
 //    kernel) and interpolated in FP32; in 1D and 2D a component's stencil values are loaded
 //    together before the sums, so that their loads are in flight at once.
-#include "phx_push_common.hpp"
+#include "phx_cell_push.hpp"
 
 namespace phx
 {
@@ -30,54 +32,13 @@ using pc::BLOCK;
 using pc::inBox;
 using pc::inNLGB;
 using pc::LANES;
-using pc::NW;
-
-// B-spline weights at u = np - start (u in [0, O+1)); the products of interpolator.hpp:54-125
-// written in u: order 2 uses 1 - u for (start + 1 - np), order 3 uses -u for (start - np)
-template<int O>
-__device__ __forceinline__ void bspline32(float u, float* w)
-{
-    if constexpr (O == 1)
-    {
-        w[1] = u;
-        w[0] = 1.f - u;
-    }
-    else if constexpr (O == 2)
-    {
-        float const d  = 1.f - u;
-        float const c1 = .5f + d;
-        float const c3 = .5f - d;
-        w[0]           = .5f * c1 * c1;
-        w[1]           = .75f - d * d;
-        w[2]           = .5f * c3 * c3;
-    }
-    else
-    {
-        float const index = -u;
-        float const c1    = 1.f + .5f * index;
-        float const c2    = index + 1.f;
-        float const c3    = index + 2.f;
-        float const c4    = 1.f - .5f * (index + 3.f);
-        float const c2s   = c2 * c2;
-        float const c3s   = c3 * c3;
-        w[0]              = (4.f / 3.f) * c1 * c1 * c1;
-        w[1]              = (2.f / 3.f) - c2s - .5f * c2s * c2;
-        w[2]              = (2.f / 3.f) - c3s + .5f * c3s * c3;
-        w[3]              = (4.f / 3.f) * c4 * c4 * c4;
-    }
-}
 
 // start index and weights of one direction (interpolator.hpp:379-406): np - start is the start
 // shift plus delta (less one half for the dual centering)
 template<int O>
 __device__ __forceinline__ int indexAndWeights32(int c, int icl, float delta, float* w)
 {
-    int const sh = startShift<O>(c, static_cast<double>(delta));
-    float u      = static_cast<float>(sh) + delta;
-    if (c == CD)
-        u -= .5f;
-    bspline32<O>(u, w);
-    return icl - sh;
+    return icl - pc::splineStencil<O>(c, delta, w);
 }
 
 template<int D, int O>
@@ -460,13 +421,6 @@ __device__ __forceinline__ void winAdd(Win32<D, O>& A, Dep32<D, O> const& dd, in
     }
 }
 
-// the window variant exists where its accumulators fit the registers: 1D, 2D, and 3D at order 1
-template<int D, int O>
-constexpr bool winFits()
-{
-    return D < 3 || O == 1;
-}
-
 // per-launch constants in FP32
 struct Push32
 {
@@ -760,13 +714,10 @@ void k_push_seg32(PushArgs A, PView32 v)
 template<int D, int O>
 static void launchPush32T(PushArgs const& A, PView32 const& v, hipStream_t s)
 {
-    if constexpr (winFits<D, O>())
-        if (A.depositWindow)
-        {
-            k_push_seg32<D, O, true><<<A.st.itemsCap, pc::SEG_BLOCK, A.tile.bytes, s>>>(A, v);
-            return;
-        }
-    k_push_seg32<D, O, false><<<A.st.itemsCap, pc::SEG_BLOCK, A.tile.bytes, s>>>(A, v);
+    if (A.depositWindow)
+        k_push_seg32<D, O, true><<<A.st.itemsCap, pc::SEG_BLOCK, A.tile.bytes, s>>>(A, v);
+    else
+        k_push_seg32<D, O, false><<<A.st.itemsCap, pc::SEG_BLOCK, A.tile.bytes, s>>>(A, v);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -828,104 +779,65 @@ __global__ __launch_bounds__(BLOCK) void k_push32_lin(PushArgs A, PView32 v)
 }
 } // namespace
 
-// the same over cell-segmented FP32 storage, one workgroup per segment with all its rows (the
-// staged 3D path's layout after its sorts)
-template<int D, int O>
-__global__ __launch_bounds__(BLOCK) void k_push32_segwg(PushArgs A, PView32 v)
+// the mixed-precision family of the cell-grouped push: the particles, their move, the stage of E and B,
+// the weights and values stay FP32, the products and sums of the deposit are FP64. 64^3 cells, order 2,
+// 64 per cell, per PPC step: 1.73 ms after a sort, 2.37 with one particle per lane added word by word
+// into the tile; with FP64 hand-over buffers two workgroups of 512 fit a CU where now three of 256 do: 2.62
+struct Fp32
 {
-    extern __shared__ double lds32[];
-    if (A.G.stopped())
-        return;
-    Geom const& G          = A.G;
-    unsigned int const seg = pc::xcdItem(blockIdx.x, gridDim.x);
-    int const t            = threadIdx.x;
-    int const lane         = t & 63;
-    unsigned long long const off = A.st.off[seg];
-    unsigned int const R         = A.st.rows[seg];
-    for (int x = t; x < 4 * A.tile.stride; x += BLOCK)
-        lds32[x] = 0.;
-    Tile32 T;
-    T.lds    = lds32;
-    T.stride = A.tile.stride;
+    using Real = float;
+    // half a step of the position without a branch; false when it moves more than two cells
+    template<int D>
+    static __device__ __forceinline__ bool halfStep(int* cell, float* delta, float const* v, float const* hdtdx)
+    {
+        bool ok = true;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-    {
-        T.ext[d]   = A.tile.ext[d];
-        T.pitch[d] = A.tile.pitch[d];
-        T.org[d]   = 0;
+        for (int d = 0; d < D; ++d)
+        {
+            float const dl = delta[d] + hdtdx[d] * v[d];
+            ok             = ok & !(fabsf(dl) > 2.f);
+            int const ic   = static_cast<int>(floorf(dl));
+            float const nd = dl - static_cast<float>(ic);
+            bool const up  = nd >= 1.f; // a tiny negative step (advancePosition32)
+            delta[d]       = up ? nd - 1.f : nd;
+            cell[d] += up ? ic + 1 : ic;
+        }
+        return ok;
     }
-    pc::segTileOrigin<D>(G, A.sg, A.tile, seg, T.org);
-    Push32 K;
+    static __device__ __forceinline__ float fma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+    static __device__ __forceinline__ float const* field(PushArgs const& A, int f) { return A.em32[f]; }
+    static __device__ __forceinline__ void accelerate(float* v, float const* E, float const* B, double q,
+                                                      double dto2m)
+    {
+        borisAccelerate32(v, E, B, static_cast<float>(q * dto2m));
+    }
+    template<int D, int O, bool RN>
+    static __device__ __forceinline__ void pushOne(PushArgs const& A, PView32 const& v, unsigned long long i,
+                                                   pc::TileView const& V)
+    {
+        Tile32 T;
+        T.lds    = V.lds;
+        T.stride = V.stride;
+        Push32 K;
 #pragma unroll
-    for (int d = 0; d < 3; ++d)
-        K.hdtdx[d] = static_cast<float>(A.hdtdx[d]);
-    K.coef1 = static_cast<float>(A.charge * A.dto2m);
-    K.coef  = static_cast<float>(A.coef);
-    __syncthreads();
-    Win32<D, O> win;
-#pragma unroll 1
-    for (unsigned int r = static_cast<unsigned int>(t >> 6); r < R; r += NW)
-        pushSlot32<D, O, false>(A, K, v, off + static_cast<unsigned long long>(r) * LANES + lane, T, win);
-    __syncthreads();
-    flushTile32<D, BLOCK>(A, T);
-}
-
-// tile of the workgroup-per-segment push: the largest segment plus the stencil and one cell of
-// motion below (2 nodes) and above (order + 2 nodes), `slabs` moment slabs, the pitches of
-// dimensions 1 and 2 padded to a multiple of `pad` nodes
-TileSpec segwgTileShape(int dim, int order, SegGeom const& sg, int slabs, int pad)
-{
-    TileSpec T{};
-    T.copies = 1;
-    for (int d = 0; d < 3; ++d)
-    {
-        T.lo[d]    = d < dim ? 2 : 0;
-        T.ext[d]   = d < dim ? sg.maxSeg[d] + 2 + order + 2 : 1;
-        T.pitch[d] = T.ext[d];
-    }
-    auto size = [&]() {
-        T.nodes  = T.ext[0] * T.pitch[1] * T.pitch[2];
-        T.stride = (T.nodes + 15) / 16 * 16;
-        T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride);
-    };
-    if (dim == 3 && pad > 1)
-    {
-        // pitches of dimensions 1 and 2 padded to a multiple of pad nodes (the padding nodes are
-        // never deposited into: the flush skips them as zeros); dropped if the tile outgrows LDS
-        for (int d = 1; d < 3; ++d)
-            T.pitch[d] = (T.ext[d] + pad - 1) / pad * pad;
-        size();
-        if (T.bytes > pc::TILE_BYTES_MAX)
-            for (int d = 1; d < 3; ++d)
-                T.pitch[d] = T.ext[d];
-    }
-    size();
-    if (T.bytes > pc::TILE_BYTES_MAX)
-    {
-        // no room: every deposit goes straight to HBM
         for (int d = 0; d < 3; ++d)
         {
-            T.ext[d]   = 1;
-            T.pitch[d] = 1;
+            T.org[d]   = V.org[d];
+            T.ext[d]   = V.ext[d];
+            T.pitch[d] = V.pitch[d];
+            K.hdtdx[d] = static_cast<float>(A.hdtdx[d]);
         }
-        T.lo[0]  = -0x10000000;
-        T.nodes  = 1;
-        T.stride = 16;
-        T.bytes  = static_cast<unsigned int>(8 * slabs * T.stride);
+        K.coef1 = static_cast<float>(A.charge * A.dto2m);
+        K.coef  = static_cast<float>(A.coef);
+        Win32<D, O> win;
+        pushSlot32<D, O, false>(A, K, v, i, T, win);
     }
-    return T;
-}
+};
 
-void launchPush32SegWG(PushArgs const& A, PView32 const& v, hipStream_t s)
+template<int D, int O>
+static void launchPushCell32(PushArgs const& A, PView32 const& v, hipStream_t s)
 {
-    unsigned int const grid = static_cast<unsigned int>(A.sg.nsegs) + 1u;
-    switch (A.G.dim * 10 + A.G.order)
-    {
-        case 31: k_push32_segwg<3, 1><<<grid, BLOCK, A.tile.bytes, s>>>(A, v); break;
-        case 32: k_push32_segwg<3, 2><<<grid, BLOCK, A.tile.bytes, s>>>(A, v); break;
-        case 33: k_push32_segwg<3, 3><<<grid, BLOCK, A.tile.bytes, s>>>(A, v); break;
-        default: break;
-    }
+    A.tile.emFix ? launchPushCellT<Fp32, D, O, true, true>(A, v, s) : launchPushCellT<Fp32, D, O, true, false>(A, v, s);
 }
 
 TileSpec brickTileShape32(int order)
@@ -967,10 +879,10 @@ void launchPush32(PushArgs const& A, PView32 const& v, hipStream_t s)
         case 13: launchPush32T<1, 3>(A, v, s); break;
         case 21: launchPush32T<2, 1>(A, v, s); break;
         case 22: launchPush32T<2, 2>(A, v, s); break;
-        case 23: launchPush32T<2, 3>(A, v, s); break;
-        case 31: launchPush32T<3, 1>(A, v, s); break;
-        case 32: launchPush32T<3, 2>(A, v, s); break;
-        case 33: launchPush32T<3, 3>(A, v, s); break;
+        case 23: launchPushCell32<2, 3>(A, v, s); break;
+        case 31: launchPushCell32<3, 1>(A, v, s); break;
+        case 32: launchPushCell32<3, 2>(A, v, s); break;
+        case 33: launchPushCell32<3, 3>(A, v, s); break;
     }
 }
 
