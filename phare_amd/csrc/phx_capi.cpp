@@ -55,10 +55,19 @@ namespace
 
 // particle arrays of one kind: int32 cells, and delta, velocity, weight (and charge) as FP64
 // (real = 8) or, in the mixed-precision family, FP32 without a charge array (real = 4)
+// share of a compacted array's particles outside their segments from which the linear push is the faster
+// one again (2D, 25 to 60 per cell, a pair of pushes with its compactions: 0.25 ms with few outside, 0.34
+// at a tenth, about 1 ms at a quarter; the linear push 0.84 to 1.0)
+constexpr double PACK_LONE = 0.25;
+
 struct Store
 {
     size_t n = 0, cap = 0;
     bool seg = false; // cell-segmented by the sort (the population's segment tables describe it)
+    // the segments of the last sort without their padding, in order (after a compaction), whatever was
+    // appended behind them: the population's st.off still says where they start. A hint: any content is
+    // pushed right, particles far from their segment slower
+    bool packed = false;
     int real = 8;
     int32_t* ic[3] = {nullptr, nullptr, nullptr};
     void* de[3]    = {nullptr, nullptr, nullptr};
@@ -284,7 +293,8 @@ phx_status storeReserve(phx_ctx* c, Store& s, size_t need)
             PHX_HIP(c, hipMemcpyAsync(ns.q, s.q, s.n * r, hipMemcpyDeviceToDevice, c->stream));
         PHX_HIP(c, hipStreamSynchronize(c->stream));
     }
-    ns.n = s.n;
+    ns.n      = s.n;
+    ns.packed = s.packed;
     storeFree(c, s);
     s = ns;
     return PHX_OK;
@@ -436,6 +446,8 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
     A.n            = c->pops[pop].arr[kind].n;
     A.err          = c->err;
     A.status       = nullptr;
+    A.lone         = nullptr;
+    A.packed       = 0;
     A.dropped      = c->dropped;
     A.pushOn       = 1;
     A.charge       = c->pops[pop].charge;
@@ -448,14 +460,21 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
     Pop const& P   = c->pops[pop];
     Store const& s = P.arr[kind];
     // the cell-grouped push, which gives every slot its fate
-    if (c->sg.dense && kind == KIND_DOMAIN && s.seg)
+    if (c->sg.dense && kind == KIND_DOMAIN && (s.seg || (s.packed && s.n < 0xFFFFFFFFull)))
     {
         A.segOn       = 1;
         A.sg          = c->sg;
         A.st          = P.seg;
+        A.packed      = s.seg ? 0 : 1;
         A.st.itemsCap = segItemsCap(c->sg, P.seg, s.cap);
         A.rhoFromN    = mixed(c) || (P.hasCharge && P.uniformCharge) ? 1 : 0;
-        A.split       = cellSplit(mixed(c), c->cfg.interp_order, c->sg, s.n);
+        if (c->cfg.dim == 3)
+            A.split = cellSplit(mixed(c), c->cfg.interp_order, c->sg, s.n);
+        else if (A.packed)
+        {
+            unsigned long long const item = 64ull * itemRowsFor(c->sg, s.n, c->tuning.rows_per_item) * c->sg.nsegs;
+            A.split                       = static_cast<unsigned int>((s.n + item - 1) / item);
+        }
         A.tile = cellTileShape(mixed(c), c->cfg.dim, c->cfg.interp_order, c->sg, A.rhoFromN ? 4 : 5, c->tuning.tile_row_pad);
         noteTileFallback(c, A.tile);
         return A;
@@ -963,6 +982,7 @@ phx_status upload(phx_ctx* c, Pop& P, Store& s, size_t n, int32_t const* ic, dou
     }
     PHX_TRY(storeReserve(c, s, offset + n));
     s.seg = false;
+    s.packed = false;
     // the copies below run on the null stream, which does not wait for the context's
     // non-blocking stream: nothing queued there may still use the array
     PHX_HIP(c, hipStreamSynchronize(c->stream));
@@ -1159,15 +1179,17 @@ phx_status sortDomain(phx_ctx* c)
             else
                 launchSegCopy(buf.view(), dom.view(), slots, c->cfg.dim, c->stream);
             PHX_TRY(checkLaunch(c, "particle sort (copy)"));
-            dom.n   = slots;
-            dom.seg = true;
+            dom.n      = slots;
+            dom.seg    = true;
+            dom.packed = false;
             continue;
         }
         buf.n   = slots;
         buf.seg = true;
         std::swap(dom, buf);
-        buf.seg = false;
-        buf.n   = 0;
+        buf.seg    = false;
+        buf.packed = false;
+        buf.n      = 0;
         if (buf.cap < dom.cap)
         {
             // the two storages the sorts alternate between keep one capacity: no reallocation
@@ -1220,6 +1242,7 @@ std::vector<unsigned long long> storageKey(phx_ctx const* c)
             k.push_back(reinterpret_cast<unsigned long long>(s.w));
             k.push_back(s.cap);
             k.push_back(s.seg ? ~0ull : s.n);
+            k.push_back(s.packed ? 1ull : 0ull);
         }
     }
     return k;
@@ -1289,7 +1312,10 @@ phx_status buildPatchTable(phx_ctx* c, int const* plo, int const* phi, int np)
     S.dim         = D;
     S.npatch      = np;
     for (Pop& P : c->pops)
-        P.itemsFor = 0;
+    {
+        P.itemsFor               = 0;
+        P.arr[PHX_DOMAIN].packed = false;
+    }
     S.rowPad      = c->tuning.tile_row_pad;
     S.dense       = cellGrouped(D, c->cfg.interp_order, mixed(c)) ? 1 : 0;
     size_t boxCells = 1;
@@ -1586,6 +1612,8 @@ phx_status createLevel(phx_config const* cfg, phx_patch const* patch, int const*
         s = devAlloc(c, (void**)&c->dropped, 64);
     if (s == PHX_OK)
         s = devAlloc(c, (void**)&c->tot, 64);
+    if (s == PHX_OK && hipMemset(c->tot, 0, 64) != hipSuccess)
+        s = fail(c, PHX_ERR_HIP, "hipMemset");
     if (s != PHX_OK)
     {
         phx_destroy(c);
@@ -2120,26 +2148,37 @@ phx_status phx_update_populations(phx_ctx* c, int em_set, double dt, int mode)
         // domain: push in place with a fate per particle, then split keep / leave
         PushArgs A = pushArgs(c, p, KIND_DOMAIN, mode, em_set, dt, false);
         A.status   = c->status;
+        A.lone     = c->tot + 1;
         launchPush(A, dom.view(), dom.view(), c->stream);
         PHX_TRY(checkLaunch(c, "push"));
         PHX_TRY(checkDeviceError(c));
         // leavers appended to patchGhost (updateAndDepositAll_ :248-254)
-        unsigned long long got = 0;
+        unsigned long long got = 0, lone[2] = {0, 0};
         launchCompact(dom.view(), pg.view(), c->status, nd, ST_LEAVE, c->blockCnt, c->tot, pg.n, D,
                       noWrap, c->stream);
         PHX_HIP(c, hipStreamSynchronize(c->stream));
-        PHX_HIP(c, hipMemcpy(&got, c->tot, 8, hipMemcpyDeviceToHost));
-        pg.n += got;
+        PHX_HIP(c, hipMemcpy(lone, c->tot, 16, hipMemcpyDeviceToHost));
+        pg.n += nd ? lone[0] : 0;
         // kept domain particles -> scratch, then swap (erase of the leavers, :273)
         launchCompact(dom.view(), c->scratch.view(), c->status, nd, ST_KEEP, c->blockCnt, c->tot, 0,
                       D, noWrap, c->stream);
         PHX_HIP(c, hipStreamSynchronize(c->stream));
         PHX_HIP(c, hipMemcpy(&got, c->tot, 8, hipMemcpyDeviceToHost));
+        // the push of the calls to come still finds the segments of the last sort, while few particles
+        // have left them
+        bool const packed = c->sg.dense && (dom.seg || dom.packed) && static_cast<double>(lone[1]) < PACK_LONE * nd;
+        if (lone[1])
+            PHX_HIP(c, hipMemsetAsync(c->tot + 1, 0, 8, c->stream));
+        if (packed)
+            launchPackOffsets(c->status, nd, c->blockCnt, c->tot, P.seg.off, static_cast<unsigned int>(c->sg.nsegs) + 1u,
+                              c->stream);
         std::swap(dom, c->scratch);
-        dom.n          = got;
+        dom.n          = nd ? got : 0;
         dom.seg        = false;
+        dom.packed     = packed;
         c->scratch.n   = 0;
         c->scratch.seg = false;
+        c->scratch.packed = false;
         if (nl)
         {
             // level ghosts (:275-288): pushed with inGhostBox / inGhostLayer selection; those that
@@ -2215,6 +2254,7 @@ phx_status phx_push(phx_ctx* c, int pop, int kind, int em_set, double dt, int n_
     std::swap(s, c->scratch);
     s.n            = off;
     s.seg          = false;
+    s.packed = false;
     c->scratch.n   = 0;
     c->scratch.seg = false;
     counts[0]      = got[0];
@@ -2687,6 +2727,7 @@ phx_status phx_fill_ion_ghost_particles(phx_ctx* c)
         Store& dom = c->pops[p].arr[PHX_DOMAIN];
         if (c->patch.periodic && pg.n)
         {
+            bool const packed = c->sg.dense && !mixed(c) && (dom.seg || dom.packed);
             PHX_TRY(storeReserve(c, dom, dom.n + pg.n));
             PHX_TRY(scratchReserve(c, pg.n));
             PHX_HIP(c, hipMemsetAsync(c->status, ST_KEEP, pg.n, c->stream));
@@ -2701,7 +2742,8 @@ phx_status phx_fill_ion_ghost_particles(phx_ctx* c)
             launchCompact(pg.view(), dom.view(), c->status, pg.n, ST_KEEP, c->blockCnt, c->tot, dom.n,
                           D, wrap, c->stream);
             dom.n += pg.n;
-            dom.seg = false;
+            dom.seg    = false;
+            dom.packed = packed;
         }
         pg.n = 0;
     }

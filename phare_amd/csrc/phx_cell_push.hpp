@@ -282,8 +282,9 @@ __device__ __forceinline__ void gatherStaged(R const* em, int e1, int e2, int no
 // density out, its flush taking the charge times n.
 // ---------------------------------------------------------------------------------------------
 // X: the particle family (storage type, arithmetic of the move and the gather, the push of one particle
-// by itself). FIX: the stage has the pitches of the default segments (the stencils' offsets are then constants)
-template<class X, int D, int O, bool RN, bool FIX>
+// by itself). FIX: the stage has the pitches of the default segments (the stencils' offsets are then constants).
+// PACKED: the segments follow each other without padding, and linear slots behind them
+template<class X, int D, int O, bool RN, bool FIX, bool PACKED>
 __global__ __launch_bounds__((pc::CellCfg<X, D, O>::BLOCK)) __attribute__((amdgpu_waves_per_eu(pc::CellCfg<X, D, O>::WAVES)))
 void k_push_cell(pc::CellArgs<X> K)
 {
@@ -299,17 +300,40 @@ void k_push_cell(pc::CellArgs<X> K)
     double* const lds = cellLds;
     __shared__ unsigned int list[LIST];
     __shared__ unsigned int listed;
-    // 3D: split workgroups per segment; 2D: the work items of the sort (captured steps keep their
-    // grid while the sorts change the items)
-    unsigned int seg, rA, rB, nItems = 0;
-    if constexpr (D == 3)
+    // 3D and packed storage: split workgroups per segment; 2D: the work items of the sort (captured
+    // steps keep their grid while the sorts change the items). slots: the segment's, whole rows but in
+    // packed storage, whose segments follow each other without padding (the overflow segment takes what
+    // was appended since)
+    unsigned int seg, rA, rB, slots, nItems = 0;
+    unsigned long long off;
+    if (D == 3 || PACKED)
     {
-        unsigned int const item = pc::xcdItem(blockIdx.x, gridDim.x);
-        seg                     = item / K.A.split;
-        unsigned int const part = item - seg * K.A.split;
-        unsigned long long const R = K.A.st.rows[seg];
-        rA = static_cast<unsigned int>(R * part / K.A.split);
-        rB = static_cast<unsigned int>(R * (part + 1) / K.A.split);
+        nItems                  = gridDim.x;
+        if constexpr (D == 2)
+            ktBegin(K.A.kt);
+        unsigned int const nsegs = static_cast<unsigned int>(K.A.sg.nsegs);
+        unsigned int const base  = nsegs * K.A.split; // workgroups before the overflow segment's
+        unsigned int part = blockIdx.x - base, parts = gridDim.x - base;
+        seg = nsegs;
+        if (blockIdx.x < base)
+        {
+            unsigned int const item = xcdItem(blockIdx.x, base);
+            seg                     = item / K.A.split;
+            part                    = item - seg * K.A.split;
+            parts                   = K.A.split;
+        }
+        off = K.A.st.off[seg];
+        if (PACKED)
+        {
+            unsigned long long const end = seg < nsegs ? K.A.st.off[seg + 1] : K.A.n;
+            off   = min(off, K.A.n);
+            slots = static_cast<unsigned int>(max(min(end, K.A.n), off) - off);
+        }
+        else
+            slots = K.A.st.rows[seg] * LANES;
+        unsigned long long const rows = (static_cast<unsigned long long>(slots) + LANES - 1) / LANES;
+        rA = static_cast<unsigned int>(rows * part / parts);
+        rB = static_cast<unsigned int>(rows * (part + 1) / parts);
     }
     else
     {
@@ -320,13 +344,22 @@ void k_push_cell(pc::CellArgs<X> K)
         seg = K.A.st.items[2 * blockIdx.x];
         pc::itemRows(K.A.st.items[2 * blockIdx.x + 1], K.A.st.rows[seg],
                      K.A.st.rowsPerItem, rA, rB);
+        off   = K.A.st.off[seg];
+        slots = rB * LANES;
     }
+    // the same in every lane: scalar from here on
+    rA    = __builtin_amdgcn_readfirstlane(rA);
+    rB    = __builtin_amdgcn_readfirstlane(rB);
+    slots = __builtin_amdgcn_readfirstlane(slots);
+    off   = static_cast<unsigned int>(__builtin_amdgcn_readfirstlane(static_cast<unsigned int>(off)))
+          | static_cast<unsigned long long>(static_cast<unsigned int>(
+                __builtin_amdgcn_readfirstlane(static_cast<unsigned int>(off >> 32))))
+                << 32;
     if (rB > rA && !K.A.G.stopped())
     {
         unsigned int const rows = rB - rA;
         unsigned int const lane = threadIdx.x & 63u;
         unsigned int const wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-        unsigned long long const off = K.A.st.off[seg];
         constexpr int EX  = cellExt(D, O) | 1;
         int const e1      = D == 2 ? (FIX ? EX : K.A.tile.emExt[1] | 1) : (FIX ? cellExt(3, O) : K.A.tile.emExt[1]);
         int const e2      = D == 2 ? 1 : (FIX ? EX : K.A.tile.emExt[2] | 1);
@@ -380,7 +413,7 @@ void k_push_cell(pc::CellArgs<X> K)
             int cur = -1; // tile node of the accumulated window's origin
             Part<D, R> next;
             if (NEXT && r < rEnd)
-                loadRow<D, RN>(K.v, off + static_cast<unsigned long long>(r) * LANES, lane, next);
+                loadRow<D, RN>(K.v, off + static_cast<unsigned long long>(r) * LANES, PACKED ? min(lane, slots - 1 - r * LANES) : lane, next);
             for (; r < rEnd; ++r)
             {
                 // until the list might overflow (each wavefront that still finds room may add 64)
@@ -392,12 +425,13 @@ void k_push_cell(pc::CellArgs<X> K)
                 {
                     P = next;
                     if (r + 1 < rEnd)
-                        loadRow<D, RN>(K.v, row + LANES, lane, next); // in flight over this row's work
+                        loadRow<D, RN>(K.v, row + LANES, PACKED ? min(lane, slots - 1 - (r + 1) * LANES) : lane, next); // in flight over this row's work
                 }
                 else
-                    loadRow<D, RN>(K.v, row, lane, P);
+                    loadRow<D, RN>(K.v, row, PACKED ? min(lane, slots - 1 - r * LANES) : lane, P);
                 double const q  = RN ? charge : static_cast<double>(P.q);
-                bool const live = P.cell[0] != DEAD_CELL;
+                bool const mine = !PACKED || lane < slots - r * LANES;
+                bool const live = mine & (P.cell[0] != DEAD_CELL);
                 bool ok         = live;
                 if (push)
                 {
@@ -497,7 +531,7 @@ void k_push_cell(pc::CellArgs<X> K)
                             rowOf(K.v.v[d], row)[lane] = P.v[d];
                     }
                     uint8_t* const status = K.A.status;
-                    if (status && (ok || !live))
+                    if (status && mine && (ok || !live))
                         rowOf(status, row)[lane] = live ? ST_KEEP : ST_DROP;
                 }
             }
@@ -510,7 +544,11 @@ void k_push_cell(pc::CellArgs<X> K)
                 X::template pushOne<D, O, RN>(L.A, L.v, off + list[x], T);
             __syncthreads();
             if (threadIdx.x == 0)
+            {
+                if (n && cellArgs<X>().A.lone)
+                    atomicAdd(cellArgs<X>().A.lone, static_cast<unsigned long long>(n));
                 listed = 0u;
+            }
         } while (__syncthreads_or(r < rEnd));
         PushArgs const& A = cellArgs<X>().A;
         flushTile<D, RN, CB>(A.G, T, A.tile.nodes, A.mom, A.charge);
@@ -522,7 +560,7 @@ void k_push_cell(pc::CellArgs<X> K)
     }
 }
 
-template<class X, int D, int O, bool RN, bool FIX>
+template<class X, int D, int O, bool RN, bool FIX, bool PACKED = false>
 static void launchPushCellT(PushArgs const& A, PViewT<typename X::Real> const& in, hipStream_t s)
 {
     // more than 64 KB of dynamic LDS has to be allowed for the kernel (once per device)
@@ -533,11 +571,15 @@ static void launchPushCellT(PushArgs const& A, PViewT<typename X::Real> const& i
     {
         std::lock_guard<std::mutex> lock(mtx);
         if (!allowed[dev])
-            allowed[dev] = hipFuncSetAttribute(reinterpret_cast<void const*>(&k_push_cell<X, D, O, RN, FIX>),
+            allowed[dev] = hipFuncSetAttribute(reinterpret_cast<void const*>(&k_push_cell<X, D, O, RN, FIX, PACKED>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, pc::CELL_LDS_MAX)
                            == hipSuccess;
     }
-    unsigned int const grid = D == 3 ? (static_cast<unsigned int>(A.sg.nsegs) + 1u) * A.split : A.st.itemsCap;
-    k_push_cell<X, D, O, RN, FIX><<<grid, pc::CellCfg<X, D, O>::BLOCK, A.tile.bytes, s>>>(pc::CellArgs<X>{A, in});
+    // packed storage: what was appended behind the segments is spread over the GPU (in the workgroups of
+    // one segment, 1.9 million particles in 3D took 1.1 ms per pair of pushes after ten steps, 7.6 after
+    // eighty, of appended leavers)
+    unsigned int const overflow = PACKED ? static_cast<unsigned int>(pc::CUS) : A.split;
+    unsigned int const grid = D == 3 || PACKED ? static_cast<unsigned int>(A.sg.nsegs) * A.split + overflow : A.st.itemsCap;
+    k_push_cell<X, D, O, RN, FIX, PACKED><<<grid, pc::CellCfg<X, D, O>::BLOCK, A.tile.bytes, s>>>(pc::CellArgs<X>{A, in});
 }
 } // namespace phx

@@ -156,7 +156,9 @@ struct PushArgs
     uint8_t* status;
     unsigned int* dropped;
     int segOn; // the array is cell-segmented (sg, st valid)
-    unsigned int split; // 3D cell-grouped push: workgroups per segment
+    unsigned int split; // cell-grouped push in 3D or over packed storage: workgroups per segment
+    unsigned long long* lone; // cell-grouped push: where to count the particles pushed one by one (or null)
+    int packed; // the segments follow each other without padding: slots st.off[s] .. st.off[s + 1], the last up to n
     SegGeom sg;
     SegTables st;
     float const* em32[6]; // mixed-precision family: FP32 copy of the E/B set (Ex..Bz)
@@ -224,6 +226,10 @@ TileSpec segTileShape32(int dim, int order, SegGeom const& sg);
 // the same over brick-ordered linear FP32 storage (3D), in place; the LDS tile of brickTileShape32
 void launchPush32Linear(PushArgs const& A, PView32 const& v, hipStream_t s);
 TileSpec brickTileShape32(int order);
+// after the compaction of a segmented or packed array of n slots whose kept particles have status
+// ST_KEEP, before the next compaction: the m segment starts in `off` moved to the first kept slots
+void launchPackOffsets(uint8_t const* status, unsigned long long n, unsigned int const* blockCounts,
+                       unsigned long long const* total, unsigned long long* off, unsigned int m, hipStream_t s);
 // whether segmented storage is dense (particles row by row in cell order) and pushed cell by cell: all
 // of 2D and 3D but FP32 in 2D at orders 1 and 2, where one particle per lane into the tile is faster
 // (256x128 cells, 100 per cell, per PPC step: 0.217 and 0.259 ms against 0.234 and 0.280; at order 3,

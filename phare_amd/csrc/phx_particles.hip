@@ -14,6 +14,8 @@
 //    (and in FP32 in 2D at orders 1 and 2) they fill the rows column by column, so that each lane walks a run of cell-ordered
 //    particles and the lanes of one LDS deposit instruction add into distinct words, except where a
 //    crowded cell spans two lanes.
+//    A stable compaction (the drop-in updater's) leaves the segments behind each other without padding
+//    ("packed"), their starts moved with them, and the cell-grouped push goes on over them.
 // Either way a workgroup accumulates its moments in an LDS tile over its cells and flushes the
 // tile with one HBM atomic per touched node and moment; the gather reads E/B through the L1/L2
 // caches, leaving the LDS to the deposit (k_push_cell stages E/B in LDS). Particles whose stencil leaves the tile deposit
@@ -1471,6 +1473,37 @@ void launchCompact(PView const& src, PView const& dst, uint8_t const* status, un
                                           wrap);
 }
 
+// the start of every segment after a stable compaction: the kept slots before its old start, those of
+// the blocks before from the compaction's scan, the rest counted by a wavefront per segment
+__global__ __launch_bounds__(BLOCK) void k_pack_offsets(uint8_t const* __restrict__ status, unsigned long long n,
+                                                        unsigned int const* __restrict__ blockCounts,
+                                                        unsigned long long const* __restrict__ total,
+                                                        unsigned long long* __restrict__ off, unsigned int m)
+{
+    unsigned int const s    = blockIdx.x * (BLOCK / LANES) + threadIdx.x / LANES;
+    unsigned int const lane = threadIdx.x % LANES;
+    if (s >= m)
+        return;
+    unsigned long long const at = off[s];
+    unsigned long long to       = *total;
+    if (at < n)
+    {
+        unsigned long long const b = at / BLOCK;
+        to                         = blockCounts[b];
+        for (unsigned long long i = b * BLOCK; i < at; i += LANES)
+            to += static_cast<unsigned int>(__popcll(__ballot(i + lane < at && status[i + lane] == ST_KEEP)));
+    }
+    if (lane == 0)
+        off[s] = to;
+}
+
+void launchPackOffsets(uint8_t const* status, unsigned long long n, unsigned int const* blockCounts,
+                       unsigned long long const* total, unsigned long long* off, unsigned int m, hipStream_t s)
+{
+    constexpr unsigned int PER = BLOCK / LANES;
+    k_pack_offsets<<<(m + PER - 1) / PER, BLOCK, 0, s>>>(status, n, blockCounts, total, off, m);
+}
+
 // tile of the cell-grouped push: the window of every cell of the largest segment and of the cells
 // around it (one cell of motion), and the staged fields of the segment's gather
 TileSpec cellTileShape(bool fp32, int dim, int order, SegGeom const& sg, int slabs, int pad)
@@ -1550,7 +1583,10 @@ unsigned int cellSplit(bool fp32, int order, SegGeom const& sg, unsigned long lo
 template<int D, int O>
 static void launchPushCellO(PushArgs const& A, PView const& in, hipStream_t s)
 {
-    if (A.rhoFromN)
+    if (A.packed)
+        A.rhoFromN ? launchPushCellT<Fp64, D, O, true, false, true>(A, in, s)
+                   : launchPushCellT<Fp64, D, O, false, false, true>(A, in, s);
+    else if (A.rhoFromN)
         A.tile.emFix ? launchPushCellT<Fp64, D, O, true, true>(A, in, s) : launchPushCellT<Fp64, D, O, true, false>(A, in, s);
     else
         A.tile.emFix ? launchPushCellT<Fp64, D, O, false, true>(A, in, s) : launchPushCellT<Fp64, D, O, false, false>(A, in, s);
