@@ -39,8 +39,8 @@ HBM_PEAK_GBS = 8000.0
 # this script, FETCH_SIZE scaled x2 and WRITE_SIZE x1 by a 1 GiB device copy's readings; keyed by
 # workload and precision family (k_push_cell, in 2D mixed precision at orders 1 and 2
 # k_push_seg32)
-MEASURED_TRAFFIC = {("harris2d", "fp64"): 395.0e6, ("harris2d", "fp32"): 224.3e6,
-                    ("uniform3d", "fp64"): 19.41e9, ("uniform3d", "fp32"): 11.03e9}
+MEASURED_TRAFFIC = {("harris2d", "fp64"): 356.3e6, ("harris2d", "fp32"): 224.3e6,
+                    ("uniform3d", "fp64"): 18.58e9, ("uniform3d", "fp32"): 11.24e9}
 
 
 def _hip():
