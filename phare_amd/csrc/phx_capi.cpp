@@ -98,7 +98,7 @@ struct Pop
     double mass = 1.;
     double charge = 0.; // the particles' charge (mixed-precision family: one per population)
     bool hasCharge = false;
-    bool uniformCharge = true; // every particle uploaded so far has charge `charge`
+    bool uniformCharge = true; // every particle uploaded or refined into it so far has charge `charge`
     Store arr[5]; // domain, patch ghost, level ghost, level ghost old, level ghost new
     double* mom[5] = {};
     SegTables seg{}; // tables of the segmented domain array (items sized for itemsAlloc items)
@@ -2412,6 +2412,19 @@ phx_status phx_refine_particles(phx_ctx* fine, phx_ctx const* coarse, int pop, i
     if (got == 0)
         return PHX_OK;
     PHX_TRY(storeReserve(fine, dst, dst.n + got));
+    // the refined particles keep the coarse ones' charges: the segmented pushes may take one charge for
+    // the whole population only while both levels hold that one alone
+    Pop& P          = fine->pops[pop];
+    Pop const& from = coarse->pops[pop];
+    bool const one  = from.hasCharge && from.uniformCharge;
+    if (!P.hasCharge)
+    {
+        P.charge        = from.charge;
+        P.hasCharge     = true;
+        P.uniformCharge = one;
+    }
+    else
+        P.uniformCharge = P.uniformCharge && one && from.charge == P.charge;
     launchSplitWrite(src.view(), src.n, S, D, fine->blockCnt, dst.view(), dst.n, fine->stream);
     PHX_TRY(checkLaunch(fine, "phx_refine_particles (write)"));
     dst.n += got;
