@@ -2151,7 +2151,12 @@ phx_status phx_update_populations(phx_ctx* c, int em_set, double dt, int mode)
         A.lone     = c->tot + 1;
         launchPush(A, dom.view(), dom.view(), c->stream);
         PHX_TRY(checkLaunch(c, "push"));
-        PHX_TRY(checkDeviceError(c));
+        if (phx_status const pushed = checkDeviceError(c); pushed != PHX_OK)
+        {
+            // the next push counts from zero
+            PHX_HIP(c, hipMemsetAsync(A.lone, 0, 8, c->stream));
+            return pushed;
+        }
         // leavers appended to patchGhost (updateAndDepositAll_ :248-254)
         unsigned long long got = 0, lone[2] = {0, 0};
         launchCompact(dom.view(), pg.view(), c->status, nd, ST_LEAVE, c->blockCnt, c->tot, pg.n, D,
