@@ -419,6 +419,8 @@ void noteTileFallback(phx_ctx* c, TileSpec const& T)
                  c->tuning.segment_shape[0], c->tuning.segment_shape[1], c->tuning.segment_shape[2]);
 }
 
+bool sortedRarely(phx_ctx const* c) { return c->sortInterval == 0 || c->sortInterval > 20; }
+
 // arguments of the push kernel; `segOk` lets a cell-segmented domain array use the segmented kernel of
 // the 1D and mixed-precision levels (callers that need a fate for every slot, the compacting path, pass false)
 PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt, bool segOk)
@@ -448,6 +450,7 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
     A.status       = nullptr;
     A.lone         = nullptr;
     A.packed       = 0;
+    A.deposit      = DEP_GROUPS;
     A.dropped      = c->dropped;
     A.pushOn       = 1;
     A.charge       = c->pops[pop].charge;
@@ -472,9 +475,10 @@ PushArgs pushArgs(phx_ctx* c, int pop, int kind, int mode, int emSet, double dt,
             A.split = cellSplit(mixed(c), c->cfg.interp_order, c->sg, s.n);
         else if (A.packed)
         {
-            unsigned long long const item = 64ull * itemRowsFor(c->sg, s.n, c->tuning.rows_per_item) * c->sg.nsegs;
+            unsigned long long const item = 64ull * itemRowsFor(c->sg, s.n, c->tuning.rows_per_item, ITEM_LEAST_PACKED) * c->sg.nsegs;
             A.split                       = static_cast<unsigned int>((s.n + item - 1) / item);
         }
+        A.deposit = cellDeposit(c->cfg.dim, c->cfg.interp_order, P.seg.sparse, A.packed || sortedRarely(c));
         A.tile = cellTileShape(mixed(c), c->cfg.dim, c->cfg.interp_order, c->sg, A.rhoFromN ? 4 : 5, c->tuning.tile_row_pad);
         noteTileFallback(c, A.tile);
         return A;
@@ -1127,7 +1131,8 @@ phx_status sortDomain(phx_ctx* c)
         if (!dom.seg || P.itemsFor == 0 || dom.n > 2 * P.itemsFor || 2 * dom.n < P.itemsFor)
         {
             P.seg.rowsPerItem = mixed(c) && !c->sg.dense ? static_cast<unsigned int>(c->tuning.rows_per_item)
-                                         : itemRowsFor(c->sg, dom.n, c->tuning.rows_per_item);
+                                         : itemRowsFor(c->sg, dom.n, c->tuning.rows_per_item, ITEM_LEAST);
+            P.seg.sparse      = cellSparse(c->cfg.dim, c->cfg.interp_order, c->sg, dom.n);
             P.itemsFor        = std::max<size_t>(dom.n, 1);
         }
         if (mixed(c))
@@ -1222,11 +1227,13 @@ phx_status sortIfLinear(phx_ctx* c)
 std::vector<unsigned long long> storageKey(phx_ctx const* c)
 {
     std::vector<unsigned long long> k;
+    k.push_back(sortedRarely(c) ? 1ull : 0ull);
     for (int p = 0; p < c->cfg.n_pop; ++p)
     {
         // the segment tables a segmented push reads (reallocated when the storage grows)
         k.push_back(reinterpret_cast<unsigned long long>(c->pops[p].seg.items));
         k.push_back(c->pops[p].seg.rowsPerItem);
+        k.push_back(c->pops[p].seg.sparse ? 1ull : 0ull);
         // the population's charge, which the push takes as an argument when it is uniform
         double const q = c->pops[p].charge;
         unsigned long long qb;

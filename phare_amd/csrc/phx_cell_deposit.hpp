@@ -414,6 +414,96 @@ __device__ __forceinline__ void cellAddOne(R const* buf, int p, double* tile, in
     }
 }
 
+// a and b turned left by `by` places (N = 2 or 4)
+template<int N, class A>
+__device__ __forceinline__ void turn(A* a, int* b, int by)
+{
+#pragma unroll
+    for (int s = 1; s < N; s *= 2)
+    {
+        bool const on = (by & s) != 0;
+        A x[N];
+        int y[N];
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+        {
+            x[i] = on ? a[(i + s) % N] : a[i];
+            y[i] = on ? b[(i + s) % N] : b[i];
+        }
+#pragma unroll
+        for (int i = 0; i < N; ++i)
+        {
+            a[i] = x[i];
+            b[i] = y[i];
+        }
+    }
+}
+
+// the particles with `ok` added to the LDS tile, each by its own lane; node0: the tile node of the
+// origin of its cell's window (2D). Neighbouring lanes, which hold particles of one cell, start at
+// different moments and nodes of the stencil
+template<int O, bool RN, bool TURN, class R>
+__device__ __forceinline__ void cellAddLanes(bool ok, R const* delta, R weight, double q, R const* v, double coef,
+                                             double* tile, int stride, int node0, int p12, int p2)
+{
+    if (!ok)
+        return;
+    int const lane = static_cast<int>(threadIdx.x & 63u);
+    R w[2][O + 1];
+    double val[4];
+    int low[2];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) // order 2: the stencil leaves the window's first or last node out
+        low[d] = splineStencil<O>(CP, delta[d], w[d]) == 0 && O == 2 ? 1 : 0;
+    val[0] = weight * static_cast<R>(coef);
+#pragma unroll
+    for (int m = 0; m < 3; ++m)
+        val[1 + m] = v[m] * weight * static_cast<R>(coef);
+    double const rho = q * weight * coef;
+    node0 += (low[0] ? p12 : 0) + (low[1] ? p2 : 0);
+    if constexpr (TURN && O == 1)
+    {
+        int x[2] = {0, p12}, y[2] = {0, p2}, slab[4] = {0, stride, 2 * stride, 3 * stride};
+        if constexpr (!RN)
+            for (int m = 1; m < 4; ++m)
+                slab[m] += stride;
+        turn<4>(val, slab, lane & 3);
+        turn<2>(w[0], x, (lane >> 2) & 1);
+        turn<2>(w[1], y, (lane >> 3) & 1);
+#pragma unroll
+        for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+            {
+                double const xy = static_cast<double>(w[0][a]) * static_cast<double>(w[1][b]);
+                double* const n = tile + node0 + x[a] + y[b];
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    atomicAdd(n + slab[m], xy * val[m]);
+                if constexpr (!RN)
+                    atomicAdd(n + stride, xy * rho);
+            }
+    }
+    else
+    {
+        // the nodes' distances anew for every row: kept over the rows they took the push's registers
+        asm volatile("" : "+s"(stride), "+s"(p12), "+s"(p2));
+#pragma unroll
+        for (int a = 0; a <= O; ++a)
+#pragma unroll
+            for (int b = 0; b <= O; ++b)
+            {
+                double const xy = static_cast<double>(w[0][a]) * static_cast<double>(w[1][b]);
+                double* const n = tile + node0 + a * p12 + b * p2;
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+                    atomicAdd(n + (RN || m == 0 ? m : m + 1) * stride, xy * val[m]);
+                if constexpr (!RN)
+                    atomicAdd(n + stride, xy * rho);
+            }
+    }
+}
+
 // add the window to the LDS tile: node0 is the tile node of the window's origin, p12 and p2 the
 // node distances along the first two directions, slab m of the tile the moments in the order n, (rho,) Fx, Fy, Fz
 template<int D, int O, bool RN>

@@ -283,8 +283,9 @@ __device__ __forceinline__ void gatherStaged(R const* em, int e1, int e2, int no
 // ---------------------------------------------------------------------------------------------
 // X: the particle family (storage type, arithmetic of the move and the gather, the push of one particle
 // by itself). FIX: the stage has the pitches of the default segments (the stencils' offsets are then constants).
-// PACKED: the segments follow each other without padding, and linear slots behind them
-template<class X, int D, int O, bool RN, bool FIX, bool PACKED>
+// PACKED: the segments follow each other without padding, and linear slots behind them. DEP: how
+// a row's particles deposit (cellDeposit)
+template<class X, int D, int O, bool RN, bool FIX, bool PACKED, int DEP>
 __global__ __launch_bounds__((pc::CellCfg<X, D, O>::BLOCK)) __attribute__((amdgpu_waves_per_eu(pc::CellCfg<X, D, O>::WAVES)))
 void k_push_cell(pc::CellArgs<X> K)
 {
@@ -377,6 +378,10 @@ void k_push_cell(pc::CellArgs<X> K)
             T.org[d] = __builtin_amdgcn_readfirstlane(T.org[d]); // the same in every lane: scalar from here on
         int const p2 = T.pitch[2], p12 = T.pitch[1] * T.pitch[2];
         bool const push   = K.A.pushOn;
+        // read at run time where the groups' code is kept beside (orders 2 and 3): without it the constants of
+        // the one-by-one push move out of the loop over the rows and spill (190x150 cells, order 2, one particle per
+        // cell: 92 us per PPC step, 82 with it; order 1: 88 and 87)
+        bool const lanes  = DEP == DEP_LANES && (O == 1 || K.A.deposit);
         bool const writes = push && K.A.mode == MODE_ALL;
         // per direction: AMR cell of the deposit tile's and of the stage's first cell, and the number
         // of cells whose windows (stencils) they hold; the stage's cells are clipped to those whose
@@ -468,11 +473,12 @@ void k_push_cell(pc::CellArgs<X> K)
                 for (int d = 0; d < 3; ++d)
                     ok = ok & __builtin_isfinite(P.v[d] * P.w * static_cast<R>(coef));
                 key = ok ? key : -1;
+                unsigned long long strays = 0; // DEP_FEW: the particles of groups below CELL_MOVE
                 // the half rows in turn: first the accumulated window's cell, then every other cell
 #pragma unroll
                 for (int half = 0; half < 2; ++half)
                 {
-                    unsigned int rest = static_cast<unsigned int>(__ballot(ok) >> (32 * half));
+                    unsigned int rest = lanes ? 0u : static_cast<unsigned int>(__ballot(ok) >> (32 * half));
                     if (rest == 0u)
                         continue;
                     pc::cellStage<D, O, RN>(buf, half, ok, P.delta, P.w, q, P.v, coef);
@@ -480,6 +486,7 @@ void k_push_cell(pc::CellArgs<X> K)
                     if (m)
                         pc::cellAdd<D, O, RN>(buf, m, acc);
                     rest &= ~m;
+                    unsigned int few = 0, fews = 0; // their lanes in this half, and the groups
                     while (rest)
                     {
                         int const p = __builtin_ctz(rest);
@@ -495,6 +502,11 @@ void k_push_cell(pc::CellArgs<X> K)
                             cur = c;
                             pc::cellAdd<D, O, RN>(buf, m, acc);
                         }
+                        else if (DEP == DEP_FEW)
+                        {
+                            few |= m;
+                            ++fews;
+                        }
                         else if (n >= CELL_GROUP)
                         {
                             C one;
@@ -505,7 +517,22 @@ void k_push_cell(pc::CellArgs<X> K)
                         else
                             pc::cellAddOne<D, O, RN>(buf, p, lds, T.stride, c, p12, p2);
                     }
+                    // one such group deposits on the matrix cores, more lane by lane after the halves
+                    if (DEP == DEP_FEW && fews > 1)
+                        strays |= static_cast<unsigned long long>(few) << (32 * half);
+                    else if (DEP == DEP_FEW && few)
+                    {
+                        C one;
+                        one.zero();
+                        pc::cellAdd<D, O, RN>(buf, few, one);
+                        pc::cellFlush<D, O, RN>(one, lds, T.stride, __builtin_amdgcn_readlane(key, __builtin_ctz(few) + 32 * half), p12, p2);
+                    }
                 }
+                if constexpr (DEP == DEP_LANES)
+                    pc::cellAddLanes<O, RN, true>(ok, P.delta, P.w, q, P.v, coef, lds, T.stride, key, p12, p2);
+                else if constexpr (DEP == DEP_FEW)
+                    if (strays)
+                        pc::cellAddLanes<O, RN, false>((strays >> lane) & 1ull, P.delta, P.w, q, P.v, coef, lds, T.stride, key, p12, p2);
                 unsigned long long const left = __ballot(live && !ok);
                 if (left)
                 {
@@ -560,9 +587,21 @@ void k_push_cell(pc::CellArgs<X> K)
     }
 }
 
-template<class X, int D, int O, bool RN, bool FIX, bool PACKED = false>
+template<class X, int D, int O, bool RN, bool FIX, bool PACKED = false, int DEP = DEP_GROUPS>
 static void launchPushCellT(PushArgs const& A, PViewT<typename X::Real> const& in, hipStream_t s)
 {
+    if constexpr (D == 2 && DEP == DEP_GROUPS)
+        if (A.deposit == DEP_LANES)
+        {
+            launchPushCellT<X, D, O, RN, FIX, PACKED, DEP_LANES>(A, in, s);
+            return;
+        }
+    if constexpr (D == 2 && O == 1 && DEP == DEP_GROUPS)
+        if (A.deposit == DEP_FEW)
+        {
+            launchPushCellT<X, D, O, RN, FIX, PACKED, DEP_FEW>(A, in, s);
+            return;
+        }
     // more than 64 KB of dynamic LDS has to be allowed for the kernel (once per device)
     static std::mutex mtx;
     static bool allowed[64] = {};
@@ -571,7 +610,7 @@ static void launchPushCellT(PushArgs const& A, PViewT<typename X::Real> const& i
     {
         std::lock_guard<std::mutex> lock(mtx);
         if (!allowed[dev])
-            allowed[dev] = hipFuncSetAttribute(reinterpret_cast<void const*>(&k_push_cell<X, D, O, RN, FIX, PACKED>),
+            allowed[dev] = hipFuncSetAttribute(reinterpret_cast<void const*>(&k_push_cell<X, D, O, RN, FIX, PACKED, DEP>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, pc::CELL_LDS_MAX)
                            == hipSuccess;
     }
@@ -580,6 +619,6 @@ static void launchPushCellT(PushArgs const& A, PViewT<typename X::Real> const& i
     // eighty, of appended leavers)
     unsigned int const overflow = PACKED ? static_cast<unsigned int>(pc::CUS) : A.split;
     unsigned int const grid = D == 3 || PACKED ? static_cast<unsigned int>(A.sg.nsegs) * A.split + overflow : A.st.itemsCap;
-    k_push_cell<X, D, O, RN, FIX, PACKED><<<grid, pc::CellCfg<X, D, O>::BLOCK, A.tile.bytes, s>>>(pc::CellArgs<X>{A, in});
+    k_push_cell<X, D, O, RN, FIX, PACKED, DEP><<<grid, pc::CellCfg<X, D, O>::BLOCK, A.tile.bytes, s>>>(pc::CellArgs<X>{A, in});
 }
 } // namespace phx

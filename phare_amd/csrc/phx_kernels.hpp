@@ -125,6 +125,7 @@ struct SegTables
     unsigned int* nItems;     // number of work items
     unsigned int itemsCap;    // work items the storage's capacity allows (grid of the push)
     unsigned int rowsPerItem; // most segment rows per work item
+    bool sparse;              // 2D: few particles per cell (cellSparse)
 };
 
 // in-kernel timing of one push launch site (a node of the captured step): the earliest
@@ -158,6 +159,7 @@ struct PushArgs
     int segOn; // the array is cell-segmented (sg, st valid)
     unsigned int split; // cell-grouped push in 3D or over packed storage: workgroups per segment
     unsigned long long* lone; // cell-grouped push: where to count the particles pushed one by one (or null)
+    int deposit; // cell-grouped push: DEP_GROUPS, DEP_FEW or DEP_LANES
     int packed; // the segments follow each other without padding: slots st.off[s] .. st.off[s + 1], the last up to n
     SegGeom sg;
     SegTables st;
@@ -197,8 +199,10 @@ unsigned int compactBlocks(unsigned long long n);
 SegPatch segPatchOf(int dim, int const* lo, int const* hi, int const* pref);
 TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies, int slabs);
 unsigned int segItemsCap(SegGeom const& sg, SegTables const& tables, unsigned long long capacity);
-// rows per work item of an array of `slots` slots, at most `most`
-unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most);
+// rows per work item of an array of `slots` slots, at most `most`; no further items where they would hold
+// fewer than `least` on the average
+unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most, int least);
+constexpr int ITEM_LEAST = 2, ITEM_LEAST_PACKED = 4;
 // first half of a sort of src (n slots) into cell-segmented storage: counts per cell, the rank
 // of every particle in its cell (rank: n words) and the segment tables up to the total slot count
 // (tables.off[nsegs + 1]); `work` holds ncells + 1 + 2 (nsegs + 1) words
@@ -240,6 +244,13 @@ inline bool cellGrouped(int dim, int order, bool fp32) { return dim == 3 || (dim
 // deposited together; the LDS tile of cellTileShape (5 slabs, 4 with A.rhoFromN)
 void launchPushCell(PushArgs const& A, PView const& in, hipStream_t s);
 TileSpec cellTileShape(bool fp32, int dim, int order, SegGeom const& sg, int slabs, int pad);
+// how the particles of a row deposit in the cell-grouped push: those of a cell together on the matrix cores;
+// in 2D also small groups lane by lane (order 1), or every particle by its own lane
+enum { DEP_GROUPS, DEP_FEW, DEP_LANES };
+// whether a 2D array of `slots` slots holds so few particles per cell that they deposit lane by lane
+bool cellSparse(int dim, int order, SegGeom const& sg, unsigned long long slots);
+// rare: the array is sorted less often than every 20 pushes in mode all, or by the caller alone
+int cellDeposit(int dim, int order, bool sparse, bool rare);
 // workgroups per segment (A.split) for an array of `slots` slots
 unsigned int cellSplit(bool fp32, int order, SegGeom const& sg, unsigned long long slots);
 // BorisPusher::move in place over A.n slots with box-list selectors; status[i] gets the slot's

@@ -1272,10 +1272,9 @@ TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies, int sla
 // order 3, 64 per cell 254 us with 32 rows, 290 with 16 (three rounds). Two species in 1D (order 3, 1000
 // cells, 200 per cell): 184 us per step in 112 workgroups of 32 rows, 121 in one round. The FP32 push holds more
 // workgroups and keeps the tuned rows (2D order 2: 287 us of 24 rows, 294 of one round)
-unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most)
+unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most, int least)
 {
     constexpr double ITEM_OVERHEAD = 6.;
-    constexpr double MIN_ROWS      = 4.;    // a row per wavefront
     constexpr double SPREAD        = 1.125; // segments this far above the average still take k items
     constexpr double HELD          = 4. * pc::CUS;
     constexpr double ROUNDS        = 4.; // past these more items only add overhead
@@ -1283,7 +1282,7 @@ unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most)
     double const rows = std::max(1., static_cast<double>(slots) / LANES / segs);
     double best       = 0.;
     int bestRows      = most;
-    for (int k = 1; k == 1 || rows / k >= MIN_ROWS; ++k)
+    for (int k = 1; k == 1 || rows / k >= least; ++k)
     {
         double const each = rows / k;
         double const cost = std::ceil(segs * k / HELD) * (each + ITEM_OVERHEAD);
@@ -1565,6 +1564,26 @@ TileSpec cellTileShape(bool fp32, int dim, int order, SegGeom const& sg, int sla
         T.bytes    = static_cast<unsigned int>(8 * (slabs * T.stride + T.emStride)) + waves * 8u * pc::WSTR * 17u;
     }
     return T;
+}
+
+// where a cell holds few particles their groups are a chain of many small steps. 2D FP64, 190x150 cells,
+// per PPC step, by lanes and by groups: order 1, 12 per cell 124 us and 128, 24 per cell 143 and 144 (100x80 cells
+// 99 and 95); order 2, 5 per cell 101 and 108, 8 per cell 134 and 125; order 3, 3 per cell 99 and 104, 5 per cell
+// 126 and 115, in FP32 92 and 97 at 3, 101 and 95 at 4. Slots count up to one empty one per cell
+bool cellSparse(int dim, int order, SegGeom const& sg, unsigned long long slots)
+{
+    double const most = order == 1 ? 14. : (order == 2 ? 6.5 : 3.75);
+    return dim == 2 && static_cast<double>(slots) <= most * sg.ncells;
+}
+
+// at order 1 in 2D a stencil is 16 words, and small groups are cheaper lane by lane, which counts as the
+// particles drift from their cells: 190x150 cells, 50 per cell, 30 steps after a sort a push takes 81 us
+// with every small group by itself, 67 lane by lane, 48 and 49 right after the sort; per PPC step sorted
+// every 30 steps 190 and 180 us, every 12 steps 174 and 176. At orders 2 and 3 (36 and 64 words) it was the
+// slower one at either interval (order 2, 100 per cell: 325 us by groups, 350)
+int cellDeposit(int dim, int order, bool sparse, bool rare)
+{
+    return dim == 2 && sparse ? DEP_LANES : (dim == 2 && order == 1 && rare ? DEP_FEW : DEP_GROUPS);
 }
 
 // workgroups per segment of the cell-grouped push: as many as give three rounds of the workgroups the
