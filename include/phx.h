@@ -349,8 +349,9 @@ typedef struct {
                              dimensions); 0 keeps the default of the dimension */
     int rows_per_item;    /* most segment rows per workgroup of the segmented push (1..4096); an
                              FP64 or cell-grouped FP32 array takes fewer where that fills the GPU */
-    int tile_row_pad;     /* LDS tile pitches padded to a multiple of this many nodes (1: none):
-                             the pitches of dimensions 1 and 2 */
+    int tile_row_pad;     /* LDS tile pitches padded to a multiple of this many nodes (1: none): the
+                             rows in mixed-precision 2D at orders 1 and 2, the pitches of dimensions 1
+                             and 2 in 3D; without effect in 1D and on the other 2D levels */
     int sort_interval;    /* PPC steps of phx_advance between two sorts (0: never) */
     int tile_copies;      /* moment copies of the LDS tile of the linear-storage push (1, 2, 4, 8;
                              lane l adds into copy l % copies) */
