@@ -205,7 +205,7 @@ def family_line(wl, workload_name, precision, res):
     a = b / (res["ms_all"] * 1e-3) / 1e9
     if wl.dim == 3:
         kernel = ("k_push_cell (mixed precision" if precision == "fp32" else "k_push_cell (FP64") + \
-            ", cell-segmented storage, one workgroup per 4x4x4-cell segment: prePush+gather+Boris+" \
+            ", cell-ordered segments of 4x4x4 cells, shared by workgroups on small levels: prePush+gather+Boris+" \
             "postPush+deposit, mode all; 3D staged path)"
     elif precision == "fp32":
         kernel = "k_push_seg32 (mixed precision, mode all)"

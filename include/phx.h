@@ -327,7 +327,8 @@ phx_status phx_advance(phx_ctx* ctx, double dt, int nsteps);
 /* Storage order (no counterpart in the reference, whose ParticleArray keeps insertion order and
    a CellMap): reorders every population's domain particles by cell, row-major over the AMR box,
    the order the push kernel's LDS deposit tile relies on. phx_initialize sorts once and
-   phx_advance every `steps` PPC steps (0: never; default 30, in 3D 7). Results do not depend on the order
+   phx_advance every `steps` PPC steps (0: never; default 30, in 3D 7; 2D levels of FP64 or order 3 run
+   fastest at 8 to 12, which phx.Level takes from the tuning table). Results do not depend on the order
    beyond the summation order of the deposit. */
 phx_status phx_sort_particles(phx_ctx* ctx);
 phx_status phx_set_sort_interval(phx_ctx* ctx, int steps);
@@ -339,8 +340,9 @@ phx_status phx_diagnostics(phx_ctx* ctx, double out[4]);
 void* phx_stream(phx_ctx* ctx);
 
 /* ---- tuning (no counterpart in the reference: launch shapes of this build) ------------------- */
-/* The shapes the segmented push and the sort use; the defaults are the winners of the project's
-   autotuner (phare_amd/autotune.py) on the 2D Harris workload. phx_set_tuning rebuilds the
+/* The shapes the segmented push and the sort use; the winners of the project's
+   autotuner (phare_amd/autotune.py) are in phare_amd/tuning_table.json, by dimension, order, precision
+   and particles per cell. phx_set_tuning rebuilds the
    segment tables of the level's patches, re-sorts the domain arrays that are cell-segmented and
    drops the captured steps (the next phx_advance captures again). */
 typedef struct {

@@ -2,8 +2,9 @@
 
 Usage: python -m phare_amd.build   (or phare_amd.build.build() from __graft_entry__.build())
 
-Every translation unit is compiled as HIP for gfx950 only, without FMA contraction (the plain
-FP64 path reproduces the reference's rounding), with hardware FP64 atomics on coarse-grained
+Every translation unit is compiled as HIP for gfx950 only, without FMA contraction (the field
+operators and the linear and 1D FP64 pushes reproduce the reference's rounding; the cell-grouped push writes
+its fused multiply-adds out), with hardware FP64 atomics on coarse-grained
 memory, and with packed-FP32 instructions disabled.
 """
 import concurrent.futures as cf

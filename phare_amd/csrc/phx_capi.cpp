@@ -1425,9 +1425,11 @@ phx_status allocSegTables(phx_ctx* c)
     return PHX_OK;
 }
 
-// the launch shapes of this build before any tuning: the autotuner's winners on the 2D Harris
-// workload (segments of 2x32 cells, at most 32 rows per work item, tile rows padded to 16 nodes,
-// a sort every 30 PPC steps); runs of 64 cells in 1D, 4x4x4 blocks in 3D
+// the launch shapes of this build before any tuning: in 2D those of the push with one particle per lane
+// (segments of 2x32 cells, at most 32 rows per work item, tile rows padded to 16 nodes, a sort every 30 PPC
+// steps), which the mixed-precision levels of orders 1 and 2 run. The cell-grouped 2D push is faster with 64 rows and a
+// sort every 12 steps (256x128 cells, order 2, 100 per cell: 0.29 ms per PPC step, 0.33 with these): the tuning
+// table holds that. Runs of 64 cells in 1D, 4x4x4 blocks in 3D
 phx_tuning defaultTuning(int dim)
 {
     phx_tuning t{};

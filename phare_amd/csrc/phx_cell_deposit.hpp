@@ -13,10 +13,14 @@
 // 108 (order 2) or 256 (order 3) lanes of ds_add_f64, about 30 cycles of the CU's LDS per
 // wavefront instruction, and costs about a quarter (W = 4) or a sixteenth (W = 2) of an MFMA here.
 //
+// An instruction takes 64 cycles of its SIMD (16x16x4) or 16 (4x4x4), the same rate, at which independent
+// chains reach 75 TFLOP/s: in the 3D push at order 2 the matrix cores are 13 % busy.
+//
 // The lanes of a wavefront hand their weights over through a small LDS buffer of the wavefront, 32
 // particles at a time: array j (the weights along x, y, z, then the values) of particle p at
-// j * WSTR + p. WSTR is 36 words, so that the four arrays and four particle pairs that one read
-// touches lie in distinct banks.
+// j * WSTR + p. WSTR is 36 words: the four arrays and four particle pairs that one read touches lie in
+// distinct banks in the FP32 buffer, and in the FP64 one pairs 2 and 3 of an array share the banks of
+// pairs 0 and 1 of the next (conflicts of the whole push: 15 % of its LDS cycles at order 2 in 3D).
 #pragma once
 
 #include "phx_push_common.hpp"

@@ -21,8 +21,9 @@ namespace pc
 // FP32 in 3D: the stage and the buffers take half the LDS and the row half the registers, 256 fit at every
 // order (PPC step, order 3: 0.54 ms against 0.63 with 512; order 1: 0.61 and 0.64; order 2: 1.87 and 1.88)
 // In 2D four workgroups of 256 fit a CU (256x128 cells, 100 per cell, order 2: 0.093 ms after a sort,
-// growing to 0.17 over 30 steps, as drifted lanes meet in LDS banks; one particle per lane into the
-// tile, in columns, took 0.137)
+// growing to 0.17 over 25 steps, as drifted particles make more and smaller groups: LDS instructions 3.9 to
+// 7.0 million, conflicts 4 to 13 % of the LDS cycles, LDS and vector units below half busy throughout; one
+// particle per lane into the tile, in columns, took 0.137)
 constexpr int cellBlock(bool fp32, int dim, int order)
 {
     return fp32 || dim == 2 || order == 2 ? 256 : 512;
@@ -39,8 +40,10 @@ struct CellCfg
     // that finds room for a workgroup's particles may add its row)
     static constexpr unsigned int LIST = 2 * BLOCK;
 };
-// the smallest group of lanes of one cell (of the 32 of a half row) that deposits on the matrix cores,
-// and the smallest that moves the accumulated window to its cell
+// the smallest group of lanes of one cell (of the 32 of a half row) that deposits on the matrix cores (one
+// lane deposits by itself), and the smallest that moves the accumulated window to its cell: 4, 8 and 16
+// lanes are within 1 % of each other at orders 2 and 3 in 2D and 3D; 16 is slower at order 1 in 2D (190x150
+// cells, 16 per cell: 157 us per PPC step, 129 with 8 and with 4; 100 per cell 264, 248 and 258)
 constexpr int CELL_GROUP = 2;
 constexpr int CELL_MOVE  = 8;
 constexpr unsigned long long CUS = 256; // compute units of the GPU
@@ -271,9 +274,11 @@ __device__ __forceinline__ void gatherStaged(R const* em, int e1, int e2, int no
 
 // ---------------------------------------------------------------------------------------------
 // fused push + deposit over cell-ordered segmented storage, A.split workgroups per segment in 3D, one
-// per work item in 2D (segments of 4x4x4 and 2x32 cells): the rows of a segment hold its particles in cell order, each wavefront
-// takes a run of them, and the particles of one cell deposit together on the matrix cores
-// (phx_cell_deposit.hpp). The tile covers the segment with the stencil and one cell of motion on
+// per work item in 2D (segments of 4x4x4 and 2x32 cells): the rows of a segment hold its particles in cell
+// order, each wavefront takes a run of them, and the particles of one cell deposit together on the matrix
+// cores (phx_cell_deposit.hpp). The gather and the weights use fused multiply-adds: a velocity differs from
+// the reference's in its last digits (1e-16 of it), where the one-by-one push below and the linear one
+// keep the reference's operations bit for bit. The tile covers the segment with the stencil and one cell of motion on
 // each side, and E and B of the segment's surroundings are staged beside it. A particle that leaves
 // the domain, the tile or the stage is left as it is and noted in a list in LDS; the listed
 // particles of the whole workgroup are pushed 64 to a wavefront, gathering from HBM, and deposit one

@@ -110,7 +110,7 @@ struct SegGeom
     int n[3];      // level box cells per dimension
     int maxSeg[3]; // largest segment extent over the patches (the launch's LDS tile)
     int dense;       // positions fill the rows one after the other
-    int rowPad;      // 2D LDS tile rows padded to a multiple of this many nodes
+    int rowPad;      // tile rows of the mixed-precision 2D push padded to a multiple of this many nodes
     SegPatch first;               // patch 0 (a one-patch level reads it from the kernel arguments)
     SegPatch const* patch;        // [npatch] (device)
     int const* owner;             // [level box cells, row-major] patch of each cell, -1: none

@@ -1265,13 +1265,17 @@ TileSpec segTileShape(int dim, int order, SegGeom const& sg, int copies, int sla
 }
 
 
-// rows per work item of an array of `slots` slots, at most `most`: of k items per segment, each as
-// costly as its rows and ITEM_OVERHEAD more (its tile zeroed, staged and flushed), the k whose items
-// finish first in rounds of the workgroups the GPU holds at once (four per CU). 2D Harris, per PPC
+// of k items per segment, each as costly as its rows and ITEM_OVERHEAD more (its tile zeroed, staged and
+// flushed), the k whose items finish first in rounds of the workgroups the GPU holds at once: four per CU, what
+// the LDS of the 2D FP64 push leaves room for and the waves of the 1D one. The same levels with two or eight per
+// CU counted: 1D of 4000 cells 104 and 102 us per PPC step, 95 with four; 2D 256x128, order 2, 30 per cell 202
+// and 201, 179; with SPREAD 1 (190x150, order 3, 50 per cell) 273, 257 with 1.125 and with 1.3; ITEM_OVERHEAD
+// from 3 to 24 rows and up to 1 or 8 rounds choose the same. 2D Harris, per PPC
 // step: 256x128, order 2, 100 per cell 287 us with one round (51 rows per item), 303 with two; 190x150,
 // order 3, 64 per cell 254 us with 32 rows, 290 with 16 (three rounds). Two species in 1D (order 3, 1000
 // cells, 200 per cell): 184 us per step in 112 workgroups of 32 rows, 121 in one round. The FP32 push holds more
-// workgroups and keeps the tuned rows (2D order 2: 287 us of 24 rows, 294 of one round)
+// workgroups and keeps the tuned rows (2D order 2: 287 us of 24 rows, 294 of one round). ITEM_LEAST: 100x80
+// cells, order 2, 8 per cell 92 us with 2, 101 with 4; packed, order 3, 20 per cell 275 and 255
 unsigned int itemRowsFor(SegGeom const& sg, unsigned long long slots, int most, int least)
 {
     constexpr double ITEM_OVERHEAD = 6.;
@@ -1586,9 +1590,13 @@ int cellDeposit(int dim, int order, bool sparse, bool rare)
     return dim == 2 && sparse ? DEP_LANES : (dim == 2 && order == 1 && rare ? DEP_FEW : DEP_GROUPS);
 }
 
-// workgroups per segment of the cell-grouped push: as many as give three rounds of the workgroups the
-// GPU holds at once, while each of a segment's wavefronts keeps two rows (a workgroup zeroes, stages
-// and flushes its tile whatever its rows)
+// workgroups per segment of the cell-grouped 3D push: as many as give three times the workgroups that the GPU
+// holds at once in FP64, while each of a segment's wavefronts keeps two rows (a workgroup zeroes, stages and
+// flushes its tile whatever its rows). Per PPC step, 36x41x30 cells, 64 per cell: order 3 with one per CU
+// counted 0.95 ms, with two 1.05; order 2 with two 0.64, with one 0.67; the FP32 push, of which three fit a CU,
+// within 2 % with one, two or three. One and five rounds instead of three: 0.67 and 0.67 for 0.64 at order 2,
+// 0.95 and 1.04 for 0.95 at order 3. One and four rows per wavefront: 24x22x20 cells, order 3, 64 per cell 0.45
+// and 0.39 for 0.42, FP32 at order 2, 16 per cell 0.20 and 0.21 for 0.23
 unsigned int cellSplit(bool fp32, int order, SegGeom const& sg, unsigned long long slots)
 {
     unsigned long long const segs = static_cast<unsigned long long>(std::max(sg.nsegs, 1));
